@@ -227,7 +227,7 @@ __global__ void fire_mask_kernel(int64_t rows, int hw, uint64_t seed, int64_t ro
 
 // ------------------------------------------------------------------------------------------
 // Readout: one workgroup per row, cells in chunks of the workgroup size; the board sum runs in
-// cell order on one lane so that its rounding matches the sequential definition.
+// cell order (ordered_sum) so that its rounding matches the sequential definition.
 __global__ void readout_kernel(const float *x, int C, int hw, int out_off, int c_out, int n_out,
                                int head_kind, const float *headw, const float *headb,
                                float *conf_cell, float *conf_board, int32_t *argmax) {
@@ -245,13 +245,53 @@ __global__ void readout_kernel(const float *x, int C, int hw, int out_off, int c
             chunk[threadIdx.x] = cf;
         }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            const int n = hw - base < 256 ? hw - base : 256;
-            for (int i = 0; i < n; ++i) sum = __fadd_rn(sum, chunk[i]);
-        }
+        if (threadIdx.x < 64) sum = nca::ordered_sum(sum, chunk, hw - base < 256 ? hw - base : 256);
         __syncthreads();
     }
     if (threadIdx.x == 0 && conf_board) conf_board[r] = __fdiv_rn(sum, (float)hw);
+}
+
+// The readout of large boards in two launches: every cell on the whole device, then one wave per
+// board that adds the cells' confidences in order. One workgroup per row leaves all but `rows` of
+// the CUs idle (16 boards of 201x201: 662 us with the sum on one lane of it, 9 + 69 us in two launches).
+__global__ void readout_cells_kernel(const float *x, int64_t rows, int C, int hw, int out_off, int c_out, int n_out,
+                                     int head_kind, const float *headw, const float *headb, float *conf_cell,
+                                     int32_t *argmax) {
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= hw) return;
+    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+        int am;
+        const float cf = nca::cell_readout(x + (r * C + out_off) * (int64_t)hw + q, hw, c_out, n_out, head_kind, headw, headb, &am);
+        conf_cell[r * hw + q] = cf;
+        if (argmax) argmax[r * hw + q] = am;
+    }
+}
+
+__global__ void board_mean_kernel(const float *conf_cell, int hw, float *conf_board) {
+    const int64_t r = blockIdx.x;
+    const float sum = nca::ordered_sum(0.0f, conf_cell + r * hw, hw);
+    if (threadIdx.x == 0) conf_board[r] = __fdiv_rn(sum, (float)hw);
+}
+
+// Boards of at least this many cells take two launches where the cells' confidences have a buffer
+// (the caller's, or the per-step path's workspace); below it a row is a few passes of one
+// workgroup and a second launch costs more than it saves.
+constexpr int kReadoutSplit = 2048;
+
+int launch_readout(hipStream_t st, int64_t rows, const float *x, int C, int hw, int out_off, int c_out, int n_out,
+                   int head_kind, const float *headw, const float *headb, float *conf_cell, float *conf_board,
+                   int32_t *argmax, float *conf_buf) {
+    if (!conf_buf) conf_buf = conf_cell;
+    if (hw >= kReadoutSplit && conf_buf) {
+        hipLaunchKernelGGL(readout_cells_kernel, dim3((unsigned)((hw + 255) / 256), (unsigned)(rows < 65535 ? rows : 65535)),
+                           dim3(256), 0, st, x, rows, C, hw, out_off, c_out, n_out, head_kind, headw, headb, conf_buf, argmax);
+        if (conf_board)
+            hipLaunchKernelGGL(board_mean_kernel, dim3((unsigned)rows), dim3(64), 0, st, conf_buf, hw, conf_board);
+    } else {
+        hipLaunchKernelGGL(readout_kernel, dim3((unsigned)rows), dim3(256), 0, st, x, C, hw, out_off, c_out, n_out,
+                           head_kind, headw, headb, conf_cell, conf_board, argmax);
+    }
+    return hip_check(hipGetLastError(), "readout launch");
 }
 
 // ------------------------------------------------------------------------------------------
@@ -463,10 +503,11 @@ int run_tiled(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t s
         if (p.rows > 0x7fffffff) return fail(NCA_ERR_UNSUPPORTED, "rows=%lld", (long long)p.rows);
         const float *hw = reinterpret_cast<const float *>(p.packed + p.off_headw);
         const float *hb = reinterpret_cast<const float *>(p.packed + p.off_headb);
-        hipLaunchKernelGGL(readout_kernel, dim3((unsigned)p.rows), dim3(256), 0, st, p.x_out, d->channels, p.H * p.W,
-                           d->out_offset, d->c_out, d->n_out, d->head_kind, hw, hb, (float *)nullptr, p.conf_out,
-                           (int32_t *)nullptr);
-        return hip_check(hipGetLastError(), "readout launch");
+        // the workspace (checked above against x_in and x_out) is free once x_out is written: the
+        // cells' confidences go there
+        float *buf = need ? A : nullptr;
+        return launch_readout(st, p.rows, p.x_out, d->channels, p.H * p.W, d->out_offset, d->c_out, d->n_out, d->head_kind,
+                              hw, hb, nullptr, p.conf_out, nullptr, buf);
     }
     return NCA_OK;
 }
@@ -872,11 +913,9 @@ int nca_readout(const nca_cell_desc *cell, const void *packed, int64_t rows, int
     if (rows > 0x7fffffff) return fail(NCA_ERR_UNSUPPORTED, "rows=%lld", (long long)rows);
     const nca::PackedLayout L = layout_of(cell);
     const unsigned char *pk = static_cast<const unsigned char *>(packed);
-    hipLaunchKernelGGL(readout_kernel, dim3((unsigned)rows), dim3(256), 0, as_stream(stream), x,
-                       cell->channels, height * width, cell->out_offset, cell->c_out, cell->n_out,
-                       cell->head_kind, reinterpret_cast<const float *>(pk + L.headw),
-                       reinterpret_cast<const float *>(pk + L.headb), conf_cell, conf_board, argmax);
-    return hip_check(hipGetLastError(), "readout launch");
+    return launch_readout(as_stream(stream), rows, x, cell->channels, height * width, cell->out_offset, cell->c_out,
+                          cell->n_out, cell->head_kind, reinterpret_cast<const float *>(pk + L.headw),
+                          reinterpret_cast<const float *>(pk + L.headb), conf_cell, conf_board, argmax, nullptr);
 }
 
 int nca_conf_select(const float *conf, const uint8_t *alive, int32_t n_boards, int32_t k_trials,
