@@ -162,9 +162,27 @@ __device__ __forceinline__ void pack_w2k(const float *w2, int C, int HD, __bf16 
     }
 }
 
-// The whole packing in one launch: workgroups [64 k, 64 k + 64) build fragment layout k (W1, W2,
-// and for bf16 cells W2 for the hidden-major fc2, W1 quad-major, W2 k-major), the last one the
-// small vectors (kernels, b1, b2, head, padding value).
+// The backward's A operands (see nca_layout.h): A(i, k) = src[i si + k sk], zero for k >= K, as 16-byte
+// units [m-tile][k-block][lane].
+__device__ __forceinline__ void pack_units(const float *src, int M, int K, int si, int sk, int bf16, void *dst, int b, int nb) {
+    const int eb = bf16 ? 8 : 4, kblock = 4 * eb, nkb = (K + kblock - 1) / kblock;
+    const int total = (M / 16) * nkb * 64;
+    for (int u = b * blockDim.x + threadIdx.x; u < total; u += nb * blockDim.x) {
+        const int lane = u & 63, blk = u >> 6, kb = blk % nkb, i = (blk / nkb) * 16 + (lane & 15);
+        for (int s = 0; s < eb; ++s) {
+            const int k = kb * kblock + (bf16 ? 8 * (lane >> 4) + s : 4 * s + (lane >> 4));
+            const float v = k < K ? src[(size_t)i * si + (size_t)k * sk] : 0.0f;
+            if (bf16)
+                reinterpret_cast<__bf16 *>(dst)[(size_t)u * eb + s] = (__bf16)v;
+            else
+                reinterpret_cast<float *>(dst)[(size_t)u * eb + s] = v;
+        }
+    }
+}
+
+// The whole packing in one launch: workgroups [64 k, 64 k + 64) build layout k (the backward's W1,
+// W1^T and W2^T, then the forward's W1, W2, and for bf16 cells W2 for the hidden-major fc2, W1
+// quad-major, W2 k-major), the last one the small vectors (kernels, b1, b2, head, padding value).
 struct PackArgs {
     const float *kernels, *w1, *b1, *w2, *b2, *head_w, *head_b, *pad_vec;
     int nk, HD, C, F, nhw, nhb, bf;
@@ -172,12 +190,20 @@ struct PackArgs {
     nca::PackedLayout L;
 };
 
+constexpr int kPackBack = 3;  // layouts of the backward
+
 __global__ void pack_all(PackArgs a) {
     constexpr int kPB = 64;
-    const int b = blockIdx.x, part = b / kPB, pb = b - part * kPB;
+    const int b = blockIdx.x, part = b / kPB - kPackBack, pb = b % kPB;
     const int nfrag = a.bf ? 5 : 2;
     unsigned char *pk = a.pk;
-    if (part >= nfrag) {
+    if (part == -3) {
+        pack_units(a.w1, a.HD, a.F, a.F, 1, a.bf, pk + a.L.bw1, pb, kPB);
+    } else if (part == -2) {
+        pack_units(a.w1, a.F, a.HD, 1, a.F, a.bf, pk + a.L.bw1t, pb, kPB);
+    } else if (part == -1) {
+        pack_units(a.w2, a.HD, a.C, 1, a.HD, a.bf, pk + a.L.bw2t, pb, kPB);
+    } else if (part >= nfrag) {
         pack_small(a.kernels, a.nk, reinterpret_cast<float *>(pk + a.L.kern), a.bf, 0, 1);
         pack_small(a.b1, a.HD, reinterpret_cast<float *>(pk + a.L.b1), a.bf, 0, 1);
         pack_small(a.b2, a.C, reinterpret_cast<float *>(pk + a.L.b2), a.bf, 0, 1);
@@ -787,7 +813,7 @@ int nca_pack_weights(const nca_cell_desc *cell, const nca_cell_weights *w, void 
     pa.bf = bf ? 1 : 0;
     pa.pk = pk;
     pa.L = L;
-    hipLaunchKernelGGL(pack_all, dim3((bf ? 5 : 2) * 64 + 1), dim3(256), 0, st, pa);
+    hipLaunchKernelGGL(pack_all, dim3((kPackBack + (bf ? 5 : 2)) * 64 + 1), dim3(256), 0, st, pa);
     return hip_check(hipGetLastError(), "pack launch");
 }
 

@@ -12,13 +12,14 @@
 //              slice of given cells (ops.py:276-294): g_u; the fire mask gives g_dx = g_u * fire;
 //              partial sums of db2, the head's gradients and the loss
 //   stencil_z  z = perception of the saved state (feature-major, F x cells)
-//   MLP        h = relu(W1 z + b1); g_a = (W2^T g_dx) * [h > 0]; g_z = W1^T g_a: bf16 cells with
-//              32 channels and 256 hidden units in one fused kernel (mlp_back32, which also sums
-//              dW1, dW2 and db1, and stores g_z as bf16), other cells on fp32 MFMA GEMMs
+//   MLP        h = relu(W1 z + b1); g_a = (W2^T g_dx) * [h > 0]; g_z = W1^T g_a, dW1, dW2 and db1
 //   stencil_back  g_x = g_u + the transposed stencil of g_z (padding-aware: wall / zero halos
 //              take no gradient, wrap halos give it to the wrapped cell), the next step's
 //              gradient, and partial sums of the kernel-weight gradient
-//   partials   dW1 = g_a z^T, dW2 = g_dx h^T (split-K GEMMs), db1 (row sums of g_a), unless fused
+//
+// bf16 cells with 32 channels and 256 hidden units run it as one launch per chunk
+// (nca_bptt_fused.h) or, where that does not take the call, as the three launches below per step
+// (the MLP in mlp_back32); all other cells as one launch per step (nca_bptt_step.h).
 //
 // Every partial sum belongs to one of 256 fixed cell ranges (slots); each step adds its sums
 // into the slots, and one kernel adds the slots up in slot order after the last step, so the
@@ -49,7 +50,6 @@ constexpr int kPlaneMax = 2048;  // cells of a board whose planes the LDS stenci
 
 struct Dims {
     int C, F, HD, c_in, in_off, c_out, out_off, n_out, padding, bf16;
-    int gz16;  // g_z is stored as bf16 (by the fused MLP backward), else fp32
     int H, W, HW;
     int64_t rows, M;  // M = rows * HW cells
 };
@@ -89,16 +89,15 @@ bool planes_fit(const Dims &d) { return d.HW <= kPlaneMax && d.rows * d.C <= 0x7
 
 // Workspace (floats, 64-float aligned pieces, after the status block). part holds kSplit slots of P partial sums
 // each (slot s: the cells of range s), added to by every step of the chunk and reduced once at
-// the end; lossacc holds the loss's kSplit slots. The GEMM path's h and g_a (Hb, Ga) are not
-// needed by the fused kernel.
+// the end; lossacc holds the loss's kSplit slots. (Cells that fused_mlp takes; the others'
+// workspace is StepLayout.)
 struct WsLayout {
-    int64_t Z, Hb, Ga, Gz, Gdx, Gu, Gx0, Gx1, part, acc, lossacc, dk, denom, img, total;
+    int64_t Z, Gz, Gdx, Gu, Gx0, Gx1, part, acc, lossacc, dk, denom, img, total;
 };
 
 WsLayout ws_layout(const Dims &d, int n) {
     (void)n;
     const ParamLayout P = param_layout(d);
-    const bool fused = fused_mlp(d);
     auto al = [](int64_t v) { return (v + 63) & ~(int64_t)63; };
     WsLayout L;
     // the first kXchStatusBytes hold the status words of the forward's and the one-launch
@@ -106,10 +105,6 @@ WsLayout ws_layout(const Dims &d, int n) {
     int64_t o = (int64_t)(nca::kXchStatusBytes / sizeof(float));
     L.Z = o;
     o = al(o + (int64_t)d.F * d.M);
-    L.Hb = o;
-    o = al(o + (fused ? 0 : (int64_t)d.HD * d.M));
-    L.Ga = o;
-    o = al(o + (fused ? 0 : (int64_t)d.HD * d.M));
     L.Gz = o;
     o = al(o + (int64_t)d.F * d.M);
     L.Gdx = o;
@@ -149,9 +144,9 @@ __device__ __forceinline__ int neighbour(int i, int j, int dy, int dx, int H, in
     return (in || wrap) ? a * W + b : -1;
 }
 
-// Element i of g_z: fp32, or bf16 where the fused MLP backward wrote it (gz16).
-__device__ __forceinline__ float gz_at(const float *Gz, int gz16, int64_t i) {
-    return gz16 ? __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(Gz)[i] << 16) : Gz[i];
+// Element i of g_z as the fused MLP backward writes it (bf16).
+__device__ __forceinline__ float gz_at(const float *Gz, int64_t i) {
+    return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t *>(Gz)[i] << 16);
 }
 
 // Block-wide sum of one float per thread in a fixed tree order (deterministic).
@@ -286,31 +281,18 @@ __device__ __forceinline__ void load_out(const Dims &d, const float *x1c, float 
     for (int c = 0; c < NO; ++c) xo[c] = c < d.c_out ? v[c] : 0.0f;
 }
 
-// The cross-entropy gradient of the mlp head's logits at a cell with output channels xo, target
-// tgt and loss-mask value mk (gl[v] = d loss / d logit v, times the step's scale; 0 for
-// v >= n_out, and everywhere on a step without a loss term) and the cell's loss term (reference
-// src/nca/train.py:183-207). n_out, c_out <= NO.
+// The cross-entropy gradient at a cell with logits l and target tgt: gl[v] = d loss / d logit v,
+// times the step's scale (and the loss-mask value mk over *denom); 0 for v >= n_out. Returns the
+// cell's loss term (reference src/nca/train.py:183-207). n_out <= NO.
 template <int NO>
-__device__ __forceinline__ float head_grad_core(const Dims &d, float wscale, bool masked, const float *denom,
-                                                const float *hw, const float *hb, const float xo[NO], int tgt, float mk,
-                                                float gl[NO]) {
-#pragma unroll
-    for (int v = 0; v < NO; ++v) gl[v] = 0.0f;
-    if (wscale == 0.0f) return 0.0f;
+__device__ __forceinline__ float softmax_grad(const Dims &d, float wscale, bool masked, const float *denom, const float l[NO],
+                                              int tgt, float mk, float gl[NO]) {
     const float scale = masked ? wscale * mk / *denom : wscale;
-    float l[NO];
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < NO; ++v) {
-        l[v] = 0.0f;
-        if (v < d.n_out) {
-            float acc = hb[v];
-#pragma unroll
-            for (int c = 0; c < NO; ++c)
-                if (c < d.c_out) acc = __builtin_fmaf(hw[v * d.c_out + c], xo[c], acc);
-            l[v] = acc;
-            mx = fmaxf(mx, acc);
-        }
+        gl[v] = 0.0f;
+        if (v < d.n_out) mx = fmaxf(mx, l[v]);
     }
     float s = 0.0f, lt = mx, e[NO];
 #pragma unroll
@@ -324,6 +306,30 @@ __device__ __forceinline__ float head_grad_core(const Dims &d, float wscale, boo
     for (int v = 0; v < NO; ++v)
         if (v < d.n_out) gl[v] = (e[v] / s - (v == tgt ? 1.0f : 0.0f)) * scale;
     return (mx + logf(s) - lt) * scale;
+}
+
+// The same from the cell's output channels xo and the head's weights and bias (zero gradients on a
+// step without a loss term). n_out, c_out <= NO.
+template <int NO>
+__device__ __forceinline__ float head_grad_core(const Dims &d, float wscale, bool masked, const float *denom,
+                                                const float *hw, const float *hb, const float xo[NO], int tgt, float mk,
+                                                float gl[NO]) {
+#pragma unroll
+    for (int v = 0; v < NO; ++v) gl[v] = 0.0f;
+    if (wscale == 0.0f) return 0.0f;
+    float l[NO];
+#pragma unroll
+    for (int v = 0; v < NO; ++v) {
+        l[v] = 0.0f;
+        if (v < d.n_out) {
+            float acc = hb[v];
+#pragma unroll
+            for (int c = 0; c < NO; ++c)
+                if (c < d.c_out) acc = __builtin_fmaf(hw[v * d.c_out + c], xo[c], acc);
+            l[v] = acc;
+        }
+    }
+    return softmax_grad<NO>(d, wscale, masked, denom, l, tgt, mk, gl);
 }
 template <int NO>
 __device__ __forceinline__ float head_grad(const FrontArgs &a, const float *hw, const float *hb, const float xo[NO], int tgt,
@@ -507,18 +513,13 @@ __device__ __forceinline__ float tap_value(const float *xr, const Dims &d, int i
     return d.bf16 ? nca::round_bf16(v) : v;
 }
 
-// z element i: fp32, or bf16 for the fused MLP backward (Z16)
-template <bool Z16>
+// z element i, a bf16 value, for the fused MLP backward
 __device__ __forceinline__ void z_store(float *Z, int64_t i, float v) {
-    if (Z16)
-        reinterpret_cast<__bf16 *>(Z)[i] = (__bf16)v;  // v is a bf16 value
-    else
-        Z[i] = v;
+    reinterpret_cast<__bf16 *>(Z)[i] = (__bf16)v;
 }
 
 // z (F x M, feature-major) of the state x (rows, C, H, W): thread (row, channel, cell) with
 // channel and cell from blockIdx.x, rows strided over blockIdx.y.
-template <bool Z16>
 __global__ void __launch_bounds__(kThreads) stencil_z_kernel(Dims d, const float *__restrict__ x,
                                                              const float *__restrict__ kern,
                                                              const float *__restrict__ padv, float *__restrict__ Z) {
@@ -537,7 +538,7 @@ __global__ void __launch_bounds__(kThreads) stencil_z_kernel(Dims d, const float
             float acc = 0.0f;
 #pragma unroll
             for (int t = 0; t < 9; ++t) acc = __builtin_fmaf(kern[k * 9 + t], xv[t], acc);
-            z_store<Z16>(Z, (int64_t)(k * d.C + c) * d.M + m, d.bf16 ? nca::round_bf16(acc) : acc);
+            z_store(Z, (int64_t)(k * d.C + c) * d.M + m, d.bf16 ? nca::round_bf16(acc) : acc);
         }
     }
 }
@@ -579,14 +580,14 @@ __global__ void __launch_bounds__(kBackThreads) stencil_back_kernel(
                 const int qc = qs < 0 ? 0 : qs;
                 float gv[4];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) gv[k] = gz_at(Gz, d.gz16, gzo + k * ks + qc);
+                for (int k = 0; k < 4; ++k) gv[k] = gz_at(Gz, gzo + k * ks + qc);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) g = qs >= 0 ? __builtin_fmaf(kern[k * 9 + t], gv[k], g) : g;
             }
             gx[e] = g;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const float gzv = gz_at(Gz, d.gz16, gzo + k * ks + q);
+                const float gzv = gz_at(Gz, gzo + k * ks + q);
 #pragma unroll
                 for (int t = 0; t < 9; ++t) acc[k * 9 + t] = __builtin_fmaf(gzv, xv[t], acc[k * 9 + t]);
             }
@@ -618,7 +619,6 @@ __device__ __forceinline__ void plane_taps(const float *xs, const Dims &d, int i
 
 // stencil_z for boards of at most kPlaneMax cells: workgroup p stages plane p = (row, channel)
 // of x in LDS and writes that channel's 4 features of the row's cells.
-template <bool Z16>
 __device__ void z_plane_body(const Dims &d, const float *__restrict__ x, const float *__restrict__ kern,
                              const float *__restrict__ padv, float *__restrict__ Z, int pl, float *xs) {
     const int row = pl / d.C, c = pl - row * d.C;
@@ -657,7 +657,7 @@ __device__ void z_plane_body(const Dims &d, const float *__restrict__ x, const f
             float acc = 0.0f;
 #pragma unroll
             for (int t = 0; t < 9; ++t) acc = __builtin_fmaf(kern[k * 9 + t], xv[t], acc);
-            z_store<Z16>(Z, (int64_t)(k * d.C + c) * d.M + m, d.bf16 ? nca::round_bf16(acc) : acc);
+            z_store(Z, (int64_t)(k * d.C + c) * d.M + m, d.bf16 ? nca::round_bf16(acc) : acc);
         }
     };
     if (W <= kThreads) {
@@ -698,14 +698,6 @@ __device__ void z_plane_body(const Dims &d, const float *__restrict__ x, const f
     }
 }
 
-template <bool Z16>
-__global__ void __launch_bounds__(kThreads) stencil_z_plane(Dims d, const float *__restrict__ x,
-                                                            const float *__restrict__ kern,
-                                                            const float *__restrict__ padv, float *__restrict__ Z) {
-    extern __shared__ float xs[];  // (H + 2) (W + 2) floats
-    z_plane_body<Z16>(d, x, kern, padv, Z, blockIdx.x, xs);
-}
-
 // The front (kSplit x C / 8 workgroups) and the bf16 z (rows x C workgroups) of one step in one
 // launch: they are independent, and each alone leaves most of the GPU idle.
 template <int NO>
@@ -719,7 +711,7 @@ __global__ void __launch_bounds__(kThreads) front_z_kernel(FrontArgs a, const fl
     if ((int)blockIdx.x < nf)
         front_body<NO>(a, (int)blockIdx.x % kSplit, (int)blockIdx.x / kSplit, red, hwL);
     else
-        z_plane_body<true>(a.d, x, kern, padv, Z, (int)blockIdx.x - nf, xs);
+        z_plane_body(a.d, x, kern, padv, Z, (int)blockIdx.x - nf, xs);
 }
 
 // stencil_back for boards of at most kPlaneMax cells: workgroup p stages plane p = (row,
@@ -746,7 +738,7 @@ __global__ void __launch_bounds__(kThreads) stencil_back_plane(Dims d, const flo
             const int q = q0 + u * kThreads + threadIdx.x, qc = q < d.HW ? q : 0;
             v[u][0] = xr[qc];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) v[u][1 + k] = gz_at(Gz, d.gz16, gzo + k * ks + qc);
+            for (int k = 0; k < 4; ++k) v[u][1 + k] = gz_at(Gz, gzo + k * ks + qc);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -800,8 +792,7 @@ constexpr int kStripPlanes = 4;  // (row, channel) planes per workgroup of stenc
 // column j) walks down rows [band R, band R + R) of column j with the 3x3 neighbourhood of x and
 // g_z in registers, loading one new row of 3 columns per cell (15 LDS reads instead of 45). Per
 // cell the sums run in the order of stencil_back_kernel; the kernel-weight sums of the
-// workgroup's planes go to slot b. GZ16: g_z is bf16.
-template <bool GZ16>
+// workgroup's planes go to slot b.
 __global__ void __launch_bounds__(kThreads) stencil_back_strip(Dims d, const float *__restrict__ x,
                                                                const float *__restrict__ Gu,
                                                                const float *__restrict__ Gz,
@@ -846,7 +837,7 @@ __global__ void __launch_bounds__(kThreads) stencil_back_strip(Dims d, const flo
             if (u * kThreads < HW) {  // uniform
                 pv[u][0] = xr[qc];
 #pragma unroll
-                for (int k = 0; k < 4; ++k) pv[u][1 + k] = gz_at(Gz, GZ16, gzo + k * ks + qc);
+                for (int k = 0; k < 4; ++k) pv[u][1 + k] = gz_at(Gz, gzo + k * ks + qc);
                 pv[u][5] = ur[qc];
             }
         }
@@ -938,33 +929,6 @@ __global__ void __launch_bounds__(kThreads) reduce_dk(const float *dk, int64_t p
     if (threadIdx.x == 0) acc[v] = __fadd_rn(acc[v], s);
 }
 
-// Row sums of a feature-major matrix G (R x M) over the kSplit cell ranges, added into the
-// slots: wave w of block (b, s) takes row 4 b + w over range s.
-__global__ void __launch_bounds__(kThreads) rowsum_kernel(const float *__restrict__ G, int64_t M, int R,
-                                                          float *__restrict__ part, int64_t P, int64_t off) {
-    const int lane = threadIdx.x & 63, r = blockIdx.x * 4 + (threadIdx.x >> 6), s = blockIdx.y;
-    if (r >= R) return;  // uniform across the wave
-    const int64_t per = (M + kSplit - 1) / kSplit, m0 = s * per, m1 = m0 + per < M ? m0 + per : M;
-    const float *g = G + (int64_t)r * M;
-    float acc = 0.0f;
-    for (int64_t mb = m0; mb < m1; mb += 256) {
-        float v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int64_t m = mb + 64 * u + lane;
-            v[u] = m < m1 ? g[m] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = __fadd_rn(acc, v[u]);
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) acc = __fadd_rn(acc, __shfl_xor(acc, o));
-    if (lane == 0) {
-        float *pp = part + s * P + off + r;
-        *pp = __fadd_rn(*pp, acc);
-    }
-}
-
 // acc[i] = the sum of the kSplit slots in slot order.
 __global__ void reduce_acc_kernel(const float *part, int64_t P, float *acc) {
     // slot order; 64 slots' loads issued before their additions (4 round trips for 256 slots)
@@ -1046,106 +1010,6 @@ __global__ void finish_kernel(const float *part, int64_t P, float *acc, GradOut 
     }
 }
 
-// ------------------------------------------------------------------------------------------
-// fp32 GEMM on v_mfma_f32_16x16x4_f32: C (M x N) = A (M x K) B (K x N) with strided operands
-// (A(m, k) = A[m sam + k sak], B(k, n) = B[k sbk + n sbn], one of each pair of strides being 1),
-// 64 x 64 block tiles, 16-deep k slices through LDS, each of the 4 waves a 32 x 32 quadrant.
-// Split-K: block z sums k in [z kps, (z + 1) kps) and writes (or adds) its partial at
-// C + z * csplit.
-// Epilogues: 0 store (+ row bias), 1 fc1: bias, bf16 rounding for bf16 cells, ReLU,
-// 2 mask: times [mask(m, n) > 0].
-struct GemmArgs {
-    const float *A;
-    int64_t sam, sak;
-    const float *B;
-    int64_t sbk, sbn;
-    float *Cm;
-    int64_t ldc, csplit;
-    int64_t M, N, K, kps;
-    const float *bias;  // per row m
-    const float *mask;
-    int64_t ldmask;
-    int epi, round_in, round_out;  // round_in: round A to bf16 on load (the forward's bf16 weights);
-                                   // round_out: round the product to bf16 (before mask / ReLU)
-    int accum;                     // add the result to C instead of storing it
-};
-
-constexpr int GBM = 64, GBN = 64, GBK = 16;
-
-__global__ void __launch_bounds__(256) gemm_f32_kernel(GemmArgs g) {
-    __shared__ float As[GBK][GBM + 4];
-    __shared__ float Bs[GBK][GBN + 4];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    const int64_t m0 = (int64_t)blockIdx.y * GBM, n0 = (int64_t)blockIdx.x * GBN;
-    const int64_t kb = (int64_t)blockIdx.z * g.kps, ke = kb + g.kps < g.K ? kb + g.kps : g.K;
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    f32x4 acc[2][2];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bool a_kfast = g.sak == 1, b_nfast = g.sbn == 1;
-    for (int64_t k0 = kb; k0 < ke; k0 += GBK) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int e = tid + 256 * r;
-            const int am = a_kfast ? e >> 4 : e & 63, ak = a_kfast ? e & 15 : e >> 6;
-            const int64_t gm = m0 + am, gk = k0 + ak;
-            float v = 0.0f;
-            if (gm < g.M && gk < ke) v = g.A[gm * g.sam + gk * g.sak];
-            As[ak][am] = g.round_in ? nca::round_bf16(v) : v;
-            const int bn = b_nfast ? e & 63 : e >> 4, bk = b_nfast ? e >> 6 : e & 15;
-            const int64_t gn = n0 + bn, gk2 = k0 + bk;
-            Bs[bk][bn] = (gn < g.N && gk2 < ke) ? g.B[gk2 * g.sbk + gn * g.sbn] : 0.0f;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < GBK; kk += 4) {
-            float af[2], bfv[2];
-#pragma unroll
-            for (int a = 0; a < 2; ++a) af[a] = As[kk + (lane >> 4)][wm * 32 + a * 16 + (lane & 15)];
-#pragma unroll
-            for (int b = 0; b < 2; ++b) bfv[b] = Bs[kk + (lane >> 4)][wn * 32 + b * 16 + (lane & 15)];
-#pragma unroll
-            for (int a = 0; a < 2; ++a)
-#pragma unroll
-                for (int b = 0; b < 2; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(af[a], bfv[b], acc[a][b], 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    float *Cz = g.Cm + (int64_t)blockIdx.z * g.csplit;
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int64_t gm = m0 + wm * 32 + a * 16 + 4 * (lane >> 4) + v;
-                const int64_t gn = n0 + wn * 32 + b * 16 + (lane & 15);
-                if (gm >= g.M || gn >= g.N) continue;
-                float r = acc[a][b][v];
-                if (g.bias) r = __fadd_rn(r, g.bias[gm]);
-                if (g.epi == 1) {
-                    if (g.round_out) r = nca::round_bf16(r);
-                    r = r > 0.0f ? r : 0.0f;
-                } else {
-                    if (g.round_out) r = nca::round_bf16(r);
-                    if (g.epi == 2) r = g.mask[gm * g.ldmask + gn] > 0.0f ? r : 0.0f;
-                }
-                if (g.accum) r = __fadd_rn(Cz[gm * g.ldc + gn], r);
-                Cz[gm * g.ldc + gn] = r;
-            }
-}
-
-int gemm(const GemmArgs &g, int splits, hipStream_t st) {
-    const int64_t gx = (g.N + GBN - 1) / GBN, gy = (g.M + GBM - 1) / GBM;
-    if (gx > 0x7fffffff || gy > 65535) return nca::set_error(NCA_ERR_UNSUPPORTED, "GEMM grid too large");
-    hipLaunchKernelGGL(gemm_f32_kernel, dim3((unsigned)gx, (unsigned)gy, (unsigned)splits), dim3(256), 0, st, g);
-    return nca::hip_status(hipGetLastError(), "gemm launch");
-}
-
 // loss_head: the call computes the chunk loss, which is the cross-entropy of an mlp head (a single
 // step's VJP has no loss term and takes any head).
 int check_dims(const nca_cell_desc *cell, int64_t rows, int32_t H, int32_t W, int32_t n, Dims *d,
@@ -1166,7 +1030,6 @@ int check_dims(const nca_cell_desc *cell, int64_t rows, int32_t H, int32_t W, in
     d->n_out = cell->n_out;
     d->padding = cell->padding;
     d->bf16 = cell->precision == NCA_BF16;
-    d->gz16 = 0;
     d->H = H;
     d->W = W;
     if ((int64_t)H * W * d->C > 0x7fffffff) return nca::set_error(NCA_ERR_UNSUPPORTED, "BPTT grid too large");
@@ -1189,9 +1052,14 @@ unsigned grid_for(int64_t n) {
 }  // namespace
 
 #include "nca_bptt_fused.h"
+#include "nca_bptt_step.h"
 
 namespace nca {
 int device_cus();
+}
+
+namespace {
+size_t backward_ws_bytes(const Dims &d, int n);
 }
 
 extern "C" {
@@ -1200,7 +1068,7 @@ size_t nca_bptt_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t
                                 int32_t n_chunk) {
     Dims d;
     if (nca_packed_weights_bytes(cell) == 0 || check_dims(cell, rows, height, width, n_chunk, &d)) return 0;
-    const size_t bwd = (size_t)ws_layout(d, n_chunk).total * sizeof(float);
+    const size_t bwd = backward_ws_bytes(d, n_chunk);
     // the forward's row exchange when its boards run in pieces (nca_bptt_forward_ws)
     const size_t xch = nca::recorded_xch_bytes(cell, rows, height, width);
     return bwd > xch ? bwd : xch;
@@ -1300,6 +1168,228 @@ FusedChoice fused_choice(const Dims &d, int n, bool fire_f32, const WsLayout &L)
     return c;
 }
 
+// Workspace (bytes, 256-aligned pieces after the status block) of the one-launch-per-step backward:
+// g_z of two consecutive steps, g_u, the kept z, h, g_a and g_dx of a group of `group` steps
+// (tile-major), the weight gradients' `splits` slots and the workgroups' slots.
+// The group is bounded to 256 MB (one step at least): beyond that the sums over a group no longer
+// save anything against their slots' traffic.
+struct StepLayout {
+    int64_t tiles;  // tiles of kBN cells per step
+    int group, splits, wgs, nslot, es;
+    size_t gz[2], gu, z, h, ga, gd, part, slots, denom, total;
+};
+
+StepLayout step_layout(const Dims &d, int n) {
+    StepLayout L;
+    const ParamLayout P = param_layout(d);
+    auto al = [](size_t v) { return (v + 255) & ~(size_t)255; };
+    L.es = d.bf16 ? 2 : 4;
+    L.tiles = (d.M + kBN - 1) / kBN;
+    const int64_t Mp = L.tiles * kBN, per = Mp * (d.F + 2 * d.HD + d.C) * L.es;
+    const int64_t fit = per > 0 ? ((int64_t)256 << 20) / per : 1;
+    L.group = fit < 1 ? 1 : fit < n ? (int)fit : n < 1 ? 1 : n;
+    const int64_t ld = L.group * Mp;
+    const int64_t tiles = (int64_t)(d.HD / 128) * (d.F / 64) + d.HD / 64;
+    int64_t sp = (1024 + tiles - 1) / tiles;
+    if (sp > ld / 256) sp = ld / 256;
+    L.splits = (int)(sp < 1 ? 1 : sp > kGroupSplits ? kGroupSplits : sp);
+    const int64_t pw = (L.tiles + kBackMaxWgs - 1) / kBackMaxWgs;  // tiles per workgroup
+    L.wgs = pw > 0 ? (int)((L.tiles + pw - 1) / pw) : 0;
+    L.nslot = 36 + d.n_out * d.c_out + d.n_out + 1;
+    size_t o = nca::kXchStatusBytes;
+    for (int k = 0; k < 2; ++k) {
+        L.gz[k] = o;
+        o = al(o + (size_t)d.M * d.F * L.es);
+    }
+    L.gu = o;
+    o = al(o + (size_t)d.M * d.C * sizeof(float));
+    L.z = o;
+    o = al(o + (size_t)d.F * ld * L.es);
+    L.h = o;
+    o = al(o + (size_t)d.HD * ld * L.es);
+    L.ga = o;
+    o = al(o + (size_t)d.HD * ld * L.es);
+    L.gd = o;
+    o = al(o + (size_t)d.C * ld * L.es);
+    L.part = o;
+    o = al(o + (size_t)L.splits * P.P * sizeof(float));
+    L.slots = o;
+    o = al(o + (size_t)L.wgs * L.nslot * sizeof(float));
+    L.denom = o;
+    o = al(o + sizeof(float));
+    L.total = o + 16;
+    return L;
+}
+
+size_t backward_ws_bytes(const Dims &d, int n) {
+    return fused_mlp(d) ? (size_t)ws_layout(d, n).total * sizeof(float) : step_layout(d, n).total;
+}
+
+GradOut grad_out(const ParamLayout &P, const Dims &d, const nca_cell_grads *grads) {
+    GradOut go;
+    float *gdst[7] = {grads->kernels, grads->w1, grads->b1, grads->w2, grads->b2, grads->head_w, grads->head_b};
+    const int64_t goff[7] = {P.K, P.W1, P.B1, P.W2, P.B2, P.HW, P.HB};
+    const int64_t gn[7] = {36, (int64_t)d.HD * d.F, d.HD, (int64_t)d.C * d.HD, d.C, (int64_t)d.n_out * d.c_out, d.n_out};
+    for (int k = 0; k < 7; ++k) {
+        go.dst[k] = gdst[k];
+        go.off[k] = goff[k];
+        go.n[k] = gn[k];
+    }
+    go.accumulate = grads->accumulate != 0;
+    return go;
+}
+
+template <int C, int HD, bool BF16, int NO>
+hipError_t launch_back_step(const BackStepArgs &a, int wgs, hipStream_t st) {
+    constexpr unsigned lds = BShape<C, HD, BF16>::END;
+    auto k = back_step<C, HD, BF16, NO>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3((unsigned)wgs), dim3(256), lds, st, a);
+    return hipGetLastError();
+}
+
+template <int C, int HD, bool BF16>
+hipError_t launch_steps_kernel(const Dims &d, const BackStepArgs *a, int wgs, const float *gu, const void *gz, const float *kern,
+                               float *gx0, hipStream_t st) {
+    if (a) return d.n_out <= 4 && d.c_out <= 4 ? launch_back_step<C, HD, BF16, 4>(*a, wgs, st)
+                                               : launch_back_step<C, HD, BF16, 16>(*a, wgs, st);
+    const int64_t items = d.M * (C / 4);
+    hipLaunchKernelGGL((back_x0<C, BF16>), dim3((unsigned)((items + 255) / 256)), dim3(256), 0, st, d, gu, gz, kern, gx0);
+    return hipGetLastError();
+}
+
+// back_step (a != NULL) or back_x0 of the cell
+hipError_t steps_kernel(const Dims &d, const BackStepArgs *a, int wgs, const float *gu, const void *gz, const float *kern,
+                        float *gx0, hipStream_t st) {
+    if (d.C == 16)
+        return d.bf16 ? launch_steps_kernel<16, 128, true>(d, a, wgs, gu, gz, kern, gx0, st)
+                      : launch_steps_kernel<16, 128, false>(d, a, wgs, gu, gz, kern, gx0, st);
+    if (d.C == 32)
+        return d.bf16 ? launch_steps_kernel<32, 256, true>(d, a, wgs, gu, gz, kern, gx0, st)
+                      : launch_steps_kernel<32, 256, false>(d, a, wgs, gu, gz, kern, gx0, st);
+    return d.bf16 ? launch_steps_kernel<64, 256, true>(d, a, wgs, gu, gz, kern, gx0, st)
+                  : launch_steps_kernel<64, 256, false>(d, a, wgs, gu, gz, kern, gx0, st);
+}
+
+int ws_error(size_t need) {
+    char msg[160];
+    snprintf(msg, sizeof(msg),
+             "the backward needs a workspace of %zu bytes (nca_bptt_workspace_bytes, "
+             "nca_step_backward_workspace_bytes)",
+             need);
+    return nca::set_error(NCA_ERR_INVALID, msg);
+}
+
+// The backward of n_chunk steps, one launch per step (nca_bptt_step.h); arguments as backward_impl's.
+int backward_steps(const Dims &d, const void *packed, const float *states, int64_t stride, const uint8_t *given,
+                   const nca_fire_desc *fire, const float *fire_f32, int32_t n_chunk, const nca_bptt_loss *loss,
+                   const float *grad_final, nca_cell_grads *grads, float *grad_x0, float *loss_out, void *workspace,
+                   size_t workspace_bytes, hipStream_t st) {
+    int rc = NCA_OK;
+    const StepLayout L = step_layout(d, n_chunk);
+    if (!workspace || workspace_bytes < L.total) return ws_error(L.total);
+    float wsum = 0.0f;
+    for (int t = 0; t < n_chunk; ++t) wsum += loss->step_weights[t];
+    const float wden = wsum < 1.0f ? 1.0f : wsum;  // weights.sum().clamp_min(1), engine.py:490
+    const ParamLayout P = param_layout(d);
+    const nca::PackedLayout PL = nca::packed_layout(d.C, 4, d.HD, d.c_out, d.n_out, d.bf16);
+    const unsigned char *pb = static_cast<const unsigned char *>(packed);
+    // 16-byte units from the first 16-byte boundary (the layout holds 16 bytes for it)
+    unsigned char *ws = static_cast<unsigned char *>(workspace) + (-reinterpret_cast<uintptr_t>(workspace) & 15u);
+    float *denom = reinterpret_cast<float *>(ws + L.denom), *part = reinterpret_cast<float *>(ws + L.part);
+    const int64_t sn = d.rows * d.C * (int64_t)d.HW;
+    if (loss->loss_mask && d.M > 0) hipLaunchKernelGGL(mask_sum, dim3(1), dim3(kThreads), 0, st, loss->loss_mask, d.M, denom);
+    if ((rc = nca::hip_status(hipGetLastError(), "bptt setup"))) return rc;
+    BackStepArgs a;
+    memset(&a, 0, sizeof(a));
+    a.f.d = d;
+    a.f.given = given;
+    a.f.targets = loss->targets;
+    a.f.mask = loss->loss_mask;
+    a.f.denom = denom;
+    a.f.head_w = reinterpret_cast<const float *>(pb + PL.headw);
+    a.f.head_b = reinterpret_cast<const float *>(pb + PL.headb);
+    a.f.fire_f32 = fire_f32;
+    a.f.key = fire->seed;
+    a.f.row0 = fire->row0;
+    a.f.p = fire->p_fire;
+    a.f.Gu = reinterpret_cast<float *>(ws + L.gu);
+    a.w1 = reinterpret_cast<const uint4 *>(pb + PL.bw1);
+    a.w1t = reinterpret_cast<const uint4 *>(pb + PL.bw1t);
+    a.w2t = reinterpret_cast<const uint4 *>(pb + PL.bw2t);
+    a.b1 = reinterpret_cast<const float *>(pb + PL.b1);
+    a.kern = reinterpret_cast<const float *>(pb + PL.kern);
+    a.padv = reinterpret_cast<const float *>(pb + PL.padv);
+    a.zs = ws + L.z;
+    a.hs = ws + L.h;
+    a.gas = ws + L.ga;
+    a.gds = ws + L.gd;
+    a.slots = reinterpret_cast<float *>(ws + L.slots);
+    a.nslot = L.nslot;
+    a.tiles = L.tiles;
+    WeightGradArgs wa;
+    memset(&wa, 0, sizeof(wa));
+    wa.ga = ws + L.ga;
+    wa.z = ws + L.z;
+    wa.gd = ws + L.gd;
+    wa.h = ws + L.h;
+    wa.C = d.C;
+    wa.F = d.F;
+    wa.HD = d.HD;
+    wa.splits = L.splits;
+    wa.part = part;
+    wa.P = P.P;
+    wa.offW1 = P.W1;
+    wa.offB1 = P.B1;
+    wa.offW2 = P.W2;
+    wa.offB2 = P.B2;
+    const bool work = n_chunk > 0 && d.M > 0;
+    // the status word of the other cells' one-launch backward: zero (cleared by the first launch)
+    a.status = static_cast<uint32_t *>(workspace) + 2;
+    if (!work) hipLaunchKernelGGL(zero_f32, dim3(1), dim3(64), 0, st, reinterpret_cast<float *>(a.status), (int64_t)1);
+    int kept = 0;
+    for (int t = n_chunk - 1; t >= 0 && work; --t) {
+        a.xt = states + t * stride;
+        a.f.x1 = states + (t + 1) * stride;
+        a.f.gin = t == n_chunk - 1 ? grad_final : nullptr;
+        a.gz_in = t == n_chunk - 1 ? nullptr : ws + L.gz[(t + 1) & 1];
+        a.gz_out = ws + L.gz[t & 1];
+        const float wt = loss->step_weights[t] / wden;
+        a.f.wscale = loss->loss_mask ? wt : wt / (float)d.M;
+        a.f.fire_u8 = fire->fire_in ? fire->fire_in + (int64_t)t * d.rows * d.HW : nullptr;
+        a.f.key_ptr = fire->step_seeds ? fire->step_seeds + t : nullptr;
+        a.f.step = (uint32_t)(fire->step0 + t);
+        a.tile0 = kept * L.tiles;
+        a.accum = t != n_chunk - 1;
+        if ((rc = nca::hip_status(steps_kernel(d, &a, L.wgs, nullptr, nullptr, nullptr, nullptr, st), "back_step"))) return rc;
+        if (++kept == L.group || t == 0) {
+            wa.K = kept * L.tiles;
+            wa.kps = (wa.K + L.splits - 1) / L.splits;
+            const unsigned tiles = (unsigned)((d.HD / 128) * (d.F / 64) + d.HD / 64);
+            hipLaunchKernelGGL(d.bf16 ? weight_grads<true> : weight_grads<false>, dim3((L.splits + 7) / 8 * 8 * tiles), dim3(256),
+                               0, st, wa);
+            if ((rc = nca::hip_status(hipGetLastError(), "weight_grads"))) return rc;
+            wa.accum = 1;
+            kept = 0;
+        }
+    }
+    if (grad_x0) {
+        if (work) {
+            if ((rc = nca::hip_status(steps_kernel(d, nullptr, 0, a.f.Gu, ws + L.gz[0], a.kern, grad_x0, st), "back_x0"))) return rc;
+        } else if (grad_final) {
+            hipLaunchKernelGGL(copy_kernel, dim3(256), dim3(256), 0, st, grad_final, grad_x0, sn);
+        } else {
+            hipLaunchKernelGGL(zero_f32, dim3(256), dim3(256), 0, st, grad_x0, sn);
+        }
+    }
+    const int nbig = (int)((P.HW - P.W1 + 255) / 256);
+    hipLaunchKernelGGL(back_finish, dim3((unsigned)(nbig + (L.nslot + 3) / 4)), dim3(256), 0, st, part, P.P,
+                       work ? L.splits : 0, a.slots, L.nslot, work ? L.wgs : 0, nbig, P.K, P.W1, P.HW, P.HW,
+                       grad_out(P, d, grads), loss_out);
+    return nca::hip_status(hipGetLastError(), "bptt finish");
+}
+
 // The backward of n_chunk steps (nca_bptt_backward). Step t reads its input state at
 // states + t * stride and its output at states + (t + 1) * stride; stride 0 (the single-step VJP,
 // which has no loss term) reads `states` for both. fire_f32, when given, is the (rows, H, W) fire
@@ -1310,16 +1400,12 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
                   const float *fire_f32, int32_t n_chunk, const nca_bptt_loss *loss, const float *grad_final,
                   nca_cell_grads *grads, float *grad_x0, float *loss_out, void *workspace, size_t workspace_bytes,
                   hipStream_t st) {
+    if (!fused_mlp(d))
+        return backward_steps(d, packed, states, stride, given, fire, fire_f32, n_chunk, loss, grad_final, grads, grad_x0,
+                              loss_out, workspace, workspace_bytes, st);
     int rc = NCA_OK;
     const WsLayout L = ws_layout(d, n_chunk);
-    if (!workspace || workspace_bytes < (size_t)L.total * sizeof(float)) {
-        char msg[160];
-        snprintf(msg, sizeof(msg),
-                 "the backward needs a workspace of %zu bytes (nca_bptt_workspace_bytes, "
-                 "nca_step_backward_workspace_bytes)",
-                 (size_t)L.total * sizeof(float));
-        return nca::set_error(NCA_ERR_INVALID, msg);
-    }
+    if (!workspace || workspace_bytes < (size_t)L.total * sizeof(float)) return ws_error((size_t)L.total * sizeof(float));
     float wsum = 0.0f;
     for (int t = 0; t < n_chunk; ++t) wsum += loss->step_weights[t];
     const float wden = wsum < 1.0f ? 1.0f : wsum;  // weights.sum().clamp_min(1), engine.py:490
@@ -1332,7 +1418,7 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
     const float *headb = reinterpret_cast<const float *>(pb + PL.headb);
     const float *padv = reinterpret_cast<const float *>(pb + PL.padv);
     float *ws = static_cast<float *>(workspace);
-    float *Z = ws + L.Z, *Hb = ws + L.Hb, *Ga = ws + L.Ga, *Gz = ws + L.Gz, *Gdx = ws + L.Gdx;
+    float *Z = ws + L.Z, *Gz = ws + L.Gz, *Gdx = ws + L.Gdx;
     float *Gu = ws + L.Gu, *Gx[2] = {ws + L.Gx0, ws + L.Gx1}, *part = ws + L.part, *acc = ws + L.acc;
     float *lossacc = ws + L.lossacc, *denom = ws + L.denom;
     const int64_t sn = d.rows * d.C * (int64_t)d.HW;
@@ -1342,7 +1428,6 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
     const FusedChoice fc = fused_choice(d, n_chunk, fire_f32 != nullptr, L);
     uint64_t *const wsw = static_cast<uint64_t *>(workspace);
     const int64_t xch_words = fc.pieces > 1 ? (int64_t)(fc.xch_bytes / sizeof(uint64_t)) - 1 : 0;
-    const bool fused = fused_mlp(d);
     if (fc.pieces > 0) {
         // the one-launch backward writes every value of its workgroups' slots (and the finish
         // launch writes acc): only the slots beyond them, the exchange words and the status word
@@ -1355,14 +1440,10 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
         hipLaunchKernelGGL(zero_f32_words, dim3(2048), dim3(256), 0, st, part, L.denom - L.part, wsw + 1, xch_words);
     }
     auto mlp_kfn = (d.M & 3) == 0 ? nca::mlp_back32<true> : nca::mlp_back32<false>;
-    if (fused && (rc = nca::hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(mlp_kfn),
-                                                           hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                           (int)nca::Mb32::TOTAL),
-                                       "mlp_back32 attribute")))
+    if ((rc = nca::hip_status(hipFuncSetAttribute(reinterpret_cast<const void *>(mlp_kfn),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)nca::Mb32::TOTAL),
+                              "mlp_back32 attribute")))
         return rc;
-    // the stencil kernels read g_z as bf16 where the fused kernel writes it
-    Dims ds = d;
-    ds.gz16 = fused ? 1 : 0;
     // boards small enough to stage (row, channel) planes in LDS
     const bool planes_ok = planes_fit(d);
     // ... and walked by columns for boards at most 256 wide (kernel-weight slot per 4 planes)
@@ -1372,7 +1453,7 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
     const int64_t strip_blocks = (d.rows * d.C + kStripPlanes - 1) / kStripPlanes;
     // cells per workgroup of the fused kernel: whole 32-cell tiles
     const int per32 = (int)((((d.M + kSplit - 1) / kSplit) + 31) / 32 * 32);
-    if (fused && fc.pieces == 0)
+    if (fc.pieces == 0)
         hipLaunchKernelGGL(nca::mlp_back32_prep, dim3(nca::kMb32PrepBlocks), dim3(512), 0, st, w->w1, w->w2,
                            reinterpret_cast<unsigned char *>(ws + L.img));
     if (loss->loss_mask && d.M > 0) hipLaunchKernelGGL(mask_sum, dim3(1), dim3(kThreads), 0, st, loss->loss_mask, d.M, denom);
@@ -1498,93 +1579,42 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
         fa.offHB = P.HB;
         const int no = d.n_out > d.c_out ? d.n_out : d.c_out;
         // recompute z (and, in the MLP stage, h) from the saved state
-        if (fused && planes_ok) {  // front and z in one launch
+        if (planes_ok) {  // front and z in one launch
             auto fz = no <= 4 ? front_z_kernel<4> : no <= 8 ? front_z_kernel<8> : front_z_kernel<16>;
             hipLaunchKernelGGL(fz, dim3((unsigned)(kSplit * (d.C / kFrontCh) + d.rows * d.C)), dim3(kThreads),
                                zlds, st, fa, xt, kern, padv, Z);
-        } else if (planes_ok) {
-            auto front = no <= 4 ? front_kernel<4> : no <= 8 ? front_kernel<8> : front_kernel<16>;
-            hipLaunchKernelGGL(front, dim3(kSplit, d.C / kFrontCh), dim3(kThreads), 0, st, fa);
-            auto zfn = fused ? stencil_z_plane<true> : stencil_z_plane<false>;
-            hipLaunchKernelGGL(zfn, dim3((unsigned)(d.rows * d.C)), dim3(kThreads), zlds, st, d, xt, kern,
-                               padv, Z);
         } else {
             auto front = no <= 4 ? front_kernel<4> : no <= 8 ? front_kernel<8> : front_kernel<16>;
             hipLaunchKernelGGL(front, dim3(kSplit, d.C / kFrontCh), dim3(kThreads), 0, st, fa);
             const dim3 zgrid(grid_for((int64_t)d.C * d.HW), (unsigned)(d.rows < 65535 ? d.rows : 65535));
-            hipLaunchKernelGGL(fused ? stencil_z_kernel<true> : stencil_z_kernel<false>, zgrid, dim3(kThreads), 0, st, d,
-                               xt, kern, padv, Z);
+            hipLaunchKernelGGL(stencil_z_kernel, zgrid, dim3(kThreads), 0, st, d, xt, kern, padv, Z);
         }
         if ((rc = nca::hip_status(hipGetLastError(), "bptt front / stencil"))) return rc;
-        GemmArgs g;
-        if (fused) {
-            nca::MlpBackArgs ma;
-            ma.Z = reinterpret_cast<const uint16_t *>(Z);
-            ma.Gdx = Gdx;
-            ma.img = reinterpret_cast<const unsigned char *>(ws + L.img);
-            ma.b1 = b1;
-            ma.Gz = reinterpret_cast<uint16_t *>(Gz);
-            ma.part = part;
-            ma.P = P.P;
-            ma.offW1 = P.W1;
-            ma.offB1 = P.B1;
-            ma.offW2 = P.W2;
-            ma.M = d.M;
-            ma.per = per32;
-            hipLaunchKernelGGL(mlp_kfn, dim3(kSplit), dim3(512), nca::Mb32::TOTAL, st, ma);
-            if ((rc = nca::hip_status(hipGetLastError(), "mlp_back32"))) return rc;
-        } else {
-            memset(&g, 0, sizeof(g));
-            // h = relu(W1 z + b1): (HD x F) (F x M)
-            g.A = w->w1; g.sam = d.F; g.sak = 1;
-            g.B = Z; g.sbk = d.M; g.sbn = 1;
-            g.Cm = Hb; g.ldc = d.M; g.M = d.HD; g.N = d.M; g.K = d.F; g.kps = d.F;
-            g.bias = b1; g.epi = 1; g.round_in = d.bf16; g.round_out = d.bf16;
-            if ((rc = gemm(g, 1, st))) return rc;
-            // g_a = (W2^T g_dx) * [h > 0]: (HD x C) (C x M)
-            memset(&g, 0, sizeof(g));
-            g.A = w->w2; g.sam = 1; g.sak = d.HD;
-            g.B = Gdx; g.sbk = d.M; g.sbn = 1;
-            g.Cm = Ga; g.ldc = d.M; g.M = d.HD; g.N = d.M; g.K = d.C; g.kps = d.C;
-            g.mask = Hb; g.ldmask = d.M; g.epi = 2; g.round_in = d.bf16; g.round_out = d.bf16;
-            if ((rc = gemm(g, 1, st))) return rc;
-            // g_z = W1^T g_a: (F x HD) (HD x M)
-            memset(&g, 0, sizeof(g));
-            g.A = w->w1; g.sam = 1; g.sak = d.F;
-            g.B = Ga; g.sbk = d.M; g.sbn = 1;
-            g.Cm = Gz; g.ldc = d.M; g.M = d.F; g.N = d.M; g.K = d.HD; g.kps = d.HD;
-            g.round_in = d.bf16; g.round_out = d.bf16;
-            if ((rc = gemm(g, 1, st))) return rc;
-        }
+        nca::MlpBackArgs ma;
+        ma.Z = reinterpret_cast<const uint16_t *>(Z);
+        ma.Gdx = Gdx;
+        ma.img = reinterpret_cast<const unsigned char *>(ws + L.img);
+        ma.b1 = b1;
+        ma.Gz = reinterpret_cast<uint16_t *>(Gz);
+        ma.part = part;
+        ma.P = P.P;
+        ma.offW1 = P.W1;
+        ma.offB1 = P.B1;
+        ma.offW2 = P.W2;
+        ma.M = d.M;
+        ma.per = per32;
+        hipLaunchKernelGGL(mlp_kfn, dim3(kSplit), dim3(512), nca::Mb32::TOTAL, st, ma);
+        if ((rc = nca::hip_status(hipGetLastError(), "mlp_back32"))) return rc;
         // gradient of the step's input state and the kernel-weight partials
-        auto strip_fn = fused ? stencil_back_strip<true> : stencil_back_strip<false>;
         if (strips_ok)
-            hipLaunchKernelGGL(strip_fn, dim3((unsigned)strip_blocks), dim3(kThreads), 6 * d.HW * sizeof(float), st, ds,
+            hipLaunchKernelGGL(stencil_back_strip, dim3((unsigned)strip_blocks), dim3(kThreads), 6 * d.HW * sizeof(float), st, d,
                                xt, Gu, Gz, kern, padv, gx, ws + L.dk);
         else if (planes_ok)
             hipLaunchKernelGGL(stencil_back_plane, dim3((unsigned)(d.rows * d.C)), dim3(kThreads),
-                               5 * d.HW * sizeof(float), st, ds, xt, Gu, Gz, kern, padv, gx, ws + L.dk);
+                               5 * d.HW * sizeof(float), st, d, xt, Gu, Gz, kern, padv, gx, ws + L.dk);
         else
-            hipLaunchKernelGGL(stencil_back_kernel, dim3(kSplit), dim3(kBackThreads), 0, st, ds, xt, Gu, Gz, kern, padv,
+            hipLaunchKernelGGL(stencil_back_kernel, dim3(kSplit), dim3(kBackThreads), 0, st, d, xt, Gu, Gz, kern, padv,
                                gx, part, P.P, P.K);
-        if (!fused) {
-            // weight-gradient partials over kSplit cell ranges
-            const int64_t kps = (((d.M + kSplit - 1) / kSplit) + GBK - 1) / GBK * GBK;
-            memset(&g, 0, sizeof(g));
-            g.A = Ga; g.sam = d.M; g.sak = 1;  // dW1 = g_a z^T: (HD x M) (M x F)
-            g.B = Z; g.sbk = 1; g.sbn = d.M;
-            g.Cm = part + P.W1; g.ldc = d.F; g.csplit = P.P; g.M = d.HD; g.N = d.F; g.K = d.M; g.kps = kps;
-            g.accum = 1;
-            if ((rc = gemm(g, kSplit, st))) return rc;
-            memset(&g, 0, sizeof(g));
-            g.A = Gdx; g.sam = d.M; g.sak = 1;  // dW2 = g_dx h^T: (C x M) (M x HD)
-            g.B = Hb; g.sbk = 1; g.sbn = d.M;
-            g.Cm = part + P.W2; g.ldc = d.HD; g.csplit = P.P; g.M = d.C; g.N = d.HD; g.K = d.M; g.kps = kps;
-            g.accum = 1;
-            if ((rc = gemm(g, kSplit, st))) return rc;
-            hipLaunchKernelGGL(rowsum_kernel, dim3((d.HD + 3) / 4, kSplit), dim3(kThreads), 0, st, Ga, d.M, d.HD, part,
-                               P.P, P.B1);
-        }
         if ((rc = nca::hip_status(hipGetLastError(), "bptt step kernels"))) return rc;
         gin = gx;
     }
@@ -1595,16 +1625,7 @@ int backward_impl(const Dims &d, const void *packed, const nca_cell_weights *w,
         }
     }
     // the gradients in the reference's parameter layouts (written, or added to the caller's)
-    GradOut go;
-    float *gdst[7] = {grads->kernels, grads->w1, grads->b1, grads->w2, grads->b2, grads->head_w, grads->head_b};
-    const int64_t goff[7] = {P.K, P.W1, P.B1, P.W2, P.B2, P.HW, P.HB};
-    const int64_t gn[7] = {36, (int64_t)d.HD * d.F, d.HD, (int64_t)d.C * d.HD, d.C, (int64_t)d.n_out * d.c_out, d.n_out};
-    for (int k = 0; k < 7; ++k) {
-        go.dst[k] = gdst[k];
-        go.off[k] = goff[k];
-        go.n[k] = gn[k];
-    }
-    go.accumulate = grads->accumulate != 0;
+    const GradOut go = grad_out(P, d, grads);
     const bool has_loss = n_chunk > 0 && d.M > 0;
     if (planes_ok && fc.pieces == 0) {
         // the slots summed in slot order, the strips' kernel-weight sums added, then the gradients
@@ -1651,7 +1672,7 @@ int nca_bptt_backward(const nca_cell_desc *cell, const void *packed, const nca_c
 size_t nca_step_backward_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t height, int32_t width) {
     Dims d;
     if (nca_packed_weights_bytes(cell) == 0 || check_dims(cell, rows, height, width, 1, &d, false)) return 0;
-    return (size_t)ws_layout(d, 1).total * sizeof(float);
+    return backward_ws_bytes(d, 1);
 }
 
 int nca_step_backward(const nca_cell_desc *cell, const void *packed, const nca_cell_weights *w, int64_t rows,

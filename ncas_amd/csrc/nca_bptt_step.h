@@ -1,0 +1,666 @@
+// One step of the BPTT backward in one launch, for every cell that mlp_back32 does not take (C = 16
+// and 64 in both precisions, C = 32 in fp32), and the weight gradients of several steps in one
+// more.
+//
+// `back_step`: a workgroup of 4 waves owns tiles of 32 consecutive cells (m = row * HW + q). For a
+// tile it
+//   1. finishes the gradient of the step's output state: the later step's g_u plus the transposed
+//      stencil of its g_z (of this cell's neighbours, written by the previous launch), the loss
+//      head's gradient, the clamp's and the fire mask's backward -> g_u, g_dx;
+//   2. recomputes z from the step's input state (9 taps, 4 kernels);
+//   3. on MFMA, wave w for a quarter of the hidden units: h = relu(W1 z + b1), g_a = (W2^T g_dx)
+//      [h > 0]; then for a quarter of the features g_z = W1^T g_a;
+//   4. adds the kernel-weight, head and loss sums of its cells into its own slots.
+// Only g_z crosses workgroups, and only from one launch to the next, so a step is one launch. It is
+// bound by latency at training sizes (10,368 cells of 9x9 are 324 tiles for 256 CUs): the weight
+// fragments come from the L2 once per tile, 16 bytes a lane, instead of staying in registers, so
+// that two workgroups fit a CU and the fp32 C = 64 cell (576 KB of weights) runs the same code.
+//
+// z, h, g_a and g_dx of up to G steps are kept tile-major ([tile][feature][32 cells]: a tile's
+// stores are one contiguous run, and so are 16 features of 32 cells, an MFMA operand), and
+// `weight_grads` sums dW1 = g_a z^T, dW2 = g_dx h^T, db1 and db2 over all their cells at once: a
+// split-K product over G * M cells writes its partial sums once per group where one over each
+// step's M cells read and wrote all of them every step (84 MB a step for C = 64).
+//
+// Against the five GEMM launches, row sums, front, stencil and strip kernels that did a step
+// before (128 boards of 9x9, C = 64, bf16, 32 steps: 665 -> 75 us a step and 93 us per group of 13
+// steps, a chunk 21.3 -> 3.5 ms; 64 boards of 13x13, C = 16, fp32: 117 -> 27 us a step and 100 us
+// per group of 18, 4.6 -> 1.9 ms).
+#pragma once
+
+#include "nca_device.h"
+
+namespace {
+
+constexpr int kBN = 32;            // cells per tile of back_step
+constexpr int kBackMaxWgs = 512;   // workgroups of back_step (two per CU), each with slots of its own
+constexpr int kGroupSplits = 256;  // most K ranges (slots) of weight_grads
+
+template <int C, int HD, bool BF16>
+struct BShape {
+    static constexpr int F = 4 * C;
+    static constexpr int ES = BF16 ? 2 : 4;     // bytes per element of z, h, g_a, g_dx, g_z
+    static constexpr int EB = 16 / ES;          // elements in a lane's 16 bytes
+    static constexpr int KB = 4 * EB;           // k per fragment block (16 rows x KB)
+    static constexpr int KF = F / KB;           // blocks of fc1's k axis
+    static constexpr int KC = (C + KB - 1) / KB;  // of W2^T's (zero-padded for bf16 C = 16)
+    static constexpr int KH = HD / KB;          // of W1^T's
+    static constexpr int MT1 = HD / 64;         // hidden m-tiles per wave
+    static constexpr int MT2 = F / 64;          // feature m-tiles per wave
+    static constexpr int ZS = F + EB, GS = HD + EB, DS = KC * KB + EB;  // LDS row strides (elements)
+    static constexpr int NZ = kBN * (C / 4) / 256 > 0 ? kBN * (C / 4) / 256 : 1;  // items per thread
+    static constexpr int ITEMS = kBN * (C / 4);
+    static constexpr unsigned Z = 0, H = Z + kBN * ZS * ES, GA = H + kBN * GS * ES, GZ = GA + kBN * GS * ES,
+                              GD = GZ + kBN * ZS * ES, END = GD + kBN * DS * ES;
+    // LDS column of MFMA operand row element k: a lane reads its 16 bytes of a block at 16 g. fp32: lane
+    // group g's element j is k = 4 j + g of the 16, so that the k axis is summed in ascending fours
+    static __device__ __forceinline__ int col(int k) { return BF16 ? k : (k & ~15) | ((k & 3) << 2) | ((k >> 2) & 3); }
+};
+
+// Fragment images in the packed weights (nca_layout.h): [m-tile][k-block][lane] 16-byte units.
+template <bool BF16>
+struct BFrag;
+template <>
+struct BFrag<true> {
+    typedef nca::bf16x8 type;
+    static __device__ __forceinline__ nca::f32x4 mma(type a, type b, nca::f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct BFrag<false> {
+    typedef nca::f32x4 type;
+    // slot j of lane group g is k = 4 j + g in both operands
+    static __device__ __forceinline__ nca::f32x4 mma(type a, type b, nca::f32x4 c) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j], c, 0, 0, 0);
+        return c;
+    }
+};
+
+template <bool BF16>
+__device__ __forceinline__ void put4(unsigned char *p, const float v[4]) {
+    if (BF16)
+        *reinterpret_cast<uint2 *>(p) = make_uint2(nca::pack_bf16x2(v[0], v[1]), nca::pack_bf16x2(v[2], v[3]));
+    else
+        *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+template <bool BF16>
+__device__ __forceinline__ void get4(const unsigned char *p, float v[4]) {
+    if (BF16) {
+        const uint2 u = *reinterpret_cast<const uint2 *>(p);
+        v[0] = nca::bf16_lo(u.x), v[1] = nca::bf16_hi(u.x), v[2] = nca::bf16_lo(u.y), v[3] = nca::bf16_hi(u.y);
+    } else {
+        const float4 u = *reinterpret_cast<const float4 *>(p);
+        v[0] = u.x, v[1] = u.y, v[2] = u.z, v[3] = u.w;
+    }
+}
+template <bool BF16>
+__device__ __forceinline__ float rnd(float v) { return BF16 ? nca::round_bf16(v) : v; }
+
+struct BackStepArgs {
+    FrontArgs f;             // x1, gin (NCHW, the chunk's last step only), targets, masks, head; Gu: (M, C)
+    const float *xt;         // the step's input state (rows, C, H, W)
+    const void *gz_in;       // g_z of the later step (M, F), or null
+    void *gz_out;            // (M, F)
+    const uint4 *w1, *w1t, *w2t;
+    const float *b1, *kern, *padv;
+    void *zs, *hs, *gas, *gds;  // kept buffers, [tile][feature][32 cells], this step's tiles from tile0
+    int64_t tile0;
+    float *slots;            // (workgroups, nslot): dK (36), dhead, head bias, loss
+    int nslot, accum;        // accum: add to the slots' contents
+    int64_t tiles;
+    uint32_t *status;        // the workspace's backward status word, cleared by the first launch
+};
+
+// acc[mt][nt] += A B over KB-blocks [0, K): A fragments from global memory (two k-blocks in flight),
+// B rows from LDS.
+template <bool BF16, int MT, int K>
+__device__ __forceinline__ void tile_mma(const uint4 *img, int mt0, const unsigned char *b, int stride_bytes, int lane,
+                                         nca::f32x4 (&acc)[MT][2]) {
+    typedef typename BFrag<BF16>::type fr;
+    constexpr int CK = K % 2 == 0 ? 2 : 1;
+    uint4 cur[MT][CK], nxt[MT][CK];
+    const uint4 *base = img + ((int64_t)mt0 * K) * 64 + lane;
+    const unsigned char *br = b + (lane & 15) * stride_bytes + 16 * (lane >> 4);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int c = 0; c < CK; ++c) cur[m][c] = base[(m * K + c) * 64];
+#pragma unroll 1
+    for (int k = 0; k < K; k += CK) {
+        const int kn = k + CK < K ? k + CK : k;  // (the last round reloads its own blocks)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < CK; ++c) nxt[m][c] = base[(m * K + kn + c) * 64];
+#pragma unroll
+        for (int c = 0; c < CK; ++c) {
+            fr bv[2];
+#pragma unroll
+            for (int n = 0; n < 2; ++n)
+                bv[n] = *reinterpret_cast<const fr *>(br + 16 * n * stride_bytes + 64 * (k + c));
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) acc[m][n] = BFrag<BF16>::mma(__builtin_bit_cast(fr, cur[m][c]), bv[n], acc[m][n]);
+        }
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int c = 0; c < CK; ++c) cur[m][c] = nxt[m][c];
+    }
+}
+
+// The gradient reaching cell (i, j) of board row `row`, channels [c0, c0 + 4), from the later step:
+// its g_u plus the transposed stencil of its g_z (M, F). The loads of
+// a row of neighbours are issued before its sums; a neighbour beyond a wall or zero border contributes nothing.
+template <int C, bool BF16>
+__device__ __forceinline__ void later_grad(const Dims &d, const float *Gu, const void *Gz, const float *kern, int64_t mrow,
+                                           int i, int j, int c0, float g[4]) {
+    constexpr int F = 4 * C, ES = BF16 ? 2 : 4;
+    const unsigned char *gz = static_cast<const unsigned char *>(Gz);
+    float4 g4 = *reinterpret_cast<const float4 *>(Gu + (mrow + i * d.W + j) * C + c0);
+    g[0] = g4.x, g[1] = g4.y, g[2] = g4.z, g[3] = g4.w;
+#pragma unroll 1
+    for (int t3 = 0; t3 < 3; ++t3) {
+        float v[3][4][4];
+        bool in[3];
+#pragma unroll
+        for (int t1 = 0; t1 < 3; ++t1) {
+            // the cell whose tap (t3, t1) reads this cell
+            const int q = neighbour(i, j, 1 - t3, 1 - t1, d.H, d.W, d.padding);
+            in[t1] = q >= 0;
+            const int64_t m = mrow + (q < 0 ? 0 : q);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) get4<BF16>(gz + (m * F + k * C + c0) * ES, v[t1][k]);
+        }
+#pragma unroll
+        for (int t1 = 0; t1 < 3; ++t1)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float w = kern[k * 9 + t3 * 3 + t1];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) g[c] = in[t1] ? __builtin_fmaf(w, v[t1][k][c], g[c]) : g[c];
+            }
+    }
+}
+
+// The 9 taps of channels [c0, c0 + 4) of cell (i, j) of a board row (rounded to bf16 for bf16 cells).
+template <int C, bool BF16>
+__device__ __forceinline__ void cell_taps(const Dims &d, const float *xt, const float *padv, int row, int i, int j, int c0,
+                                          float xv[4][9]) {
+    const float *xr = xt + ((int64_t)row * C + c0) * d.HW;
+    float hv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (d.padding == 1) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) hv[c] = padv[c0 + c];
+    }
+#pragma unroll
+    for (int t = 0; t < 9; ++t) {
+        const int nq = neighbour(i, j, t / 3 - 1, t % 3 - 1, d.H, d.W, d.padding);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const float x = xr[(int64_t)c * d.HW + (nq < 0 ? 0 : nq)];
+            xv[c][t] = rnd<BF16>(nq >= 0 ? x : hv[c]);
+        }
+    }
+}
+
+// A tile's LDS rows (cells) out to a kept buffer, transposed to (feats, 32 cells), 16 bytes a lane.
+template <class S, bool BF16, bool PERM>
+__device__ __forceinline__ void flush_tile(const unsigned char *L, int stride, int feats, void *out, int64_t tile) {
+    constexpr int PARTS = kBN / S::EB;
+    uint4 *o = static_cast<uint4 *>(out) + tile * feats * PARTS;
+    for (int e = threadIdx.x; e < feats * PARTS; e += 256) {
+        const int part = e % PARTS, f = e / PARTS;
+        const unsigned char *src = L + (part * S::EB * stride + (PERM ? S::col(f) : f)) * S::ES;
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            w[i] = BF16 ? *reinterpret_cast<const uint16_t *>(src + 2 * i * stride * 2) |
+                              ((uint32_t)*reinterpret_cast<const uint16_t *>(src + (2 * i + 1) * stride * 2) << 16)
+                        : *reinterpret_cast<const uint32_t *>(src + i * stride * 4);
+        o[e] = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+}
+
+template <int C, int HD, bool BF16, int NO>
+__global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
+    using S = BShape<C, HD, BF16>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    // the head: weights [v][c] and transposed [c][v], bias; per cell: logit gradients, output channels
+    __shared__ __attribute__((aligned(16))) float hwL[NO * NO], hwT[NO][NO], hbL[NO], glL[kBN][NO], xoL[kBN][NO];
+    __shared__ float fireL[kBN], lossL[kBN], red[4 * 36];
+    __shared__ int givenL[kBN], rowL[kBN], iL[kBN], jL[kBN];
+    unsigned char *ZL = smem + S::Z, *HL = smem + S::H, *GAL = smem + S::GA, *GZL = smem + S::GZ, *GDL = smem + S::GD;
+    const Dims &d = a.f.d;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
+    const bool has_loss = a.f.wscale != 0.0f;
+    const int M = (int)d.M;
+    if (has_loss) {
+        for (int i = tid; i < NO * NO; i += 256) {
+            const int v = i / NO, c = i - v * NO;
+            const float w = v < d.n_out && c < d.c_out ? a.f.head_w[v * d.c_out + c] : 0.0f;
+            hwL[i] = w;
+            hwT[c][v] = w;
+        }
+        if (tid < NO) hbL[tid] = tid < d.n_out ? a.f.head_b[tid] : 0.0f;
+    }
+    if (S::KC * S::KB > C)  // the zero part of g_dx's k axis
+        for (int i = tid; i < kBN * S::DS; i += 256) reinterpret_cast<uint16_t *>(GDL)[i] = 0;
+    float dk[36];
+#pragma unroll
+    for (int v = 0; v < 36; ++v) dk[v] = 0.0f;
+    if (!a.accum && blockIdx.x == 0 && tid == 0) *a.status = 0;
+    const int npw = d.n_out * d.c_out, np = npw + d.n_out;
+    float hs[2] = {0.0f, 0.0f}, lossv = 0.0f;
+
+    for (int64_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+        const int m0 = (int)(tile * kBN);
+        if (tid < kBN) {
+            const int m = m0 + tid < M ? m0 + tid : M - 1, row = m / d.HW, q = m - row * d.HW, i = q / d.W;
+            rowL[tid] = row;
+            iL[tid] = i;
+            jL[tid] = q - i * d.W;
+        }
+        __syncthreads();
+        // ---- per cell (wave 3): given flag and fire value; the head's output channels
+        if (has_loss) {
+#pragma unroll
+            for (int e = tid; e < kBN * NO; e += 256) {
+                const int n = e & (kBN - 1), c = e / kBN;
+                const int q = iL[n] * d.W + jL[n];
+                xoL[n][c] = c < d.c_out ? a.f.x1[((int64_t)rowL[n] * C + d.out_off + c) * d.HW + q] : 0.0f;
+            }
+        }
+        if (tid >= 192 && tid < 192 + kBN) {
+            const int n = tid - 192, m = m0 + n;
+            float f = 0.0f;
+            int gv = 0;
+            if (m < M) {
+                gv = a.f.given[m] != 0;
+                if (a.f.fire_f32) {
+                    f = a.f.fire_f32[m];
+                } else if (a.f.fire_u8) {
+                    f = a.f.fire_u8[m] ? 1.0f : 0.0f;
+                } else {
+                    const int q = iL[n] * d.W + jL[n], e4 = q & 3;
+                    float u[4];
+                    nca::cell_uniforms4(a.f.key_ptr ? *a.f.key_ptr : a.f.key, (uint32_t)(a.f.row0 + rowL[n]), a.f.step,
+                                        (uint32_t)(q >> 2), u);
+                    f = (e4 == 0 ? u[0] : e4 == 1 ? u[1] : e4 == 2 ? u[2] : u[3]) < a.f.p ? 1.0f : 0.0f;
+                }
+            }
+            fireL[n] = f;
+            givenL[n] = gv;
+        }
+        // ---- z: item (cell n, channel quad), lanes over cells
+#pragma unroll
+        for (int it = 0; it < S::NZ; ++it) {
+            const int e = tid + 256 * it, n = e & (kBN - 1), c0 = 4 * (e / kBN);
+            if (e >= S::ITEMS) continue;
+            const bool ok = m0 + n < M;
+            float xv[4][9];
+            cell_taps<C, BF16>(d, a.xt, a.padv, rowL[n], iL[n], jL[n], c0, xv);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float z[4];
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    float s = 0.0f;
+#pragma unroll
+                    for (int t = 0; t < 9; ++t) s = __builtin_fmaf(a.kern[k * 9 + t], xv[c][t], s);
+                    z[c] = ok ? rnd<BF16>(s) : 0.0f;
+                }
+                if (BF16) {
+                    put4<BF16>(ZL + (n * S::ZS + k * C + c0) * S::ES, z);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) reinterpret_cast<float *>(ZL)[n * S::ZS + S::col(k * C + c0 + c)] = z[c];
+                }
+            }
+        }
+        // ---- the gradient of the output state: item (cell n, channel quad), lanes over quads
+        float gg[S::NZ][4];
+#pragma unroll
+        for (int it = 0; it < S::NZ; ++it) {
+            const int e = tid + 256 * it, c0 = 4 * (e & (C / 4 - 1)), n = e / (C / 4);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) gg[it][c] = 0.0f;
+            if (e >= S::ITEMS || m0 + n >= M) continue;
+            const int row = rowL[n], i = iL[n], j = jL[n];
+            if (a.gz_in) {
+                later_grad<C, BF16>(d, a.f.Gu, a.gz_in, a.kern, (int64_t)row * d.HW, i, j, c0, gg[it]);
+            } else if (a.f.gin) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) gg[it][c] = a.f.gin[((int64_t)row * C + c0 + c) * d.HW + i * d.W + j];
+            }
+        }
+        __syncthreads();
+        // ---- the loss head: logits per (cell, class), then the soft-max gradient per cell
+        if (has_loss) {
+            for (int e = tid; e < kBN * NO; e += 256) {
+                const int n = e & (kBN - 1), v = e / kBN;
+                float acc = hbL[v];
+#pragma unroll
+                for (int c = 0; c < NO; ++c) acc = c < d.c_out ? __builtin_fmaf(hwL[v * NO + c], xoL[n][c], acc) : acc;
+                glL[n][v] = acc;
+            }
+            __syncthreads();
+            if (tid < kBN) {
+                const int n = tid, m = m0 + n < M ? m0 + n : M - 1;
+                float l[NO], gl[NO];
+#pragma unroll
+                for (int v = 0; v < NO; ++v) l[v] = glL[n][v];
+                const float lc = softmax_grad<NO>(d, a.f.wscale, a.f.mask != nullptr, a.f.denom, l, a.f.targets[m],
+                                                  a.f.mask ? a.f.mask[m] : 0.0f, gl);
+                const bool ok = m0 + n < M;
+                lossL[n] = ok ? lc : 0.0f;
+#pragma unroll
+                for (int v = 0; v < NO; ++v) glL[n][v] = ok ? gl[v] : 0.0f;
+            }
+            __syncthreads();
+        }
+        // ---- clamp and fire: g_u, g_dx
+#pragma unroll
+        for (int it = 0; it < S::NZ; ++it) {
+            const int e = tid + 256 * it, c0 = 4 * (e & (C / 4 - 1)), n = e / (C / 4);
+            if (e >= S::ITEMS) continue;
+            const bool gv = givenL[n] != 0, ok = m0 + n < M;
+            const float f = fireL[n];
+            float gd[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int ch = c0 + c, co = ch - d.out_off;
+                float v = gg[it][c];
+                if (has_loss && co >= 0 && co < d.c_out) {
+#pragma unroll
+                    for (int o = 0; o < NO; ++o) v = __builtin_fmaf(hwT[co][o], glL[n][o], v);
+                }
+                if (gv && ch >= d.in_off && ch < d.in_off + d.c_in) v = 0.0f;
+                gg[it][c] = v;
+                // bf16 cells: dx is a bf16 tensor, so its gradient is bf16
+                gd[c] = ok ? rnd<BF16>(v * f) : 0.0f;
+            }
+            if (BF16) {
+                put4<BF16>(GDL + (n * S::DS + c0) * S::ES, gd);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) reinterpret_cast<float *>(GDL)[n * S::DS + S::col(c0 + c)] = gd[c];
+            }
+        }
+        if (has_loss) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int p = tid + 256 * s;
+                if (p < np) {
+                    const int v = p < npw ? p / d.c_out : p - npw, c = p < npw ? p - v * d.c_out : -1;
+#pragma unroll 8
+                    for (int n = 0; n < kBN; ++n) hs[s] = __builtin_fmaf(glL[n][v], c < 0 ? 1.0f : xoL[n][c < 0 ? 0 : c], hs[s]);
+                }
+            }
+            if (tid == 255)
+#pragma unroll
+                for (int n = 0; n < kBN; ++n) lossv = __fadd_rn(lossv, lossL[n]);
+        }
+        __syncthreads();
+        // ---- h and g_a: wave w, hidden units [w HD / 4, (w + 1) HD / 4)
+        {
+            nca::f32x4 h[S::MT1][2], ga[S::MT1][2];
+#pragma unroll
+            for (int m = 0; m < S::MT1; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) h[m][n] = ga[m][n] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            tile_mma<BF16, S::MT1, S::KF>(a.w1, wave * S::MT1, ZL, S::ZS * S::ES, lane, h);
+            tile_mma<BF16, S::MT1, S::KC>(a.w2t, wave * S::MT1, GDL, S::DS * S::ES, lane, ga);
+#pragma unroll
+            for (int m = 0; m < S::MT1; ++m) {
+                const int hid = (wave * S::MT1 + m) * 16 + 4 * g;
+                const float4 b4 = *reinterpret_cast<const float4 *>(a.b1 + hid);
+                const float bb[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    const int cell = 16 * n + l16;
+                    float hr[4], gv[4];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const float hv = rnd<BF16>(__fadd_rn(h[m][n][v], bb[v]));
+                        hr[v] = hv > 0.0f ? hv : 0.0f;
+                        gv[v] = hr[v] > 0.0f ? rnd<BF16>(ga[m][n][v]) : 0.0f;
+                    }
+                    put4<BF16>(HL + (cell * S::GS + hid) * S::ES, hr);
+                    if (BF16) {
+                        put4<BF16>(GAL + (cell * S::GS + hid) * S::ES, gv);
+                    } else {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) reinterpret_cast<float *>(GAL)[cell * S::GS + S::col(hid + v)] = gv[v];
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        // ---- g_z: wave w, features [w F / 4, (w + 1) F / 4)
+        {
+            nca::f32x4 gz[S::MT2][2];
+#pragma unroll
+            for (int m = 0; m < S::MT2; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) gz[m][n] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            tile_mma<BF16, S::MT2, S::KH>(a.w1t, wave * S::MT2, GAL, S::GS * S::ES, lane, gz);
+#pragma unroll
+            for (int m = 0; m < S::MT2; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    const float v[4] = {gz[m][n][0], gz[m][n][1], gz[m][n][2], gz[m][n][3]};
+                    put4<BF16>(GZL + ((16 * n + l16) * S::ZS + (wave * S::MT2 + m) * 16 + 4 * g) * S::ES, v);
+                }
+        }
+        __syncthreads();
+        // ---- the kernel-weight sums (the taps again, from the caches)
+#pragma unroll
+        for (int it = 0; it < S::NZ; ++it) {
+            const int e = tid + 256 * it, n = e & (kBN - 1), c0 = 4 * (e / kBN);
+            if (e >= S::ITEMS || m0 + n >= M) continue;
+            float xv[4][9];
+            cell_taps<C, BF16>(d, a.xt, a.padv, rowL[n], iL[n], jL[n], c0, xv);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                float gv[4];
+                get4<BF16>(GZL + (n * S::ZS + k * C + c0) * S::ES, gv);
+#pragma unroll
+                for (int c = 0; c < 4; ++c)
+#pragma unroll
+                    for (int t = 0; t < 9; ++t) dk[k * 9 + t] = __builtin_fmaf(gv[c], xv[c][t], dk[k * 9 + t]);
+            }
+        }
+        // ---- everything out: stores last, so that no load of the tile waits behind them (they
+        // complete in order with the loads)
+#pragma unroll
+        for (int it = 0; it < S::NZ; ++it) {
+            const int e = tid + 256 * it, c0 = 4 * (e & (C / 4 - 1)), n = e / (C / 4);
+            if (e < S::ITEMS && m0 + n < M)
+                *reinterpret_cast<float4 *>(a.f.Gu + (int64_t)(m0 + n) * C + c0) =
+                    make_float4(gg[it][0], gg[it][1], gg[it][2], gg[it][3]);
+        }
+        constexpr int UPR = S::F * S::ES / 16;  // 16-byte units per cell of g_z
+        for (int u = tid; u < kBN * UPR; u += 256) {
+            const int n = u / UPR, o = u - n * UPR;
+            if (m0 + n < M)
+                reinterpret_cast<uint4 *>(a.gz_out)[(int64_t)(m0 + n) * UPR + o] =
+                    *reinterpret_cast<const uint4 *>(GZL + n * S::ZS * S::ES + 16 * o);
+        }
+        flush_tile<S, BF16, true>(ZL, S::ZS, S::F, a.zs, a.tile0 + tile);
+        flush_tile<S, BF16, false>(HL, S::GS, HD, a.hs, a.tile0 + tile);
+        flush_tile<S, BF16, true>(GAL, S::GS, HD, a.gas, a.tile0 + tile);
+        flush_tile<S, BF16, true>(GDL, S::DS, C, a.gds, a.tile0 + tile);
+        __syncthreads();
+    }
+    // ---- the workgroup's slots
+    float *sl = a.slots + (int64_t)blockIdx.x * a.nslot;
+    const float r = block_sums<36, 4>(dk, red);
+    if (tid < 36) sl[tid] = a.accum ? __fadd_rn(sl[tid], r) : r;
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int p = tid + 256 * s;
+        if (p < np) sl[36 + p] = a.accum ? __fadd_rn(sl[36 + p], hs[s]) : hs[s];
+    }
+    if (tid == 255) sl[36 + np] = a.accum ? __fadd_rn(sl[36 + np], lossv) : lossv;
+}
+
+// The gradient of the chunk's first state, (rows, C, H, W), from the first step's g_u and g_z.
+template <int C, bool BF16>
+__global__ void __launch_bounds__(256) back_x0(Dims d, const float *Gu, const void *Gz, const float *kern, float *gx) {
+    const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;  // (cell, channel quad), quads fastest
+    const int64_t m = e / (C / 4);
+    if (m >= d.M) return;
+    const int c0 = 4 * (int)(e - m * (C / 4));
+    const int64_t row = m / d.HW;
+    const int q = (int)(m - row * d.HW), i = q / d.W, j = q - i * d.W;
+    float g[4];
+    later_grad<C, BF16>(d, Gu, Gz, kern, row * d.HW, i, j, c0, g);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) gx[(row * C + c0 + c) * (int64_t)d.HW + q] = g[c];
+}
+
+struct WeightGradArgs {
+    const unsigned char *ga, *z, *gd, *h;  // [tile][feature][32 cells]
+    int64_t K, kps;  // tiles in use, per split
+    int C, F, HD, splits;
+    float *part;         // slot s: part + s P
+    int64_t P, offW1, offB1, offW2, offB2;
+    int accum;
+};
+
+// dW1 (HD x F) = g_a z^T, dW2 (C x HD) = g_dx h^T and the row sums db1 of g_a and db2 of g_dx over
+// the tiles [s kps, (s + 1) kps): a workgroup takes a 128 x 64 tile of dW1 (or up to 64 x 64 of
+// dW2), wave w its 64 x 32 part, for one s. A lane's 16 bytes of a tile's row are its MFMA
+// operand as they lie: no LDS. The kernel reads its operands once per
+// tile of the other one, so it is bound by those reads; the workgroups of one s have the same index
+// modulo 8, hence the same XCD and L2.
+template <bool BF16>
+__global__ void __launch_bounds__(256, 3) weight_grads(WeightGradArgs a) {
+    typedef typename BFrag<BF16>::type fr;
+    constexpr int ES = BF16 ? 2 : 4, KT = kBN * ES / 64;  // k-blocks (64 bytes of a row) per tile
+    constexpr int RA = 4, RB = 2;                   // 16-row blocks of A and B per wave
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, l16 = lane & 15;
+    const int nt1 = a.F / 64, t1 = (a.HD / 128) * nt1, nt = t1 + a.HD / 64;
+    const int grp = blockIdx.x / (8 * nt), rem = blockIdx.x - grp * 8 * nt;
+    const int t = rem >> 3, split = grp * 8 + (rem & 7);
+    if (split >= a.splits) return;
+    const bool first = t < t1;
+    const int tt = first ? t : t - t1;
+    const int ti = first ? tt / nt1 : 0, tj = first ? tt - ti * nt1 : tt;
+    const int r0 = 128 * ti + 64 * (wave >> 1), c0 = 64 * tj + 32 * (wave & 1);
+    const int rows = first ? a.HD : a.C, ldo = first ? a.F : a.HD;
+    const unsigned char *A = first ? a.ga : a.gd, *B = first ? a.z : a.h;
+    if (r0 >= rows) return;  // dW2 has at most 64 rows
+    const int nr = rows - r0 < 64 ? (rows - r0) / 16 : RA;  // row blocks in use
+    const bool bias = tj == 0 && (wave & 1) == 0;
+    // in k-blocks
+    const int64_t k0 = split * a.kps * KT, k1 = (split + 1) * a.kps < a.K ? k0 + a.kps * KT : a.K * KT;
+    const int64_t ta = (int64_t)rows * kBN * ES, tb = (int64_t)ldo * kBN * ES;  // bytes per tile
+    const unsigned char *pa[RA], *pb[RB];
+#pragma unroll
+    for (int r = 0; r < RA; ++r) pa[r] = A + (r0 + 16 * (r < nr ? r : 0) + l16) * kBN * ES + 16 * g;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) pb[r] = B + (c0 + 16 * r + l16) * kBN * ES + 16 * g;
+    nca::f32x4 acc[RA][RB], ab[RA];
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+        ab[r] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < RB; ++c) acc[r][c] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    fr ones;
+#pragma unroll
+    for (int i = 0; i < 16 / ES; ++i) ones[i] = 1.0f;
+    constexpr int U = 2;  // k-blocks in flight
+    uint4 va[U][RA], vb[U][RB];
+    auto load = [&](int u, int64_t k) {
+        const int64_t kk = k < k1 ? k : k0;  // a block past the range: loaded, not used
+        const int64_t oa = kk / KT * ta + kk % KT * 64, ob = kk / KT * tb + kk % KT * 64;
+#pragma unroll
+        for (int r = 0; r < RA; ++r) va[u][r] = *reinterpret_cast<const uint4 *>(pa[r] + oa);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) vb[u][r] = *reinterpret_cast<const uint4 *>(pb[r] + ob);
+    };
+    if (k0 < k1) {
+        load(0, k0);
+        load(1, k0 + 1);
+    }
+    for (int64_t k = k0; k < k1; k += U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k + u < k1) {  // uniform
+#pragma unroll
+                for (int r = 0; r < RA; ++r) {
+                    const fr av = __builtin_bit_cast(fr, va[u][r]);
+#pragma unroll
+                    for (int c = 0; c < RB; ++c) acc[r][c] = BFrag<BF16>::mma(av, __builtin_bit_cast(fr, vb[u][c]), acc[r][c]);
+                    if (bias) ab[r] = BFrag<BF16>::mma(av, ones, ab[r]);
+                }
+            }
+            load(u, k + U + u);
+        }
+    }
+    float *out = a.part + (int64_t)split * a.P + (first ? a.offW1 : a.offW2);
+    float *ob = a.part + (int64_t)split * a.P + (first ? a.offB1 : a.offB2);
+#pragma unroll
+    for (int r = 0; r < RA; ++r) {
+        if (r >= nr) break;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int row = r0 + 16 * r + 4 * g + v;
+#pragma unroll
+            for (int c = 0; c < RB; ++c) {
+                float *p = out + (int64_t)row * ldo + c0 + 16 * c + l16;
+                *p = a.accum ? __fadd_rn(*p, acc[r][c][v]) : acc[r][c][v];
+            }
+            if (bias && l16 == 0) ob[row] = a.accum ? __fadd_rn(ob[row], ab[r][v]) : ab[r][v];
+        }
+    }
+}
+
+// The chunk's gradients out of the slots: thread per MLP parameter (`splits` slots of part, in slot
+// order), wave per kernel weight, head parameter and the loss (`wgs` slots, lanes strided, then a
+// fixed fold). `nbig` workgroups do the former.
+__global__ void __launch_bounds__(256) back_finish(const float *part, int64_t P, int splits, const float *slots, int nslot,
+                                                   int wgs, int nbig, int64_t offK, int64_t lo, int64_t hi, int64_t offHW,
+                                                   GradOut go, float *loss_out) {
+    if ((int)blockIdx.x < nbig) {
+        const int64_t i = lo + blockIdx.x * (int64_t)256 + threadIdx.x;
+        if (i >= hi) return;
+        constexpr int kB = 32;
+        float s = 0.0f;
+        for (int k0 = 0; k0 < splits; k0 += kB) {
+            float v[kB];
+#pragma unroll
+            for (int k = 0; k < kB; ++k) v[k] = k0 + k < splits ? part[(int64_t)(k0 + k) * P + i] : 0.0f;
+#pragma unroll
+            for (int k = 0; k < kB; ++k)
+                if (k0 + k < splits) s = __fadd_rn(s, v[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < 7; ++k)
+            if (go.dst[k] && i >= go.off[k] && i < go.off[k] + go.n[k]) grad_put(go, k, i - go.off[k], s);
+        return;
+    }
+    const int v = (blockIdx.x - nbig) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (v >= nslot) return;
+    float s = 0.0f;
+    for (int w = lane; w < wgs; w += 64) s = __fadd_rn(s, slots[(int64_t)w * nslot + v]);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s = __fadd_rn(s, __shfl_xor(s, o));
+    if (lane != 0) return;
+    if (v == nslot - 1) {
+        if (loss_out) *loss_out = s;
+        return;
+    }
+    const int64_t i = v < 36 ? offK + v : offHW + (v - 36);
+#pragma unroll
+    for (int k = 0; k < 7; ++k)
+        if (go.dst[k] && i >= go.off[k] && i < go.off[k] + go.n[k]) grad_put(go, k, i - go.off[k], s);
+}
+
+}  // namespace

@@ -20,6 +20,11 @@
 //          each own a quarter and keep fc1's accumulators as the B operand:
 //          [q][m-tile][k-tile][lane][slot], A[i][slot] = W2[16 m + i][q hidden/4 +
 //          16 (2 k + slot / 4) + 4 (lane / 16) + slot % 4]
+//   bw1, bw1t, bw2t
+//          the backward's A operands W1 (hidden x F), W1^T (F x hidden) and W2^T (hidden x C, the
+//          k axis zero-padded to a block): [m-tile][k-block][lane] units of 16 bytes, a block 32 k
+//          (bf16) or 16 k (fp32), unit element s = A[i = lane % 16][block + 8 (lane / 16) + s] (bf16)
+//          or A[i][block + 4 s + lane / 16] (fp32)
 // bf16 cells use v_mfma_f32_16x16x32_bf16 fragments (k-tile 32, 8 bf16 slots per lane:
 // A[i = lane % 16][k = 8 * (lane / 16) + slot]); fp32 cells use v_mfma_f32_16x16x4_f32
 // fragments (k-tile 4, one float per lane: A[i = lane % 16][k = lane / 16]).
@@ -30,7 +35,7 @@
 namespace nca {
 
 struct PackedLayout {
-    size_t kern, b1, b2, headw, headb, padv, w1, w2, w2h, w1q, w2k, total;
+    size_t kern, b1, b2, headw, headb, padv, w1, w2, w2h, w1q, w2k, bw1, bw1t, bw2t, total;
 };
 
 __host__ __device__ inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -62,6 +67,13 @@ __host__ __device__ inline PackedLayout packed_layout(int C, int heads, int hidd
     o = align256(o + (bf16 ? 2 * (size_t)hidden * heads * C : 0));
     L.w2k = o;  // bf16 cells: fc2 fragments per hidden quarter
     o = align256(o + (bf16 ? 2 * (size_t)C * hidden : 0));
+    L.bw1 = o;
+    o = align256(o + esz * (size_t)hidden * heads * C);
+    L.bw1t = o;
+    o = align256(o + esz * (size_t)hidden * heads * C);
+    const size_t kblock = bf16 ? 32 : 16;
+    L.bw2t = o;
+    o = align256(o + esz * (size_t)hidden * ((C + kblock - 1) / kblock * kblock));
     L.total = o;
     return L;
 }
