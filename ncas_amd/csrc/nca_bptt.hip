@@ -281,18 +281,31 @@ __device__ __forceinline__ void load_out(const Dims &d, const float *x1c, float 
     for (int c = 0; c < NO; ++c) xo[c] = c < d.c_out ? v[c] : 0.0f;
 }
 
-// The cross-entropy gradient at a cell with logits l and target tgt: gl[v] = d loss / d logit v,
-// times the step's scale (and the loss-mask value mk over *denom); 0 for v >= n_out. Returns the
-// cell's loss term (reference src/nca/train.py:183-207). n_out <= NO.
+// The cross-entropy gradient of the mlp head's logits at a cell with output channels xo, target
+// tgt and loss-mask value mk (gl[v] = d loss / d logit v, times the step's scale; 0 for
+// v >= n_out, and everywhere on a step without a loss term) and the cell's loss term (reference
+// src/nca/train.py:183-207). n_out, c_out <= NO.
 template <int NO>
-__device__ __forceinline__ float softmax_grad(const Dims &d, float wscale, bool masked, const float *denom, const float l[NO],
-                                              int tgt, float mk, float gl[NO]) {
+__device__ __forceinline__ float head_grad_core(const Dims &d, float wscale, bool masked, const float *denom,
+                                                const float *hw, const float *hb, const float xo[NO], int tgt, float mk,
+                                                float gl[NO]) {
+#pragma unroll
+    for (int v = 0; v < NO; ++v) gl[v] = 0.0f;
+    if (wscale == 0.0f) return 0.0f;
     const float scale = masked ? wscale * mk / *denom : wscale;
+    float l[NO];
     float mx = -INFINITY;
 #pragma unroll
     for (int v = 0; v < NO; ++v) {
-        gl[v] = 0.0f;
-        if (v < d.n_out) mx = fmaxf(mx, l[v]);
+        l[v] = 0.0f;
+        if (v < d.n_out) {
+            float acc = hb[v];
+#pragma unroll
+            for (int c = 0; c < NO; ++c)
+                if (c < d.c_out) acc = __builtin_fmaf(hw[v * d.c_out + c], xo[c], acc);
+            l[v] = acc;
+            mx = fmaxf(mx, acc);
+        }
     }
     float s = 0.0f, lt = mx, e[NO];
 #pragma unroll
@@ -306,30 +319,6 @@ __device__ __forceinline__ float softmax_grad(const Dims &d, float wscale, bool 
     for (int v = 0; v < NO; ++v)
         if (v < d.n_out) gl[v] = (e[v] / s - (v == tgt ? 1.0f : 0.0f)) * scale;
     return (mx + logf(s) - lt) * scale;
-}
-
-// The same from the cell's output channels xo and the head's weights and bias (zero gradients on a
-// step without a loss term). n_out, c_out <= NO.
-template <int NO>
-__device__ __forceinline__ float head_grad_core(const Dims &d, float wscale, bool masked, const float *denom,
-                                                const float *hw, const float *hb, const float xo[NO], int tgt, float mk,
-                                                float gl[NO]) {
-#pragma unroll
-    for (int v = 0; v < NO; ++v) gl[v] = 0.0f;
-    if (wscale == 0.0f) return 0.0f;
-    float l[NO];
-#pragma unroll
-    for (int v = 0; v < NO; ++v) {
-        l[v] = 0.0f;
-        if (v < d.n_out) {
-            float acc = hb[v];
-#pragma unroll
-            for (int c = 0; c < NO; ++c)
-                if (c < d.c_out) acc = __builtin_fmaf(hw[v * d.c_out + c], xo[c], acc);
-            l[v] = acc;
-        }
-    }
-    return softmax_grad<NO>(d, wscale, masked, denom, l, tgt, mk, gl);
 }
 template <int NO>
 __device__ __forceinline__ float head_grad(const FrontArgs &a, const float *hw, const float *hb, const float xo[NO], int tgt,

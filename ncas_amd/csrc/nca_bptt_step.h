@@ -23,10 +23,15 @@
 // step's M cells read and wrote all of them every step (84 MB a step for C = 64).
 //
 // Against the five GEMM launches, row sums, front, stencil and strip kernels that did a step
-// before (128 boards of 9x9, C = 64, bf16, 32 steps: 665 -> 75 us a step and 93 us per group of 13
-// steps, a chunk 21.3 -> 3.5 ms; 64 boards of 13x13, C = 16, fp32: 117 -> 27 us a step and 100 us
-// per group of 18, 4.6 -> 1.9 ms).
+// before (128 boards of 9x9, C = 64, bf16, 32 steps: 665 -> 46 us a step and 97 us per group of 13
+// steps; 64 boards of 13x13, C = 16, fp32: 117 -> 22 us a step and 100 us per group of 18). Every
+// stage issues its loads before it uses the first (one at a time they took twice as long: the
+// compiler packs each pair of taps as it arrives), the weight fragments' loads are in flight
+// beside the head, the stores come last (a load waits for the stores issued before it), and the
+// LDS plan lets two workgroups share a CU (with one the 324 tiles take two rounds: 66 us).
 #pragma once
+
+#include <type_traits>
 
 #include "nca_device.h"
 
@@ -50,7 +55,9 @@ struct BShape {
     static constexpr int ZS = F + EB, GS = HD + EB, DS = KC * KB + EB;  // LDS row strides (elements)
     static constexpr int NZ = kBN * (C / 4) / 256 > 0 ? kBN * (C / 4) / 256 : 1;  // items per thread
     static constexpr int ITEMS = kBN * (C / 4);
-    static constexpr unsigned Z = 0, H = Z + kBN * ZS * ES, GA = H + kBN * GS * ES, GZ = GA + kBN * GS * ES,
+    // fp32 h goes straight to its kept buffer (64-byte runs): with it in LDS only one workgroup of the
+    // C = 32 cell would fit a CU
+    static constexpr unsigned Z = 0, H = Z + kBN * ZS * ES, GA = H + (BF16 ? kBN * GS * ES : 0), GZ = GA + kBN * GS * ES,
                               GD = GZ + kBN * ZS * ES, END = GD + kBN * DS * ES;
     // LDS column of MFMA operand row element k: a lane reads its 16 bytes of a block at 16 g. fp32: lane
     // group g's element j is k = 4 j + g of the 16, so that the k axis is summed in ascending fours
@@ -113,76 +120,83 @@ struct BackStepArgs {
     uint32_t *status;        // the workspace's backward status word, cleared by the first launch
 };
 
-// acc[mt][nt] += A B over KB-blocks [0, K): A fragments from global memory (two k-blocks in flight),
-// B rows from LDS.
+// A wave's weight fragments of one product: MT m-tiles, K k-blocks, of which up to PRE are in
+// registers: `load` issues the first ones (early, so that their latency passes beside other work),
+// `mma` adds A B to acc (B rows from LDS) and refills each slot once it is used.
 template <bool BF16, int MT, int K>
-__device__ __forceinline__ void tile_mma(const uint4 *img, int mt0, const unsigned char *b, int stride_bytes, int lane,
-                                         nca::f32x4 (&acc)[MT][2]) {
+struct WFrags {
     typedef typename BFrag<BF16>::type fr;
-    constexpr int CK = K % 2 == 0 ? 2 : 1;
-    uint4 cur[MT][CK], nxt[MT][CK];
-    const uint4 *base = img + ((int64_t)mt0 * K) * 64 + lane;
-    const unsigned char *br = b + (lane & 15) * stride_bytes + 16 * (lane >> 4);
+    static constexpr int PRE = K < (BF16 ? 8 : 4) ? K : (BF16 ? 8 : 4);
+    const uint4 *base;  // uniform
+    uint4 f[PRE][MT];
+    __device__ __forceinline__ uint4 at(int m, int k, int lane) const { return (base + (m * K + k) * 64)[lane]; }
+    __device__ __forceinline__ void load(const uint4 *img, int mt0, int lane) {
+        base = img + (int64_t)mt0 * K * 64;
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+        for (int k = 0; k < PRE; ++k)
 #pragma unroll
-        for (int c = 0; c < CK; ++c) cur[m][c] = base[(m * K + c) * 64];
-#pragma unroll 1
-    for (int k = 0; k < K; k += CK) {
-        const int kn = k + CK < K ? k + CK : k;  // (the last round reloads its own blocks)
+            for (int m = 0; m < MT; ++m) f[k][m] = at(m, k, lane);
+    }
+    __device__ __forceinline__ void mma(const unsigned char *b, int stride_bytes, int lane, nca::f32x4 (&acc)[MT][2]) {
+        const unsigned char *br = b + (lane & 15) * stride_bytes + 16 * (lane >> 4);
 #pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int c = 0; c < CK; ++c) nxt[m][c] = base[(m * K + kn + c) * 64];
-#pragma unroll
-        for (int c = 0; c < CK; ++c) {
+        for (int k = 0; k < K; ++k) {
+            __builtin_amdgcn_sched_barrier(0);
             fr bv[2];
 #pragma unroll
-            for (int n = 0; n < 2; ++n)
-                bv[n] = *reinterpret_cast<const fr *>(br + 16 * n * stride_bytes + 64 * (k + c));
+            for (int n = 0; n < 2; ++n) bv[n] = *reinterpret_cast<const fr *>(br + 16 * n * stride_bytes + 64 * k);
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
-                for (int n = 0; n < 2; ++n) acc[m][n] = BFrag<BF16>::mma(__builtin_bit_cast(fr, cur[m][c]), bv[n], acc[m][n]);
+                for (int n = 0; n < 2; ++n) acc[m][n] = BFrag<BF16>::mma(__builtin_bit_cast(fr, f[k % PRE][m]), bv[n], acc[m][n]);
+            if (k + PRE < K) {
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int m = 0; m < MT; ++m) f[k % PRE][m] = at(m, k + PRE, lane);
+            }
         }
-#pragma unroll
-        for (int m = 0; m < MT; ++m)
-#pragma unroll
-            for (int c = 0; c < CK; ++c) cur[m][c] = nxt[m][c];
     }
-}
+};
 
 // The gradient reaching cell (i, j) of board row `row`, channels [c0, c0 + 4), from the later step:
-// its g_u plus the transposed stencil of its g_z (M, F). The loads of
-// a row of neighbours are issued before its sums; a neighbour beyond a wall or zero border contributes nothing.
+// its g_u plus the transposed stencil of its g_z (M, F). The loads
+// (of 9 neighbours, or of a row of 3 in fp32) are issued before their sums; a neighbour beyond a wall or zero border contributes nothing.
 template <int C, bool BF16>
 __device__ __forceinline__ void later_grad(const Dims &d, const float *Gu, const void *Gz, const float *kern, int64_t mrow,
                                            int i, int j, int c0, float g[4]) {
     constexpr int F = 4 * C, ES = BF16 ? 2 : 4;
+    typedef std::conditional_t<BF16, uint2, float4> raw_t;
     const unsigned char *gz = static_cast<const unsigned char *>(Gz);
-    float4 g4 = *reinterpret_cast<const float4 *>(Gu + (mrow + i * d.W + j) * C + c0);
+    const float4 g4 = *reinterpret_cast<const float4 *>(Gu + (mrow + i * d.W + j) * C + c0);
+    constexpr int R = BF16 ? 9 : 3;  // neighbours at a time
     g[0] = g4.x, g[1] = g4.y, g[2] = g4.z, g[3] = g4.w;
-#pragma unroll 1
-    for (int t3 = 0; t3 < 3; ++t3) {
-        float v[3][4][4];
-        bool in[3];
 #pragma unroll
-        for (int t1 = 0; t1 < 3; ++t1) {
-            // the cell whose tap (t3, t1) reads this cell
-            const int q = neighbour(i, j, 1 - t3, 1 - t1, d.H, d.W, d.padding);
-            in[t1] = q >= 0;
-            const int64_t m = mrow + (q < 0 ? 0 : q);
+    for (int t0 = 0; t0 < 9; t0 += R) {
+        raw_t v[R][4];
+        unsigned in = 0;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) get4<BF16>(gz + (m * F + k * C + c0) * ES, v[t1][k]);
+        for (int t = 0; t < R; ++t) {
+            // the cell whose tap t0 + t reads this cell
+            const int q = neighbour(i, j, 1 - (t0 + t) / 3, 1 - (t0 + t) % 3, d.H, d.W, d.padding);
+            in |= (q >= 0 ? 1u : 0u) << t;
+            const unsigned char *p = gz + ((mrow + (q < 0 ? 0 : q)) * F + c0) * ES;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) v[t][k] = *reinterpret_cast<const raw_t *>(p + k * C * ES);
         }
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int t1 = 0; t1 < 3; ++t1)
+        for (int t = 0; t < R; ++t) {
+            const bool ok = (in >> t) & 1u;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const float w = kern[k * 9 + t3 * 3 + t1];
+                float f[4];
+                get4<BF16>(reinterpret_cast<const unsigned char *>(&v[t][k]), f);
+                const float w = kern[k * 9 + t0 + t];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) g[c] = in[t1] ? __builtin_fmaf(w, v[t1][k][c], g[c]) : g[c];
+                for (int c = 0; c < 4; ++c) g[c] = ok ? __builtin_fmaf(w, f[c], g[c]) : g[c];
             }
+        }
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
@@ -196,15 +210,20 @@ __device__ __forceinline__ void cell_taps(const Dims &d, const float *xt, const 
 #pragma unroll
         for (int c = 0; c < 4; ++c) hv[c] = padv[c0 + c];
     }
+    unsigned in = 0;
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
         const int nq = neighbour(i, j, t / 3 - 1, t % 3 - 1, d.H, d.W, d.padding);
+        in |= (nq >= 0 ? 1u : 0u) << t;
+        const float *xp = xr + (nq < 0 ? 0 : nq);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const float x = xr[(int64_t)c * d.HW + (nq < 0 ? 0 : nq)];
-            xv[c][t] = rnd<BF16>(nq >= 0 ? x : hv[c]);
-        }
+        for (int c = 0; c < 4; ++c) xv[c][t] = xp[c * d.HW];
     }
+    __builtin_amdgcn_sched_barrier(0);  // every load issued before the first use
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) xv[c][t] = rnd<BF16>((in >> t) & 1u ? xv[c][t] : hv[c]);
 }
 
 // A tile's LDS rows (cells) out to a kept buffer, transposed to (feats, 32 cells), 16 bytes a lane.
@@ -230,12 +249,21 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
     using S = BShape<C, HD, BF16>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     // the head: weights [v][c] and transposed [c][v], bias; per cell: logit gradients, output channels
-    __shared__ __attribute__((aligned(16))) float hwL[NO * NO], hwT[NO][NO], hbL[NO], glL[kBN][NO], xoL[kBN][NO];
-    __shared__ float fireL[kBN], lossL[kBN], red[4 * 36];
-    __shared__ int givenL[kBN], rowL[kBN], iL[kBN], jL[kBN];
+    __shared__ __attribute__((aligned(16))) float hwL[NO * NO], hwT[NO][NO], hbL[NO];
+    __shared__ float mxL[kBN], fireL[kBN], lossL[kBN], mkL[kBN], red[16 * 36];
+    __shared__ int givenL[kBN], rowL[kBN], iL[kBN], jL[kBN], tgtL[kBN];
+    // the head's per-cell values are done with before g_a and g_z are written: they share their LDS
+    // (so that two workgroups of the bf16 C = 64 cell fit a CU)
+    struct Head {
+        float gl[kBN][NO], xo[kBN][NO], lg[kBN][NO + 1], ex[kBN][NO + 1];
+    };
+    static_assert(sizeof(Head) <= S::GD - S::GA, "the head's values exceed g_a's and g_z's LDS");
+    Head &hd = *reinterpret_cast<Head *>(smem + S::GA);
+    auto &glL = hd.gl, &xoL = hd.xo;
+    auto &lgL = hd.lg, &exL = hd.ex;
     unsigned char *ZL = smem + S::Z, *HL = smem + S::H, *GAL = smem + S::GA, *GZL = smem + S::GZ, *GDL = smem + S::GD;
     const Dims &d = a.f.d;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
+    int tid = threadIdx.x;
     const bool has_loss = a.f.wscale != 0.0f;
     const int M = (int)d.M;
     if (has_loss) {
@@ -249,14 +277,17 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
     }
     if (S::KC * S::KB > C)  // the zero part of g_dx's k axis
         for (int i = tid; i < kBN * S::DS; i += 256) reinterpret_cast<uint16_t *>(GDL)[i] = 0;
-    float dk[36];
-#pragma unroll
-    for (int v = 0; v < 36; ++v) dk[v] = 0.0f;
+    for (int i = tid; i < 16 * 36; i += 256) red[i] = 0.0f;
     if (!a.accum && blockIdx.x == 0 && tid == 0) *a.status = 0;
     const int npw = d.n_out * d.c_out, np = npw + d.n_out;
     float hs[2] = {0.0f, 0.0f}, lossv = 0.0f;
+    const float denom = has_loss && a.f.mask ? *a.f.denom : 1.0f;
 
     for (int64_t tile = blockIdx.x; tile < a.tiles; tile += gridDim.x) {
+        // opaque per tile: the address arithmetic stays in the loop (hoisted out of it, it spills)
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, g = lane >> 4, l16 = lane & 15;
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: the fragments' addresses are scalar
         const int m0 = (int)(tile * kBN);
         if (tid < kBN) {
             const int m = m0 + tid < M ? m0 + tid : M - 1, row = m / d.HW, q = m - row * d.HW, i = q / d.W;
@@ -268,7 +299,9 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
         // ---- per cell (wave 3): given flag and fire value; the head's output channels
         if (has_loss) {
 #pragma unroll
-            for (int e = tid; e < kBN * NO; e += 256) {
+            for (int it = 0; it < (kBN * NO + 255) / 256; ++it) {
+                const int e = tid + 256 * it;
+                if (e >= kBN * NO) continue;
                 const int n = e & (kBN - 1), c = e / kBN;
                 const int q = iL[n] * d.W + jL[n];
                 xoL[n][c] = c < d.c_out ? a.f.x1[((int64_t)rowL[n] * C + d.out_off + c) * d.HW + q] : 0.0f;
@@ -294,6 +327,8 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
             }
             fireL[n] = f;
             givenL[n] = gv;
+            tgtL[n] = has_loss && m < M ? a.f.targets[m] : 0;
+            mkL[n] = has_loss && a.f.mask && m < M ? a.f.mask[m] : 0.0f;
         }
         // ---- z: item (cell n, channel quad), lanes over cells
 #pragma unroll
@@ -338,27 +373,48 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
             }
         }
         __syncthreads();
-        // ---- the loss head: logits per (cell, class), then the soft-max gradient per cell
+        WFrags<BF16, S::MT1, S::KF> w1;
+        WFrags<BF16, S::MT1, S::KC> w2t;
+        w1.load(a.w1, wave * S::MT1, lane);
+        w2t.load(a.w2t, wave * S::MT1, lane);
+        // ---- the loss head, thread (cell, class): the logit, its exponential, the soft-max gradient
         if (has_loss) {
-            for (int e = tid; e < kBN * NO; e += 256) {
+#pragma unroll
+            for (int it = 0; it < (kBN * NO + 255) / 256; ++it) {
+                const int e = tid + 256 * it;
+                if (e >= kBN * NO) continue;
                 const int n = e & (kBN - 1), v = e / kBN;
                 float acc = hbL[v];
 #pragma unroll
                 for (int c = 0; c < NO; ++c) acc = c < d.c_out ? __builtin_fmaf(hwL[v * NO + c], xoL[n][c], acc) : acc;
-                glL[n][v] = acc;
+                lgL[n][v] = acc;
             }
             __syncthreads();
-            if (tid < kBN) {
-                const int n = tid, m = m0 + n < M ? m0 + n : M - 1;
-                float l[NO], gl[NO];
 #pragma unroll
-                for (int v = 0; v < NO; ++v) l[v] = glL[n][v];
-                const float lc = softmax_grad<NO>(d, a.f.wscale, a.f.mask != nullptr, a.f.denom, l, a.f.targets[m],
-                                                  a.f.mask ? a.f.mask[m] : 0.0f, gl);
+            for (int it = 0; it < (kBN * NO + 255) / 256; ++it) {
+                const int e = tid + 256 * it;
+                if (e >= kBN * NO) continue;
+                const int n = e & (kBN - 1), v = e / kBN;
+                float mx = -INFINITY;
+#pragma unroll
+                for (int w = 0; w < NO; ++w) mx = w < d.n_out ? fmaxf(mx, lgL[n][w]) : mx;
+                exL[n][v] = v < d.n_out ? expf(lgL[n][v] - mx) : 0.0f;
+                if (v == 0) mxL[n] = mx;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int it = 0; it < (kBN * NO + 255) / 256; ++it) {
+                const int e = tid + 256 * it;
+                if (e >= kBN * NO) continue;
+                const int n = e & (kBN - 1), v = e / kBN, tgt = tgtL[n];
+                const float scale = a.f.mask ? a.f.wscale * mkL[n] / denom : a.f.wscale;
+                float s = 0.0f;
+#pragma unroll
+                for (int w = 0; w < NO; ++w) s += exL[n][w];
                 const bool ok = m0 + n < M;
-                lossL[n] = ok ? lc : 0.0f;
-#pragma unroll
-                for (int v = 0; v < NO; ++v) glL[n][v] = ok ? gl[v] : 0.0f;
+                glL[n][v] = ok && v < d.n_out ? (exL[n][v] / s - (v == tgt ? 1.0f : 0.0f)) * scale : 0.0f;
+                if (v == 0)
+                    lossL[n] = ok ? (mxL[n] + logf(s) - (tgt >= 0 && tgt < d.n_out ? lgL[n][tgt] : mxL[n])) * scale : 0.0f;
             }
             __syncthreads();
         }
@@ -406,14 +462,17 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
         }
         __syncthreads();
         // ---- h and g_a: wave w, hidden units [w HD / 4, (w + 1) HD / 4)
+        WFrags<BF16, S::MT2, S::KH> w1t;
         {
             nca::f32x4 h[S::MT1][2], ga[S::MT1][2];
 #pragma unroll
             for (int m = 0; m < S::MT1; ++m)
 #pragma unroll
                 for (int n = 0; n < 2; ++n) h[m][n] = ga[m][n] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            tile_mma<BF16, S::MT1, S::KF>(a.w1, wave * S::MT1, ZL, S::ZS * S::ES, lane, h);
-            tile_mma<BF16, S::MT1, S::KC>(a.w2t, wave * S::MT1, GDL, S::DS * S::ES, lane, ga);
+            w1.mma(ZL, S::ZS * S::ES, lane, h);
+            w2t.mma(GDL, S::DS * S::ES, lane, ga);
+            w1t.load(a.w1t, wave * S::MT2, lane);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int m = 0; m < S::MT1; ++m) {
                 const int hid = (wave * S::MT1 + m) * 16 + 4 * g;
@@ -429,12 +488,15 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
                         hr[v] = hv > 0.0f ? hv : 0.0f;
                         gv[v] = hr[v] > 0.0f ? rnd<BF16>(ga[m][n][v]) : 0.0f;
                     }
-                    put4<BF16>(HL + (cell * S::GS + hid) * S::ES, hr);
                     if (BF16) {
+                        put4<BF16>(HL + (cell * S::GS + hid) * S::ES, hr);
                         put4<BF16>(GAL + (cell * S::GS + hid) * S::ES, gv);
                     } else {
 #pragma unroll
-                        for (int v = 0; v < 4; ++v) reinterpret_cast<float *>(GAL)[cell * S::GS + S::col(hid + v)] = gv[v];
+                        for (int v = 0; v < 4; ++v) {
+                            reinterpret_cast<float *>(GAL)[cell * S::GS + S::col(hid + v)] = gv[v];
+                            static_cast<float *>(a.hs)[((a.tile0 + tile) * HD + hid + v) * kBN + cell] = hr[v];
+                        }
                     }
                 }
             }
@@ -447,7 +509,7 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
             for (int m = 0; m < S::MT2; ++m)
 #pragma unroll
                 for (int n = 0; n < 2; ++n) gz[m][n] = nca::f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            tile_mma<BF16, S::MT2, S::KH>(a.w1t, wave * S::MT2, GAL, S::GS * S::ES, lane, gz);
+            w1t.mma(GAL, S::GS * S::ES, lane, gz);
 #pragma unroll
             for (int m = 0; m < S::MT2; ++m)
 #pragma unroll
@@ -457,21 +519,35 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
                 }
         }
         __syncthreads();
-        // ---- the kernel-weight sums (the taps again, from the caches)
+        // ---- the kernel-weight sums (the taps again, from the caches), folded over rows of 16 lanes
+        {
+            float dk[36];
 #pragma unroll
-        for (int it = 0; it < S::NZ; ++it) {
-            const int e = tid + 256 * it, n = e & (kBN - 1), c0 = 4 * (e / kBN);
-            if (e >= S::ITEMS || m0 + n >= M) continue;
-            float xv[4][9];
-            cell_taps<C, BF16>(d, a.xt, a.padv, rowL[n], iL[n], jL[n], c0, xv);
+            for (int v = 0; v < 36; ++v) dk[v] = 0.0f;
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                float gv[4];
-                get4<BF16>(GZL + (n * S::ZS + k * C + c0) * S::ES, gv);
+            for (int it = 0; it < S::NZ; ++it) {
+                const int e = tid + 256 * it, n = e & (kBN - 1), c0 = 4 * (e / kBN);
+                if (e >= S::ITEMS || m0 + n >= M) continue;
+                float xv[4][9];
+                cell_taps<C, BF16>(d, a.xt, a.padv, rowL[n], iL[n], jL[n], c0, xv);
 #pragma unroll
-                for (int c = 0; c < 4; ++c)
+                for (int k = 0; k < 4; ++k) {
+                    float gv[4];
+                    get4<BF16>(GZL + (n * S::ZS + k * C + c0) * S::ES, gv);
 #pragma unroll
-                    for (int t = 0; t < 9; ++t) dk[k * 9 + t] = __builtin_fmaf(gv[c], xv[c][t], dk[k * 9 + t]);
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int t = 0; t < 9; ++t) dk[k * 9 + t] = __builtin_fmaf(gv[c], xv[c][t], dk[k * 9 + t]);
+                }
+            }
+#pragma unroll
+            for (int v = 0; v < 36; ++v) {
+                float x = dk[v];
+                x = __fadd_rn(x, dpp_f32<0xb1>(x));
+                x = __fadd_rn(x, dpp_f32<0x4e>(x));
+                x = __fadd_rn(x, dpp_f32<0x141>(x));
+                x = __fadd_rn(x, dpp_f32<0x140>(x));
+                if (l16 == 0) red[(tid >> 4) * 36 + v] = __fadd_rn(red[(tid >> 4) * 36 + v], x);
             }
         }
         // ---- everything out: stores last, so that no load of the tile waits behind them (they
@@ -491,15 +567,19 @@ __global__ void __launch_bounds__(256, 2) back_step(BackStepArgs a) {
                     *reinterpret_cast<const uint4 *>(GZL + n * S::ZS * S::ES + 16 * o);
         }
         flush_tile<S, BF16, true>(ZL, S::ZS, S::F, a.zs, a.tile0 + tile);
-        flush_tile<S, BF16, false>(HL, S::GS, HD, a.hs, a.tile0 + tile);
+        if (BF16) flush_tile<S, BF16, false>(HL, S::GS, HD, a.hs, a.tile0 + tile);
         flush_tile<S, BF16, true>(GAL, S::GS, HD, a.gas, a.tile0 + tile);
         flush_tile<S, BF16, true>(GDL, S::DS, C, a.gds, a.tile0 + tile);
         __syncthreads();
     }
     // ---- the workgroup's slots
     float *sl = a.slots + (int64_t)blockIdx.x * a.nslot;
-    const float r = block_sums<36, 4>(dk, red);
-    if (tid < 36) sl[tid] = a.accum ? __fadd_rn(sl[tid], r) : r;
+    if (tid < 36) {
+        float r = a.accum ? sl[tid] : 0.0f;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) r = __fadd_rn(r, red[w * 36 + tid]);  // the 16 lane rows in order
+        sl[tid] = r;
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const int p = tid + 256 * s;
