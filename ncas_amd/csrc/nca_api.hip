@@ -13,6 +13,7 @@
 #include "nca_device.h"
 #include "nca_layout.h"
 #include "nca_rollout.h"
+#include "nca_split_launch.h"
 #include "nca_stream.h"
 #include "nca_tiled_launch.h"
 #include "nca_status.h"
@@ -180,9 +181,30 @@ __device__ __forceinline__ void pack_units(const float *src, int M, int K, int s
     }
 }
 
+// The three bf16 parts of the C = 16 cell's W1 and W2 (see nca_layout.h), 16-byte units
+// [m-tile][k-tile][part][lane].
+__device__ __forceinline__ void pack_split16(const float *w1, const float *w2, unsigned char *dst, int b, int nb) {
+    constexpr int C = 16, HD = 128, F = 64, n1 = 8 * 2 * 64, n = n1 + 4 * 64;  // (m-tile, k-tile, lane)
+    for (int u = b * blockDim.x + threadIdx.x; u < n; u += nb * blockDim.x) {
+        const bool first = u < n1;
+        const int lane = u & 63, e = (first ? u : u - n1) >> 6, kt = first ? e % 2 : e, mt = first ? e / 2 : 0, g = lane >> 4;
+        const float *row = first ? w1 + (16 * mt + (lane & 15)) * F : w2 + (lane & 15) * HD;
+        __bf16 *d = reinterpret_cast<__bf16 *>(dst) + ((size_t)(u >> 6) * 3 * 64 + lane) * 8;
+        for (int s = 0; s < 8; ++s) {
+            const float v = row[(2 * kt + s / 4) * (first ? C : 16) + 4 * g + s % 4];
+            const __bf16 h = (__bf16)v;
+            const float r = v - (float)h;
+            const __bf16 m = (__bf16)r;
+            d[s] = h;
+            d[64 * 8 + s] = m;
+            d[2 * 64 * 8 + s] = (__bf16)(r - (float)m);
+        }
+    }
+}
+
 // The whole packing in one launch: workgroups [64 k, 64 k + 64) build layout k (the backward's W1,
-// W1^T and W2^T, then the forward's W1, W2, and for bf16 cells W2 for the hidden-major fc2, W1
-// quad-major, W2 k-major), the last one the small vectors (kernels, b1, b2, head, padding value).
+// W1^T and W2^T, then the forward's W1, W2, and their bf16 parts (fp32 cells) or W2 for the
+// hidden-major fc2, W1 quad-major, W2 k-major (bf16 cells)), the last one the small vectors (kernels, b1, b2, head, padding value).
 struct PackArgs {
     const float *kernels, *w1, *b1, *w2, *b2, *head_w, *head_b, *pad_vec;
     int nk, HD, C, F, nhw, nhb, bf;
@@ -195,7 +217,7 @@ constexpr int kPackBack = 3;  // layouts of the backward
 __global__ void pack_all(PackArgs a) {
     constexpr int kPB = 64;
     const int b = blockIdx.x, part = b / kPB - kPackBack, pb = b % kPB;
-    const int nfrag = a.bf ? 5 : 2;
+    const int nfrag = a.bf ? 5 : 3;
     unsigned char *pk = a.pk;
     if (part == -3) {
         pack_units(a.w1, a.HD, a.F, a.F, 1, a.bf, pk + a.L.bw1, pb, kPB);
@@ -214,6 +236,8 @@ __global__ void pack_all(PackArgs a) {
         pack_frags(a.w1, a.HD, a.F, a.bf, 0, (void *)(pk + a.L.w1), pb, kPB);
     } else if (part == 1) {
         pack_frags(a.w2, a.C, a.HD, a.bf, 0, (void *)(pk + a.L.w2), pb, kPB);
+    } else if (part == 2 && !a.bf) {
+        if (a.C == 16) pack_split16(a.w1, a.w2, pk + a.L.split, pb, kPB);
     } else if (part == 2) {
         pack_w2h(a.w2, a.C, a.HD, reinterpret_cast<__bf16 *>(pk + a.L.w2h), pb, kPB);
     } else if (part == 3) {
@@ -428,6 +452,16 @@ int launch_rollout(nca::RolloutParams p, hipStream_t st) {
     return hip_check(hipGetLastError(), "rollout launch");
 }
 
+// Does the call run on the fp32 kernels on the bf16 matrix cores (nca_split.h)? Every call of a shape
+// does or does not, whatever its steps, so that fused rollouts equal chained steps bit for bit.
+// Boards that fit neither their LDS plan nor the 31-bit offsets of their per-step kernel, and the few
+// that fit only the generic resident kernel's plan (which needs no workspace), stay there.
+bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
+    if (g_path != 0 || g_window_steps > 1 || d->precision != NCA_FP32 || d->channels != 16 || d->hidden != 128) return false;
+    if (nca::split16_resident_fits(H, W, d->c_out, d->n_out)) return true;
+    return !takes_resident(d, rows, H, W) && nca::split16_step_fits(rows, H, W);
+}
+
 size_t state_bytes(const nca_cell_desc *d, int64_t rows, int H, int W) {
     return (size_t)rows * d->channels * (size_t)H * W * sizeof(float);
 }
@@ -466,6 +500,7 @@ size_t per_step_need(const nca_cell_desc *d, int64_t rows, int H, int W, int n, 
 int run_tiled(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t st, void *ws, size_t ws_bytes) {
     const size_t sb = state_bytes(d, p.rows, p.H, p.W);
     const int n = p.n_steps;
+    const bool split = takes_split16(d, p.rows, p.H, p.W);
     const bool alias = p.x_in == p.x_out;
     if (!alias && overlaps(p.x_in, sb, p.x_out, sb))
         return fail(NCA_ERR_INVALID, "x_in and x_out overlap without being the same buffer");
@@ -509,7 +544,12 @@ int run_tiled(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t s
                 if (rc) return rc;
             } else {
                 bool ok = false;
-                int rc = hip_check(nca::tiled_step(d->channels, d->hidden, d->precision == NCA_BF16, q, s, s == 0,
+                int rc;
+                if (split) {
+                    rc = hip_check(nca::split16_step(q, s, s == 0, s == 0, last, st), "split step launch");
+                    ok = true;
+                } else
+                    rc = hip_check(nca::tiled_step(d->channels, d->hidden, d->precision == NCA_BF16, q, s, s == 0,
                                                    s == 0, last, st, g_path == 3, &ok),
                                    "tiled step launch");
                 if (rc) return rc;
@@ -557,6 +597,14 @@ int launch_cell(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t
         const int rc = hip_check(nca::launch_stream32(p, st, kLdsBytes, &used), "streamed rollout launch");
         if (rc || used) return rc;
     }
+    if (C == 16 && takes_split16(d, p.rows, p.H, p.W)) {
+        // one step on the per-step kernel, whose tiles spread over the whole device (out of place: in
+        // place it would need a workspace); more of them in LDS where the boards fit
+        const size_t sb = state_bytes(d, p.rows, p.H, p.W);
+        const bool one = p.n_steps == 1 && nca::split16_step_fits(p.rows, p.H, p.W) && !overlaps(p.x_in, sb, p.x_out, sb);
+        if (one || !nca::split16_resident_fits(p.H, p.W, d->c_out, d->n_out)) return run_tiled(d, p, st, ws, ws_bytes);
+        return hip_check(nca::split16_rollout(p, st), "split rollout launch");
+    }
     if (!takes_resident(d, p.rows, p.H, p.W)) return run_tiled(d, p, st, ws, ws_bytes);
     if (bf && C == 64 && HD == 256 && g_path == 0) {
         bool used = false;
@@ -603,6 +651,7 @@ nca::RolloutParams base_params(const nca_cell_desc *d, const void *packed, int64
     p.off_w2h = (unsigned)L.w2h;
     p.off_w1q = (unsigned)L.w1q;
     p.off_w2k = (unsigned)L.w2k;
+    p.off_split = (unsigned)L.split;
     return p;
 }
 
@@ -665,7 +714,8 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
         return NCA_OK;
     }
     if (!packed || !x_in || !given || (!clamp && cell->c_in > 0) || !x_out || !x_rec) return NCA_OK;
-    if (fire->adaptive || rows < 1 || n_steps < 1 || !takes_stream32(cell, rows, H, W)) return NCA_OK;
+    const bool split = takes_split16(cell, rows, H, W) && nca::split16_resident_fits(H, W, cell->c_out, cell->n_out);
+    if (fire->adaptive || rows < 1 || n_steps < 1 || (!split && !takes_stream32(cell, rows, H, W))) return NCA_OK;
     nca::RolloutParams p = base_params(cell, packed, rows, H, W);
     p.x_in = x_in;
     p.x_out = x_out;
@@ -683,6 +733,10 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
     p.x_rec = x_rec;
     p.rec_stride = rec_stride;
     p.x_rec0 = x_rec0;
+    if (split) {
+        *used = true;
+        return hip_check(nca::split16_rollout(p, st), "split rollout launch");
+    }
     int P = xch ? recorded_pieces(cell, rows, H, W) : 1;
     if (P > 1 && xch_bytes < nca::stream32_xch_bytes(rows, P, W)) P = 1;
     const int rc = hip_check(nca::launch_stream32(p, st, kLdsBytes, used, P, static_cast<uint64_t *>(xch)),
@@ -773,6 +827,7 @@ int nca_set_window_steps(int steps) {
 size_t nca_rollout_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t height, int32_t width) {
     if (check_cell(cell) || check_grid(rows, height, width)) return 0;
     if (takes_resident(cell, rows, height, width) || takes_stream32(cell, rows, height, width)) return 0;
+    if (takes_split16(cell, rows, height, width) && nca::split16_resident_fits(height, width, cell->c_out, cell->n_out)) return 0;
     return 2 * state_bytes(cell, rows, height, width);
 }
 
@@ -813,7 +868,7 @@ int nca_pack_weights(const nca_cell_desc *cell, const nca_cell_weights *w, void 
     pa.bf = bf ? 1 : 0;
     pa.pk = pk;
     pa.L = L;
-    hipLaunchKernelGGL(pack_all, dim3((kPackBack + (bf ? 5 : 2)) * 64 + 1), dim3(256), 0, st, pa);
+    hipLaunchKernelGGL(pack_all, dim3((kPackBack + (bf ? 5 : 3)) * 64 + 1), dim3(256), 0, st, pa);
     return hip_check(hipGetLastError(), "pack launch");
 }
 

@@ -25,6 +25,10 @@
 //          k axis zero-padded to a block): [m-tile][k-block][lane] units of 16 bytes, a block 32 k
 //          (bf16) or 16 k (fp32), unit element s = A[i = lane % 16][block + 8 (lane / 16) + s] (bf16)
 //          or A[i][block + 4 s + lane / 16] (fp32)
+//   split  (fp32, C = 16 only) W1 and W2 in three bf16 parts (nca_split.h): [m-tile][k-tile][part][lane]
+//          units of 16 bytes (8 k slots), W1's then W2's. Slot s of lane group g of k-tile k is feature
+//          (2 k + s / 4) C + 4 g + s % 4 of W1 and hidden unit 16 (2 k + s / 4) + 4 g + s % 4 of W2
+//          (fc1's accumulators as they lie)
 // bf16 cells use v_mfma_f32_16x16x32_bf16 fragments (k-tile 32, 8 bf16 slots per lane:
 // A[i = lane % 16][k = 8 * (lane / 16) + slot]); fp32 cells use v_mfma_f32_16x16x4_f32
 // fragments (k-tile 4, one float per lane: A[i = lane % 16][k = lane / 16]).
@@ -35,7 +39,7 @@
 namespace nca {
 
 struct PackedLayout {
-    size_t kern, b1, b2, headw, headb, padv, w1, w2, w2h, w1q, w2k, bw1, bw1t, bw2t, total;
+    size_t kern, b1, b2, headw, headb, padv, w1, w2, w2h, w1q, w2k, bw1, bw1t, bw2t, split, total;
 };
 
 __host__ __device__ inline size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -74,6 +78,8 @@ __host__ __device__ inline PackedLayout packed_layout(int C, int heads, int hidd
     const size_t kblock = bf16 ? 32 : 16;
     L.bw2t = o;
     o = align256(o + esz * (size_t)hidden * ((C + kblock - 1) / kblock * kblock));
+    L.split = o;
+    o = align256(o + (!bf16 && C == 16 ? 6 * (size_t)hidden * (heads + 1) * C : 0));
     L.total = o;
     return L;
 }

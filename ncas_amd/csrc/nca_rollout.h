@@ -56,8 +56,8 @@ struct RolloutParams {
     float *conf_out;
     int32_t *fired_out;
     float *x_rec;        // or null: the state after step s of the call goes to x_rec + s rec_stride
-    int64_t rec_stride;  // (the streamed C = 32 kernel only)
-    float *x_rec0;       // or null: the call's input state copied there (the same kernel, with x_rec)
+    int64_t rec_stride;  // (the streamed C = 32 kernel and the fp32 C = 16 kernel only)
+    float *x_rec0;       // or null: the call's input state copied there (the same kernels, with x_rec)
     int64_t rows;
     int H, W;
     int c_in, in_off, c_out, out_off, n_out, head_kind, padding;
@@ -67,7 +67,7 @@ struct RolloutParams {
     float p, p_low, tau;
     int adaptive, given_confident;
     int rows_per_wg;
-    unsigned off_kern, off_b1, off_b2, off_headw, off_headb, off_padv, off_w1, off_w2, off_w2h, off_w1q, off_w2k;
+    unsigned off_kern, off_b1, off_b2, off_headw, off_headb, off_padv, off_w1, off_w2, off_w2h, off_w1q, off_w2k, off_split;
     unsigned l_P, l_M, l_Z, l_H, l_clamp, l_given, l_fire, l_conf, l_fired, l_head, l_cinfo;
 };
 
