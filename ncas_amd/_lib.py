@@ -220,6 +220,20 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+def as_f32(t: torch.Tensor) -> torch.Tensor:
+    """`t` as the kernels read it: detached, fp32, contiguous; itself where it is all of that."""
+    if t.requires_grad:
+        t = t.detach()
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.to(torch.float32).contiguous()
+
+
+def as_u8(t: torch.Tensor) -> torch.Tensor:
+    """A mask as contiguous bytes: a view of a contiguous bool mask's (no conversion launch)."""
+    if t.dtype == torch.bool and t.is_contiguous():
+        return t.view(torch.uint8)
+    return t.detach().to(torch.uint8).contiguous()
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 

@@ -65,8 +65,7 @@ def rollout_steps(
     xs = x.detach()
     if xs.dtype != torch.float32 or not xs.is_contiguous():
         xs = xs.to(torch.float32).contiguous()
-    g8 = given4.detach().to(torch.uint8).contiguous()
-    cl = clamp.detach().to(torch.float32).contiguous()
+    g8, cl = _lib.as_u8(given4), _lib.as_f32(clamp)
     m8 = None
     if masks is not None:
         if masks.shape[0] != n_steps or masks[0].numel() != B * H * W:

@@ -92,16 +92,14 @@ def _check_shapes(model, x, given4, clamp, fire, noise):
         raise ValueError("noise must have the state's shape")
 
 
-def _forward(model, prec, dev, x, given4, clamp, fire, noise):
-    """x_out = step(x) through `nca_step`; returns (x_out, the fp32 / u8 operands it read)."""
+def _forward(model, prec, dev, x, g8, clamp, fire, noise):
+    """x_out = step(x) through `nca_step` (g8: the given mask as contiguous bytes); returns (x_out,
+    the fp32 / u8 operands it read)."""
     B, _, H, W = x.shape
     pk = model.packed(prec, dev)
-    xs = x.detach().to(torch.float32).contiguous()
-    g8 = given4.detach().to(torch.uint8).contiguous()
-    cl = clamp.detach().to(torch.float32).contiguous()
-    fi = fire.detach().to(torch.float32).contiguous()
-    nz = None if noise is None else noise.detach().to(torch.float32).contiguous()
-    out = torch.empty_like(xs)
+    xs, cl, fi = _lib.as_f32(x), _lib.as_f32(clamp), _lib.as_f32(fire)
+    nz = None if noise is None else _lib.as_f32(noise)
+    out = torch.empty(x.shape, dtype=torch.float32, device=dev)
     _lib.check(
         _lib.load().nca_step(ctypes.byref(pk.desc), pk.buf.data_ptr(), B, H, W, xs.data_ptr(),
                              g8.data_ptr(), cl.data_ptr(), fi.data_ptr(), _lib.ptr(nz),
@@ -152,7 +150,9 @@ class _HipStep(torch.autograd.Function):
     @staticmethod
     def forward(ctx, model, prec, x, given4, clamp, fire, noise, *params):
         dev = x.device
-        out, xs, g8, fi = _forward(model, prec, dev, x, given4, clamp, fire, noise)
+        # a copy of the mask: the backward reads it later
+        g8 = given4.detach().to(torch.uint8).contiguous()
+        out, xs, g8, fi = _forward(model, prec, dev, x.detach(), g8, clamp, fire, noise)
         ctx.model, ctx.prec = model, prec
         ctx.dtypes = (x.dtype, clamp.dtype, None if noise is None else noise.dtype)
         ctx.save_for_backward(xs, g8, fi)
@@ -185,7 +185,7 @@ def hip_step(model, x, given4, clamp, fire, noise=None, precision=None):
     prec = _autocast_precision(dev, precision)
     _check_shapes(model, x, given4, clamp, fire, noise)
     if not _needs_grad(model, x, clamp, noise):
-        return _forward(model, prec, dev, x, given4, clamp, fire, noise)[0]
+        return _forward(model, prec, dev, x, _lib.as_u8(given4), clamp, fire, noise)[0]
     if fire.requires_grad:
         raise ValueError("the HIP step does not differentiate w.r.t. the fire mask")
     return _HipStep.apply(model, prec, x, given4, clamp, fire, noise, *_params(model))
