@@ -31,6 +31,7 @@ SOURCES = {
     "nca_stream32.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "nca_tiled.hip": [],
     "nca_split16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "nca_split_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     # mlp_back32 keeps its weight fragments in AGPRs and its accumulators in VGPRs
     "nca_bptt.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
     "nca_prune.hip": [],

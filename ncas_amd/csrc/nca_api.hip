@@ -202,6 +202,34 @@ __device__ __forceinline__ void pack_split16(const float *w1, const float *w2, u
     }
 }
 
+// The same of the 256-hidden cells' W1 and W2: [wave][k-step][part][lane], then
+// [wave][m-tile][k-step][part][lane].
+__device__ __forceinline__ void pack_split_wide(const float *w1, const float *w2, int C, unsigned char *dst, int b, int nb) {
+    constexpr int HD = 256;
+    const int ks = C / 4, mt = C / 32, n1 = 8 * ks * 64, n = n1 + 8 * mt * 2 * 64;
+    for (int u = b * blockDim.x + threadIdx.x; u < n; u += nb * blockDim.x) {
+        const bool first = u < n1;
+        const int lane = u & 63, e = (first ? u : u - n1) >> 6, hf = lane >> 5;
+        __bf16 *d = reinterpret_cast<__bf16 *>(dst) + ((size_t)(u >> 6) * 3 * 64 + lane) * 8;
+        for (int s = 0; s < 8; ++s) {
+            float v;
+            if (first) {
+                const int w = e / ks, j = e % ks, kk = 8 * hf + s;
+                v = w1[(size_t)(32 * w + (lane & 31)) * 4 * C + (kk / 4) * C + 4 * j + kk % 4];
+            } else {
+                const int w = e / (2 * mt), m = e / 2 % mt, j = e & 1;
+                v = w2[(size_t)(32 * m + (lane & 31)) * HD + 32 * w + 8 * (2 * j + s / 4) + 4 * hf + s % 4];
+            }
+            const __bf16 h = (__bf16)v;
+            const float r = v - (float)h;
+            const __bf16 m3 = (__bf16)r;
+            d[s] = h;
+            d[64 * 8 + s] = m3;
+            d[2 * 64 * 8 + s] = (__bf16)(r - (float)m3);
+        }
+    }
+}
+
 // The whole packing in one launch: workgroups [64 k, 64 k + 64) build layout k (the backward's W1,
 // W1^T and W2^T, then the forward's W1, W2, and their bf16 parts (fp32 cells) or W2 for the
 // hidden-major fc2, W1 quad-major, W2 k-major (bf16 cells)), the last one the small vectors (kernels, b1, b2, head, padding value).
@@ -237,7 +265,10 @@ __global__ void pack_all(PackArgs a) {
     } else if (part == 1) {
         pack_frags(a.w2, a.C, a.HD, a.bf, 0, (void *)(pk + a.L.w2), pb, kPB);
     } else if (part == 2 && !a.bf) {
-        if (a.C == 16) pack_split16(a.w1, a.w2, pk + a.L.split, pb, kPB);
+        if (a.C == 16)
+            pack_split16(a.w1, a.w2, pk + a.L.split, pb, kPB);
+        else
+            pack_split_wide(a.w1, a.w2, a.C, pk + a.L.split, pb, kPB);
     } else if (part == 2) {
         pack_w2h(a.w2, a.C, a.HD, reinterpret_cast<__bf16 *>(pk + a.L.w2h), pb, kPB);
     } else if (part == 3) {
@@ -462,6 +493,26 @@ bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
     return !takes_resident(d, rows, H, W) && nca::split16_step_fits(rows, H, W);
 }
 
+// The same for the C = 32 and C = 64 cells. The per-step kernel takes the C = 32 boards that the generic
+// kernels run step by step too (with a workspace); other boards that do not fit the LDS plan
+// stay there.
+bool takes_split_wide(const nca_cell_desc *d, int64_t rows, int H, int W) {
+    if (g_path != 0 || d->precision != NCA_FP32 || d->hidden != 256 || (d->channels != 32 && d->channels != 64)) return false;
+    if (nca::split_wide_resident_fits(d->channels, H, W, d->c_out, d->n_out)) return true;
+    return !takes_resident(d, rows, H, W) && nca::split_wide_step_fits(d->channels, rows, H, W);
+}
+
+// Does a rollout or recorded chunk run on one of these kernels in LDS, in one launch?
+bool split_resident(const nca_cell_desc *d, int64_t rows, int H, int W) {
+    if (d->channels == 16)
+        return takes_split16(d, rows, H, W) && nca::split16_resident_fits(H, W, d->c_out, d->n_out);
+    return takes_split_wide(d, rows, H, W) && nca::split_wide_resident_fits(d->channels, H, W, d->c_out, d->n_out);
+}
+
+hipError_t split_rollout(int C, const nca::RolloutParams &p, hipStream_t st) {
+    return C == 16 ? nca::split16_rollout(p, st) : nca::split_wide_rollout(C, p, st);
+}
+
 size_t state_bytes(const nca_cell_desc *d, int64_t rows, int H, int W) {
     return (size_t)rows * d->channels * (size_t)H * W * sizeof(float);
 }
@@ -500,7 +551,7 @@ size_t per_step_need(const nca_cell_desc *d, int64_t rows, int H, int W, int n, 
 int run_tiled(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t st, void *ws, size_t ws_bytes) {
     const size_t sb = state_bytes(d, p.rows, p.H, p.W);
     const int n = p.n_steps;
-    const bool split = takes_split16(d, p.rows, p.H, p.W);
+    const bool split = takes_split16(d, p.rows, p.H, p.W), wide = takes_split_wide(d, p.rows, p.H, p.W);
     const bool alias = p.x_in == p.x_out;
     if (!alias && overlaps(p.x_in, sb, p.x_out, sb))
         return fail(NCA_ERR_INVALID, "x_in and x_out overlap without being the same buffer");
@@ -547,6 +598,9 @@ int run_tiled(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t s
                 int rc;
                 if (split) {
                     rc = hip_check(nca::split16_step(q, s, s == 0, s == 0, last, st), "split step launch");
+                    ok = true;
+                } else if (wide) {
+                    rc = hip_check(nca::split_wide_step(q, s, s == 0, s == 0, last, st), "split step launch");
                     ok = true;
                 } else
                     rc = hip_check(nca::tiled_step(d->channels, d->hidden, d->precision == NCA_BF16, q, s, s == 0,
@@ -597,13 +651,14 @@ int launch_cell(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t
         const int rc = hip_check(nca::launch_stream32(p, st, kLdsBytes, &used), "streamed rollout launch");
         if (rc || used) return rc;
     }
-    if (C == 16 && takes_split16(d, p.rows, p.H, p.W)) {
+    if (takes_split16(d, p.rows, p.H, p.W) || takes_split_wide(d, p.rows, p.H, p.W)) {
         // one step on the per-step kernel, whose tiles spread over the whole device (out of place: in
         // place it would need a workspace); more of them in LDS where the boards fit
         const size_t sb = state_bytes(d, p.rows, p.H, p.W);
-        const bool one = p.n_steps == 1 && nca::split16_step_fits(p.rows, p.H, p.W) && !overlaps(p.x_in, sb, p.x_out, sb);
-        if (one || !nca::split16_resident_fits(p.H, p.W, d->c_out, d->n_out)) return run_tiled(d, p, st, ws, ws_bytes);
-        return hip_check(nca::split16_rollout(p, st), "split rollout launch");
+        const bool fits = C == 16 ? nca::split16_step_fits(p.rows, p.H, p.W) : nca::split_wide_step_fits(C, p.rows, p.H, p.W);
+        const bool one = p.n_steps == 1 && fits && !overlaps(p.x_in, sb, p.x_out, sb);
+        if (one || !split_resident(d, p.rows, p.H, p.W)) return run_tiled(d, p, st, ws, ws_bytes);
+        return hip_check(split_rollout(C, p, st), "split rollout launch");
     }
     if (!takes_resident(d, p.rows, p.H, p.W)) return run_tiled(d, p, st, ws, ws_bytes);
     if (bf && C == 64 && HD == 256 && g_path == 0) {
@@ -714,7 +769,7 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
         return NCA_OK;
     }
     if (!packed || !x_in || !given || (!clamp && cell->c_in > 0) || !x_out || !x_rec) return NCA_OK;
-    const bool split = takes_split16(cell, rows, H, W) && nca::split16_resident_fits(H, W, cell->c_out, cell->n_out);
+    const bool split = split_resident(cell, rows, H, W);
     if (fire->adaptive || rows < 1 || n_steps < 1 || (!split && !takes_stream32(cell, rows, H, W))) return NCA_OK;
     nca::RolloutParams p = base_params(cell, packed, rows, H, W);
     p.x_in = x_in;
@@ -735,7 +790,7 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
     p.x_rec0 = x_rec0;
     if (split) {
         *used = true;
-        return hip_check(nca::split16_rollout(p, st), "split rollout launch");
+        return hip_check(split_rollout(cell->channels, p, st), "split rollout launch");
     }
     int P = xch ? recorded_pieces(cell, rows, H, W) : 1;
     if (P > 1 && xch_bytes < nca::stream32_xch_bytes(rows, P, W)) P = 1;
@@ -827,7 +882,7 @@ int nca_set_window_steps(int steps) {
 size_t nca_rollout_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t height, int32_t width) {
     if (check_cell(cell) || check_grid(rows, height, width)) return 0;
     if (takes_resident(cell, rows, height, width) || takes_stream32(cell, rows, height, width)) return 0;
-    if (takes_split16(cell, rows, height, width) && nca::split16_resident_fits(height, width, cell->c_out, cell->n_out)) return 0;
+    if (split_resident(cell, rows, height, width)) return 0;
     return 2 * state_bytes(cell, rows, height, width);
 }
 

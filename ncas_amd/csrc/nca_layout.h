@@ -25,10 +25,13 @@
 //          k axis zero-padded to a block): [m-tile][k-block][lane] units of 16 bytes, a block 32 k
 //          (bf16) or 16 k (fp32), unit element s = A[i = lane % 16][block + 8 (lane / 16) + s] (bf16)
 //          or A[i][block + 4 s + lane / 16] (fp32)
-//   split  (fp32, C = 16 only) W1 and W2 in three bf16 parts (nca_split.h): [m-tile][k-tile][part][lane]
-//          units of 16 bytes (8 k slots), W1's then W2's. Slot s of lane group g of k-tile k is feature
+//   split  (fp32 only) W1 and W2 in three bf16 parts (nca_split.h), 16-byte units (8 k slots), W1's then
+//          W2's. C = 16: [m-tile][k-tile][part][lane]. Slot s of lane group g of k-tile k is feature
 //          (2 k + s / 4) C + 4 g + s % 4 of W1 and hidden unit 16 (2 k + s / 4) + 4 g + s % 4 of W2
-//          (fc1's accumulators as they lie)
+//          (fc1's accumulators as they lie). C = 32, 64 (256 hidden units, 32x32x16 fragments): W1
+//          [32 hidden units][k-step][part][lane], k slot 8 (lane / 32) + s of k-step j feature
+//          ((8 (lane / 32) + s) / 4) C + 4 j + s % 4; W2 [32 hidden units w][m-tile][k-step][part][lane],
+//          hidden unit 32 w + 8 (2 j + s / 4) + 4 (lane / 32) + s % 4
 // bf16 cells use v_mfma_f32_16x16x32_bf16 fragments (k-tile 32, 8 bf16 slots per lane:
 // A[i = lane % 16][k = 8 * (lane / 16) + slot]); fp32 cells use v_mfma_f32_16x16x4_f32
 // fragments (k-tile 4, one float per lane: A[i = lane % 16][k = lane / 16]).
@@ -79,7 +82,7 @@ __host__ __device__ inline PackedLayout packed_layout(int C, int heads, int hidd
     L.bw2t = o;
     o = align256(o + esz * (size_t)hidden * ((C + kblock - 1) / kblock * kblock));
     L.split = o;
-    o = align256(o + (!bf16 && C == 16 ? 6 * (size_t)hidden * (heads + 1) * C : 0));
+    o = align256(o + (!bf16 ? 6 * (size_t)hidden * (heads + 1) * C : 0));
     L.total = o;
     return L;
 }

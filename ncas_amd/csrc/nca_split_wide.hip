@@ -1,0 +1,110 @@
+// Plans and launches of the fp32 C = 32 and C = 64 kernels (nca_split_wide.h).
+#include <hip/hip_runtime.h>
+
+#include <string.h>
+
+#include "nca_split_launch.h"
+#include "nca_split_wide.h"
+
+namespace nca {
+
+namespace {
+
+constexpr unsigned kWideLds = 160u * 1024u;
+constexpr unsigned kSmallBytes = 4u * (256 + kSWN + 4 + 36);  // fc1's bias, fire factors, NaN flags, kernels
+
+// LDS plan of R rows' rollout; false when it does not fit
+bool wide_plan(int C, int R, int H, int W, int c_out, int n_out, SplitWide *sp) {
+    const unsigned hw = (unsigned)H * W, hwp = (unsigned)(H + 2) * (W + 2);
+    if ((uint64_t)R * hwp > 4096) return false;  // beyond any plan (and ci's 16 bits)
+    sp->R = R;
+    sp->l_Z = sp->l_red = 0;  // RED takes Z's place after fc1
+    unsigned o = 2 * kSWZ;
+    sp->l_small = o;
+    o = st_al16(o + kSmallBytes);
+    sp->l_P = o;
+    o = st_al16(o + 2u * R * hwp * 4u * (C + 4));
+    sp->l_ci = o;
+    o = st_al16(o + 2u * R * hw);
+    sp->l_fire = o;
+    o = st_al16(o + 2u * R * hw);
+    sp->l_given = o;
+    o = st_al16(o + R * hw);
+    sp->l_fired = o;
+    o = st_al16(o + 4u * R);
+    sp->l_head = o;
+    o = st_al16(o + 4u * (n_out * c_out + n_out));
+    sp->total = o;
+    return o <= kWideLds;
+}
+static_assert(2 * kSWZ >= kSWRed, "RED in Z's place");
+
+int cu_count() {
+    int dev = 0, n = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 256;
+    return n;
+}
+
+template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW>
+hipError_t launch(const SplitWide &sp, unsigned grid, hipStream_t st) {
+    auto k = split_wide<C, GLOBAL, IN_NCHW, OUT_NCHW>;
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sp.total);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(kSWT), sp.total, st, sp);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool split_wide_resident_fits(int C, int H, int W, int c_out, int n_out) {
+    SplitWide sp;
+    return wide_plan(C, 1, H, W, c_out, n_out, &sp);
+}
+
+bool split_wide_step_fits(int C, int64_t rows, int H, int W) {
+    // 31-bit byte offsets into the state
+    return C == 32 && rows * (int64_t)H * W * C * (int64_t)sizeof(float) < ((int64_t)1 << 31);
+}
+
+hipError_t split_wide_rollout(int C, const RolloutParams &p, hipStream_t st) {
+    SplitWide sp;
+    memset(&sp, 0, sizeof(sp));
+    // the rows per workgroup with the fewest passes of 96 cells one after another on a CU
+    static const int n_cu = cu_count();
+    int best = 0;
+    int64_t cost = 0;
+    for (int R = 1; R <= 16 && wide_plan(C, R, p.H, p.W, p.c_out, p.n_out, &sp); ++R) {
+        const int64_t wgs = (p.rows + R - 1) / R;
+        const int64_t c = ((wgs + n_cu - 1) / n_cu) * (((int64_t)R * p.H * p.W + kSWN - 1) / kSWN);
+        if (!best || c < cost) best = R, cost = c;
+    }
+    if (!best || !wide_plan(C, best, p.H, p.W, p.c_out, p.n_out, &sp)) return hipErrorInvalidValue;
+    sp.a = p;
+    sp.wsplit = p.packed + p.off_split;
+    const unsigned grid = (unsigned)((p.rows + best - 1) / best);
+    return C == 32 ? launch<32, false, true, true>(sp, grid, st) : launch<64, false, true, true>(sp, grid, st);
+}
+
+hipError_t split_wide_step(const RolloutParams &p, int step, int first, int in_nchw, int out_nchw, hipStream_t st) {
+    SplitWide sp;
+    memset(&sp, 0, sizeof(sp));
+    sp.a = p;
+    sp.wsplit = p.packed + p.off_split;
+    sp.step = step;
+    sp.first = first;
+    sp.n_cells = (int)(p.rows * p.H * p.W);
+    if (sp.n_cells < 1) return hipSuccess;
+    sp.n_tiles = (sp.n_cells + kSWN - 1) / kSWN;
+    static const int n_cu = cu_count();
+    sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
+    sp.l_Z = 0;
+    sp.l_red = 2 * kSWZ;
+    sp.l_small = sp.l_red + kSWRed;
+    sp.total = st_al16(sp.l_small + kSmallBytes);
+    const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
+    if (in_nchw) return out_nchw ? launch<32, true, true, true>(sp, grid, st) : launch<32, true, true, false>(sp, grid, st);
+    return out_nchw ? launch<32, true, false, true>(sp, grid, st) : launch<32, true, false, false>(sp, grid, st);
+}
+
+}  // namespace nca
