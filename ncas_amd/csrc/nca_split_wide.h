@@ -56,8 +56,10 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     float4 *RED = reinterpret_cast<float4 *>(smem + sp.l_red);
     float *b1L = reinterpret_cast<float *>(smem + sp.l_small);
     float *fireG = b1L + HD;                                // GLOBAL: fire factors of the pass's cells
-    int *bad = reinterpret_cast<int *>(fireG + kSWN);       // NaN among a 32-cell tile's sums
-    f32x4 *kernL = reinterpret_cast<f32x4 *>(bad + 4);      // the 4 kernels' weights of each tap
+    // NaN among a 32-cell tile's sums, for even and odd passes: a pass clears the other's after its first
+    // barrier, when every wave is past the last look at them
+    int *badL = reinterpret_cast<int *>(fireG + kSWN), *bad = badL;
+    f32x4 *kernL = reinterpret_cast<f32x4 *>(badL + 8);      // the 4 kernels' weights of each tap
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int H = a.H, W = a.W, HWn = H * W;
@@ -65,6 +67,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     const bool wrap = a.padding == 2;
     const int c_in = a.c_in, in_off = a.in_off;
     for (int e = tid; e < HD; e += kSWT) b1L[e] = reinterpret_cast<const float *>(a.packed + a.off_b1)[e];
+    if (tid < 8) badL[tid] = 0;
     if (tid < 36) reinterpret_cast<float *>(kernL)[tid] = reinterpret_cast<const float *>(a.packed + a.off_kern)[(tid & 3) * 9 + (tid >> 2)];
     __syncthreads();
 
@@ -135,7 +138,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
 
     // the stencil item of a thread: cell sc, quad sq of an interval's 4. Quads fastest for global loads
     // (64 bytes of a cell), cells fastest for LDS taps (an odd stride of 16-byte slots). Waves 6 and 7
-    // repeat waves 0 and 1's, so that no branch keeps the stencil from the MFMAs.
+    // repeat waves 0 and 1's: a branch here doubles the intervals' code and spills the accumulators.
     const int sid = tid < 4 * kSWN ? tid : tid - 4 * kSWN;
     const int sc = GLOBAL ? sid >> 2 : 16 * (sid >> 6) + (sid & 15), sq = GLOBAL ? sid & 3 : (sid >> 4) & 3;
     auto put_half = [&](const float z[4][4], int h, int buf) __attribute__((always_inline)) {
@@ -178,7 +181,52 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     Split8 af[2] = {frag(wA, 0), frag(wA, 1)};
 
     // ---- one pass: cells [g0, g0 + 96) of step s (its index in the call)
-    const float4 *b2 = reinterpret_cast<const float4 *>(a.packed + a.off_b2);
+    const float4 b2v = reinterpret_cast<const float4 *>(a.packed + a.off_b2)[tid / (32 * NTR)];
+    // GLOBAL: waves 6 and 7 draw the fire factors of the pass's cells. What they read is touched an
+    // interval earlier.
+    auto warm_fire = [&](int g0) __attribute__((always_inline)) {
+        const int k = tid & 127, gc = k < kSWN && g0 + k < ncell ? g0 + k : g0;
+        float v = (float)a.given[gc];
+        if (a.adaptive && !IN_NCHW) v += a.x_in[(int64_t)gc * C + a.out_off];
+        return v;
+    };
+    auto draw_pass = [&](int g0) __attribute__((always_inline)) {
+        const int k = tid - 384, gq = g0 + k;
+        const bool live = k < kSWN && gq < ncell;
+        const int gc = live ? gq : g0, row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
+        float f;
+        if (a.fire_f32) {
+            f = a.fire_f32[gc];
+        } else if (a.fire_u8) {
+            f = a.fire_u8[(int64_t)sp.step * ncell + gc] ? 1.0f : 0.0f;
+        } else {
+            const uint64_t key = a.step_seeds ? a.step_seeds[sp.step] : a.seed;
+            float u4[4];
+            cell_uniforms4(key, (uint32_t)(a.row0 + row), (uint32_t)(a.step0 + sp.step), (uint32_t)(q >> 2), u4);
+            const float u = (q & 3) == 0 ? u4[0] : (q & 3) == 1 ? u4[1] : (q & 3) == 2 ? u4[2] : u4[3];
+            float p = a.p;
+            if (a.adaptive) {
+                const float *hw = reinterpret_cast<const float *>(a.packed + a.off_headw);
+                const float *hb = reinterpret_cast<const float *>(a.packed + a.off_headb);
+                int am;
+                const float *xc = IN_NCHW ? a.x_in + ((int64_t)row * C + a.out_off) * HWn + q : a.x_in + (int64_t)gc * C + a.out_off;
+                const float cf = cell_readout(xc, IN_NCHW ? HWn : 1, a.c_out, a.n_out, a.head_kind, hw, hb, &am);
+                if (cf > a.tau || (a.given_confident && a.given[gc])) p = a.p_low;
+            }
+            f = u < p ? 1.0f : 0.0f;
+        }
+        if (k < kSWN) fireG[k] = f;
+        if (a.fired_out) {
+            // one addition per row of the wave's cells
+            uint64_t rest = __ballot(live && f != 0.0f);
+            while (rest) {
+                const int r0 = __builtin_amdgcn_readlane(row, (int)__builtin_ctzll(rest));
+                const uint64_t mine = __ballot(live && f != 0.0f && row == r0);
+                if (lane == 0) atomicAdd(a.fired_out + r0, (int)__popcll(mine));
+                rest &= ~mine;
+            }
+        }
+    };
     auto pass = [&](int g0, int g0_next, int s, bool first, Pos &pos) __attribute__((always_inline)) {
         f32x16 big[kSWNT], small[kSWNT];
         auto bias = [&]() __attribute__((always_inline)) {
@@ -196,16 +244,18 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             big[t] = b1v;
             small[t] = f32x16{};
         }
-        if (tid < kSWNT) bad[tid] = 0;
         // An interval is 12 steps: per 16 features the l, m and h parts of Z, each with the weight parts
-        // it meets. A step's fragments are read two steps ahead; steps 0 to 8 also take one tap each
-        // into the next interval's z, whose tap was loaded three steps ahead; steps 9 and 10 split and
-        // store it. The barriers for the scheduler keep the loads where they are.
+        // it meets. A step's fragments are read two steps ahead; the steps between
+        // also add the taps into the next interval's z, which the last two split and store. Taps from
+        // global memory are loaded in the first three steps and added from the third on (later, at about 2,000
+        // cycles, they hold registers for longer: 30x30 steps 5 % slower), taps from LDS two steps ahead.
+        // The barriers for the scheduler keep the loads where they are.
         auto interval = [&](int i, const Pos &ps, int cq, int next, auto with_stencil) __attribute__((always_inline)) {
             constexpr bool ST = decltype(with_stencil)::value;
             const uint4 *zb = reinterpret_cast<const uint4 *>(Zb + (i & 1) * kSWZ) + hf * kSWStride + n;
             uint4 v[3][kSWNT];
-            f32x4 tp[4], kw[2], pq;
+            constexpr int NTP = GLOBAL ? 9 : 4;
+            f32x4 tp[NTP], pq;
             float z[4][4];
             auto load_v = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
@@ -213,20 +263,16 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             };
             load_v(0);
             load_v(1);
-            if constexpr (ST) {
-                pq = pad_quad(cq);
-                kw[0] = kernL[0];
-#pragma unroll
-                for (int t = 0; t < 3; ++t) tp[t] = load_tap(ps, cq, t);
-            }
+            if constexpr (ST) pq = pad_quad(cq);
 #pragma unroll
             for (int st = 0; st < 12; ++st) {
                 __builtin_amdgcn_sched_barrier(0);
                 const int j = st / 3;
                 if (st + 2 < 12) load_v(st + 2);
                 if constexpr (ST) {
-                    if (st + 3 < 9) tp[(st + 3) & 3] = load_tap(ps, cq, st + 3);
-                    if (st + 1 < 9) kw[(st + 1) & 1] = kernL[st + 1];
+#pragma unroll
+                    for (int t = 0; t < 9; ++t)
+                        if (st == (GLOBAL ? t / 3 : t > 1 ? t - 1 : 0)) tp[t % NTP] = load_tap(ps, cq, t);
                 }
                 const Split8 &wf = af[j & 1];
 #pragma unroll
@@ -246,60 +292,47 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                     af[j & 1] = frag(wA, j < 2 ? 4 * i + j + 2 : 4 * next + j - 2);
                 }
                 if constexpr (ST) {
-                    if (st < 9) add_tap(ps, pq, tp[st & 3], kw[st & 1], st, z);
-                    if (st == 9) put_half(z, 0, (i + 1) & 1);
-                    if (st == 10) put_half(z, 1, (i + 1) & 1);
+#pragma unroll
+                    for (int t = 0; t < 9; ++t)
+                        if (st == (GLOBAL ? 2 + t : 1 + t)) add_tap(ps, pq, tp[t % NTP], kernL[t], t, z);
+                    if (st == 10) put_half(z, 0, (i + 1) & 1);
+                    if (st == 11) put_half(z, 1, (i + 1) & 1);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
-            __syncthreads();
         };
 #pragma unroll 1
-        for (int i = 0; i + 1 < KS; ++i) interval(i, pos, 4 * (i + 1) + sq, i + 1, std::true_type{});
+        for (int i = 0; i + 1 < KS; ++i) {
+            const float warm = GLOBAL ? warm_fire(g0) : 0.0f;
+            interval(i, pos, 4 * (i + 1) + sq, i + 1, std::true_type{});
+            if constexpr (GLOBAL) {
+                asm volatile("" ::"v"(warm));
+                if (i == 0 && w >= 6) draw_pass(g0);
+            }
+            __syncthreads();
+            if (tid < 4) badL[(bad == badL ? 4 : 0) + tid] = 0;
+        }
         if constexpr (GLOBAL) pos = locate(g0_next + sc);
         interval(KS - 1, pos, sq, 0, std::integral_constant<bool, GLOBAL>{});
-        // ---- fc2 and the update, NTR 32-cell tiles at a time
+
+        // ---- fc2 and the update, a round of NTR 32-cell tiles after another: the partial sums of a
+        // round meet in RED between two barriers; a round's update runs beside the next one's products
+        constexpr int RC = 32 * NTR, NR = (kSWNT + NTR - 1) / NTR;
+        const int ic = tid % RC, iq = tid / RC;  // this thread's item of a round: cell, channel quad
+        Split8 wf[MT][2];
+        bool nanh[2][NTR];
 #pragma unroll
-        for (int t0 = 0; t0 < kSWNT; t0 += NTR) {
-            // the item of this thread: cell ic of the round, channel quad iq
-            constexpr int RC = 32 * NTR;
-            const int ic = tid % RC, iq = tid / RC;
-            const int gq = g0 + 32 * t0 + ic;
-            const bool live = gq < ncell && 32 * t0 + ic < kSWN;
-            const int gc = live ? gq : g0;
-            const int row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
-            const int64_t grow = rbase + row;
-            f32x4 xo;
-            int gv;
-            float f;
-            if constexpr (GLOBAL) {
-                if (IN_NCHW) {
-                    const float *xr = a.x_in + (grow * C + 4 * iq) * HWn + q;
-                    xo = f32x4{xr[0], xr[HWn], xr[2 * HWn], xr[3 * HWn]};
-                } else {
-                    xo = *reinterpret_cast<const f32x4 *>(a.x_in + (int64_t)gc * C + 4 * iq);
-                }
-                gv = a.given[gc];
-                f = fireG[live ? 32 * t0 + ic : 0];
-            } else {
-                xo = *reinterpret_cast<const f32x4 *>(P + cur * PB + ci[gc] * CP + 4 * iq);
-                gv = givenL[gc];
-                f = a.fire_f32 ? a.fire_f32[grow * HWn + q] : fireL[(s & 1) * sp.R * HWn + gc] ? 1.0f : 0.0f;
-            }
-            Split8 wf[2] = {frag(wB, 0), frag(wB, 1)};
-            auto put_part = [&](int tr, int mt, f32x16 d) __attribute__((always_inline)) {
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    RED[(w * NQ + 8 * mt + 2 * v + hf) * RC + 32 * tr + n] =
-                        make_float4(d[4 * v], d[4 * v + 1], d[4 * v + 2], d[4 * v + 3]);
-            };
+        for (int mt = 0; mt < MT; ++mt) wf[mt][0] = frag(wB, 2 * mt), wf[mt][1] = frag(wB, 2 * mt + 1);
+        f32x16 part[NTR][MT];
+        Split8 hs[2][NTR][2];
+        // h of the round's tiles in three parts, as the products' B operands; round rd's in hs[rd & 1]
+        auto split_h = [&](int rd) __attribute__((always_inline)) {
 #pragma unroll
             for (int tr = 0; tr < NTR; ++tr) {
-                const int t = t0 + tr;
+                const int t = rd * NTR + tr;
                 if (t >= kSWNT) break;
                 const f32x16 h = big[t] + small[t];
                 bool nan = false;
-                Split8 hs[2];
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
                     float hv[8];
@@ -307,121 +340,223 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                     for (int v = 0; v < 8; ++v) hv[v] = relu_f32(h[8 * j + v]);
 #pragma unroll
                     for (int v = 0; v < 8; v += 2) nan |= __builtin_isunordered(h[8 * j + v], h[8 * j + v + 1]);
-                    hs[j] = split8(hv);
+                    hs[rd & 1][tr][j] = split8(hv);
+                }
+                nanh[rd & 1][tr] = nan;
+            }
+        };
+        auto products = [&](int rd) __attribute__((always_inline)) {
+            // the smaller products first: the sums are full-size for the last two only
+#pragma unroll
+            for (int tr = 0; tr < NTR; ++tr)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) part[tr][mt] = f32x16{};
+            auto add = [&](auto pw, auto ph) __attribute__((always_inline)) {
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int tr = 0; tr < NTR; ++tr)
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt)
+                            if (rd * NTR + tr < kSWNT)
+                                part[tr][mt] = mfma32(wf[mt][j].*pw, hs[rd & 1][tr][j].*ph, part[tr][mt]);
+            };
+            add(&Split8::l, &Split8::h);
+            add(&Split8::h, &Split8::l);
+            add(&Split8::m, &Split8::m);
+            add(&Split8::m, &Split8::h);
+            add(&Split8::h, &Split8::m);
+            add(&Split8::h, &Split8::h);
+        };
+        // marks tiles with a NaN among h
+        auto mark = [&](int rd) __attribute__((always_inline)) {
+#pragma unroll
+            for (int tr = 0; tr < NTR; ++tr)
+                if (rd * NTR + tr < kSWNT && __ballot(nanh[rd & 1][tr]) && lane == 0) bad[rd * NTR + tr] = 1;
+        };
+        // one MFMA, then VALU work beside it
+        auto mix = [&](int mfmas) __attribute__((always_inline)) {
+#pragma unroll
+            for (int k = 0; k < 24; ++k)
+                if (k < mfmas) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+                }
+        };
+        auto put_part = [&](int tr, int mt, f32x16 d) __attribute__((always_inline)) {
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                RED[(w * NQ + 8 * mt + 2 * v + hf) * RC + 32 * tr + n] =
+                    make_float4(d[4 * v], d[4 * v + 1], d[4 * v + 2], d[4 * v + 3]);
+        };
+        // the update of the round's items: the sums from RED and the new state, without a branch, then the
+        // rest; a NaN of dx marks the round's tiles
+        auto sums = [&](f32x4 xo, int gv, float f, f32x4 &u) __attribute__((always_inline)) {
+            float4 r[8];
+#pragma unroll
+            for (int k8 = 0; k8 < 8; ++k8) r[k8] = RED[(k8 * NQ + iq) * RC + ic];
+            f32x4 dx;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                auto e = [&](int k8) { return (&r[k8].x)[v]; };
+                dx[v] = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(e(0), e(1)), __fadd_rn(e(2), e(3))),
+                                            __fadd_rn(__fadd_rn(e(4), e(5)), __fadd_rn(e(6), e(7)))),
+                                  (&b2v.x)[v]);
+                const int c = 4 * iq + v;
+                const float uv = __fadd_rn(xo[v], __fmul_rn(f, dx[v]));
+                u[v] = (gv != 0) & (c >= in_off) & (c < in_off + c_in) ? xo[v] : uv;
+            }
+            return __builtin_isunordered(dx[0], dx[1]) | __builtin_isunordered(dx[2], dx[3]);
+        };
+        auto finish = [&](int t0, f32x4 u, int gv, float f, bool nan, bool again) __attribute__((always_inline)) {
+            const int k = 32 * t0 + ic, gq = g0 + k;
+            const bool live = gq < ncell && k < kSWN;
+            const int gc = live ? gq : g0;
+            if (!again && __ballot(live && nan) && lane == 0) {
+                bad[t0] = 1;  // a wave's lanes lie in one of the round's tiles, or in both
+                if (NTR > 1 && t0 + 1 < kSWNT) bad[t0 + 1] = 1;
+            }
+            if (a.noise || (first && c_in > 0) || (!GLOBAL && (a.x_rec || a.fire_f32)) || (GLOBAL && OUT_NCHW)) {
+                const int row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
+                const int64_t grow = rbase + row;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int c = 4 * iq + v;
+                    const bool frozen = (gv != 0) & (c >= in_off) & (c < in_off + c_in);
+                    if (a.noise && !frozen) u[v] = __fadd_rn(u[v], a.noise[(grow * C + c) * HWn + q]);
+                    if (first && frozen) u[v] = a.clamp[(grow * c_in + c - in_off) * HWn + q];
+                }
+                float *xr = nullptr;
+                if (GLOBAL && OUT_NCHW) xr = a.x_out;
+                if (!GLOBAL && a.x_rec) xr = a.x_rec + s * a.rec_stride;
+                if (xr && live) {
+                    xr += (grow * C + 4 * iq) * HWn + q;
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) xr[(int64_t)v * HWn] = u[v];
+                }
+                if (!GLOBAL && a.fire_f32 && !again && live && iq == 0 && f != 0.0f) atomicAdd(&firedL[row], 1);
+            }
+            if (!live) return;
+            if constexpr (!GLOBAL)
+                *reinterpret_cast<f32x4 *>(P + (cur ^ 1) * PB + ci[gc] * CP + 4 * iq) = u;
+            else if constexpr (!OUT_NCHW)
+                *reinterpret_cast<f32x4 *>(a.x_out + (int64_t)gc * C + 4 * iq) = u;
+        };
+        // what the update of this thread's item reads besides
+        auto load_item = [&](int t0, f32x4 &xo, int &gv, float &f) __attribute__((always_inline)) {
+            const int k = 32 * t0 + ic, gq = g0 + k;
+            const bool live = gq < ncell && k < kSWN;
+            const int gc = live ? gq : g0;
+            if constexpr (GLOBAL) {
+                if (IN_NCHW) {
+                    const int row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
+                    const float *xr = a.x_in + ((int64_t)row * C + 4 * iq) * HWn + q;
+                    xo = f32x4{xr[0], xr[HWn], xr[2 * HWn], xr[3 * HWn]};
+                } else {
+                    xo = *reinterpret_cast<const f32x4 *>(a.x_in + (int64_t)gc * C + 4 * iq);
+                }
+                gv = a.given[gc];
+                f = fireG[live ? k : 0];
+            } else {
+                xo = *reinterpret_cast<const f32x4 *>(P + cur * PB + ci[gc] * CP + 4 * iq);
+                gv = givenL[gc];
+                f = a.fire_f32 ? a.fire_f32[rbase * HWn + gc] : fireL[(s & 1) * sp.R * HWn + gc] ? 1.0f : 0.0f;
+            }
+        };
+        // a NaN among a round's sums: its cells on fp32 MFMA (z through RED, feature-major)
+        auto redo = [&](int t0) {
+            const int k = 32 * t0 + ic, gq = g0 + k;
+            const int gc = gq < ncell && k < kSWN ? gq : g0;
+            float *zf = reinterpret_cast<float *>(RED);
+            const float *w1f = reinterpret_cast<const float *>(a.packed + a.off_w1);
+            const float *w2f = reinterpret_cast<const float *>(a.packed + a.off_w2);
+            asm volatile("" : "+s"(w1f), "+s"(w2f));  // addresses formed here, not kept across the passes
+            {
+                const Pos p = locate(gc);
+                float z[4][4];
+                stencil_quad(p, iq, z);
+#pragma unroll
+                for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) zf[(kk * C + 4 * iq + c) * RC + ic] = z[kk][c];
+            }
+            __syncthreads();
+            f32x16 pt[NTR][MT];
+#pragma unroll
+            for (int tr = 0; tr < NTR; ++tr) {
+                f32x16 h = bias();
+#pragma unroll 1
+                for (int kk = 0; kk < 4 * C; kk += 2) {
+                    const float av = w1f[((2 * w + (n >> 4)) * C + (kk >> 2)) * 64 + ((kk & 3) + hf) * 16 + (n & 15)];
+                    h = __builtin_amdgcn_mfma_f32_32x32x2f32(av, zf[(kk + hf) * RC + 32 * tr + n], h, 0, 0, 0);
                 }
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
-                    __builtin_amdgcn_sched_barrier(0);
-                    const Split8 w0 = wf[0], w1 = wf[1];
-                    if (tr + 1 < NTR || mt + 1 < MT) {
-                        wf[0] = frag(wB, 2 * ((mt + 1) % MT));
-                        wf[1] = frag(wB, 2 * ((mt + 1) % MT) + 1);
-                    }
-                    f32x16 db = f32x16{}, ds = f32x16{};
-                    ds = mfma32(w0.l, hs[0].h, ds);
-                    db = mfma32(w0.h, hs[0].h, db);
-                    ds = mfma32(w0.h, hs[0].l, ds);
-                    ds = mfma32(w0.m, hs[0].m, ds);
-                    ds = mfma32(w1.l, hs[1].h, ds);
-                    db = mfma32(w1.h, hs[1].h, db);
-                    ds = mfma32(w1.h, hs[1].l, ds);
-                    ds = mfma32(w1.m, hs[1].m, ds);
-                    ds = mfma32(w0.m, hs[0].h, ds);
-                    ds = mfma32(w0.h, hs[0].m, ds);
-                    ds = mfma32(w1.m, hs[1].h, ds);
-                    ds = mfma32(w1.h, hs[1].m, ds);
-                    const f32x16 d = db + ds;
+                    f32x16 d = f32x16{};
 #pragma unroll
-                    for (int v = 0; v < 16; v += 2) nan |= __builtin_isunordered(d[v], d[v + 1]);
-                    put_part(tr, mt, d);
+                    for (int v = 0; v < 16; ++v) {
+                        const int hid = 32 * w + 8 * (v / 4) + 4 * hf + v % 4, m = 32 * mt + n;
+                        const float av = w2f[((m >> 4) * (HD / 4) + (hid >> 2)) * 64 + (hid & 3) * 16 + (m & 15)];
+                        d = __builtin_amdgcn_mfma_f32_32x32x2f32(av, h[v] > 0.0f ? h[v] : 0.0f, d, 0, 0, 0);
+                    }
+                    pt[tr][mt] = d;
                 }
-                if (__ballot(nan) && lane == 0) bad[t] = 1;
             }
             __syncthreads();
-            bool redo = false;
 #pragma unroll
             for (int tr = 0; tr < NTR; ++tr)
-                if (t0 + tr < kSWNT) redo |= bad[t0 + tr] != 0;
-            if (__builtin_amdgcn_readfirstlane(redo)) {
-                // a NaN among the sums: this round's cells on fp32 MFMA (z through RED, feature-major)
-                float *zf = reinterpret_cast<float *>(RED);
-                const float *w1f = reinterpret_cast<const float *>(a.packed + a.off_w1);
-                const float *w2f = reinterpret_cast<const float *>(a.packed + a.off_w2);
-                asm volatile("" : "+s"(w1f), "+s"(w2f));  // addresses formed here, not kept across the passes
-                {
-                    const Pos p = locate(gc);
-                    float z[4][4];
-                    stencil_quad(p, iq, z);
 #pragma unroll
-                    for (int k = 0; k < 4; ++k)
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) zf[(k * C + 4 * iq + c) * RC + ic] = z[k][c];
-                }
-                __syncthreads();
-                f32x16 part[NTR][MT];
-                for (int tr = 0; tr < NTR; ++tr) {
-                    f32x16 h = bias();
-#pragma unroll 1
-                    for (int k = 0; k < 4 * C; k += 2) {
-                        const float av = w1f[((2 * w + (n >> 4)) * C + (k >> 2)) * 64 + ((k & 3) + hf) * 16 + (n & 15)];
-                        h = __builtin_amdgcn_mfma_f32_32x32x2f32(av, zf[(k + hf) * RC + 32 * tr + n], h, 0, 0, 0);
-                    }
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) {
-                        f32x16 d = f32x16{};
-#pragma unroll
-                        for (int v = 0; v < 16; ++v) {
-                            const int hid = 32 * w + 8 * (v / 4) + 4 * hf + v % 4, m = 32 * mt + n;
-                            const float av = w2f[((m >> 4) * (HD / 4) + (hid >> 2)) * 64 + (hid & 3) * 16 + (m & 15)];
-                            d = __builtin_amdgcn_mfma_f32_32x32x2f32(av, h[v] > 0.0f ? h[v] : 0.0f, d, 0, 0, 0);
-                        }
-                        part[tr][mt] = d;
-                    }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int tr = 0; tr < NTR; ++tr)
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) put_part(tr, mt, part[tr][mt]);
-                __syncthreads();
-            }
-            float4 r[8];
-#pragma unroll
-            for (int k = 0; k < 8; ++k) r[k] = RED[(k * NQ + iq) * RC + ic];
-            const float4 bq = b2[iq];
-            f32x4 u;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                auto e = [&](int k) { return (&r[k].x)[v]; };
-                const float dx = __fadd_rn(__fadd_rn(__fadd_rn(__fadd_rn(e(0), e(1)), __fadd_rn(e(2), e(3))),
-                                                     __fadd_rn(__fadd_rn(e(4), e(5)), __fadd_rn(e(6), e(7)))),
-                                           (&bq.x)[v]);
-                const int c = 4 * iq + v;
-                float uv = __fadd_rn(xo[v], __fmul_rn(f, dx));
-                if (a.noise) uv = __fadd_rn(uv, a.noise[(grow * C + c) * HWn + q]);
-                const bool frozen = gv && c >= in_off && c < in_off + c_in;
-                if (frozen) uv = first ? a.clamp[(grow * c_in + c - in_off) * HWn + q] : xo[v];
-                u[v] = uv;
-            }
-            if (live) {
-                if constexpr (!GLOBAL) {
-                    *reinterpret_cast<f32x4 *>(P + (cur ^ 1) * PB + ci[gc] * CP + 4 * iq) = u;
-                    if (a.x_rec) {
-                        float *xr = a.x_rec + s * a.rec_stride + (grow * C + 4 * iq) * HWn + q;
-#pragma unroll
-                        for (int v = 0; v < 4; ++v) xr[(int64_t)v * HWn] = u[v];
-                    }
-                    if (a.fire_f32 && iq == 0 && f != 0.0f) atomicAdd(&firedL[row], 1);
-                } else if (OUT_NCHW) {
-                    float *xr = a.x_out + (grow * C + 4 * iq) * HWn + q;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) xr[(int64_t)v * HWn] = u[v];
-                } else {
-                    *reinterpret_cast<f32x4 *>(a.x_out + (int64_t)gc * C + 4 * iq) = u;
-                }
-            }
+                for (int mt = 0; mt < MT; ++mt) put_part(tr, mt, pt[tr][mt]);
             __syncthreads();
+            f32x4 xo, u;
+            int gv;
+            float f;
+            load_item(t0, xo, gv, f);
+            sums(xo, gv, f, u);
+            finish(t0, u, gv, f, false, true);
+            __syncthreads();
+        };
+        // the global ones of all rounds now, ahead of their use
+        f32x4 xo[NR];
+        int gv[NR];
+        float f[NR];
+        if constexpr (GLOBAL) {
+#pragma unroll
+            for (int rd = 0; rd < NR; ++rd) load_item(rd * NTR, xo[rd], gv[rd], f[rd]);
         }
+        split_h(0);
+        __builtin_amdgcn_sched_barrier(0);
+        products(0);
+        if (NR > 1) split_h(1);
+        mix(12 * NTR * MT);
+        __builtin_amdgcn_sched_barrier(0);
+        mark(0);
+        __syncthreads();  // Z's last half is read (RED may take its place)
+#pragma unroll
+        for (int rd = 0; rd < NR; ++rd) {
+            const int t0 = rd * NTR;
+#pragma unroll
+            for (int tr = 0; tr < NTR; ++tr)
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    if (t0 + tr < kSWNT) put_part(tr, mt, part[tr][mt]);
+            if constexpr (!GLOBAL) load_item(t0, xo[rd], gv[rd], f[rd]);
+            __syncthreads();
+            f32x4 u;
+            __builtin_amdgcn_sched_barrier(0);
+            if (rd + 1 < NR) products(rd + 1);
+            const bool nan = sums(xo[rd], gv[rd], f[rd], u);
+            if (rd + 2 < NR) split_h(rd + 2);
+            if (rd + 1 < NR) mix(12 * NTR * MT);
+            __builtin_amdgcn_sched_barrier(0);
+            if (rd + 1 < NR) mark(rd + 1);
+            finish(t0, u, gv[rd], f[rd], nan, false);
+            __syncthreads();
+            bool any = bad[t0] != 0;
+            if (NTR > 1 && t0 + 1 < kSWNT) any |= bad[t0 + 1] != 0;
+            if (__builtin_amdgcn_readfirstlane(any)) redo(t0);
+        }
+        bad = bad == badL ? badL + 4 : badL;
     };
 
     if constexpr (GLOBAL) {
@@ -429,47 +564,9 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         const int t_end = t_begin + sp.tiles_per_wg < sp.n_tiles ? t_begin + sp.tiles_per_wg : sp.n_tiles;
         Pos pos = locate(t_begin * kSWN + sc);
         put_z(pos);
-        const uint64_t key = a.step_seeds ? a.step_seeds[sp.step] : a.seed;
         __syncthreads();
         for (int t = t_begin; t < t_end; ++t) {
             const int g0 = t * kSWN;
-            if (w >= 6) {  // the fire factors of the pass's cells
-                const int k = tid - 384, gq = g0 + k;
-                const bool live = k < kSWN && gq < ncell;
-                const int gc = live ? gq : g0, row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
-                float f;
-                if (a.fire_f32) {
-                    f = a.fire_f32[gc];
-                } else if (a.fire_u8) {
-                    f = a.fire_u8[(int64_t)sp.step * ncell + gc] ? 1.0f : 0.0f;
-                } else {
-                    float u4[4];
-                    cell_uniforms4(key, (uint32_t)(a.row0 + row), (uint32_t)(a.step0 + sp.step), (uint32_t)(q >> 2), u4);
-                    const float u = (q & 3) == 0 ? u4[0] : (q & 3) == 1 ? u4[1] : (q & 3) == 2 ? u4[2] : u4[3];
-                    float p = a.p;
-                    if (a.adaptive) {
-                        const float *hw = reinterpret_cast<const float *>(a.packed + a.off_headw);
-                        const float *hb = reinterpret_cast<const float *>(a.packed + a.off_headb);
-                        int am;
-                        const float *xc = IN_NCHW ? a.x_in + ((int64_t)row * C + a.out_off) * HWn + q
-                                                  : a.x_in + (int64_t)gc * C + a.out_off;
-                        const float cf = cell_readout(xc, IN_NCHW ? HWn : 1, a.c_out, a.n_out, a.head_kind, hw, hb, &am);
-                        if (cf > a.tau || (a.given_confident && a.given[gc])) p = a.p_low;
-                    }
-                    f = u < p ? 1.0f : 0.0f;
-                }
-                if (k < kSWN) fireG[k] = f;
-                if (a.fired_out) {
-                    // one addition per row of the wave's cells
-                    uint64_t rest = __ballot(live && f != 0.0f);
-                    while (rest) {
-                        const int r0 = __builtin_amdgcn_readlane(row, (int)__builtin_ctzll(rest));
-                        const uint64_t mine = __ballot(live && f != 0.0f && row == r0);
-                        if (lane == 0) atomicAdd(a.fired_out + r0, (int)__popcll(mine));
-                        rest &= ~mine;
-                    }
-                }
-            }
             pass(g0, t + 1 < t_end ? g0 + kSWN : g0, sp.step, sp.first != 0, pos);
         }
     } else {

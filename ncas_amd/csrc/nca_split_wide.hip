@@ -11,7 +11,7 @@ namespace nca {
 namespace {
 
 constexpr unsigned kWideLds = 160u * 1024u;
-constexpr unsigned kSmallBytes = 4u * (256 + kSWN + 4 + 36);  // fc1's bias, fire factors, NaN flags, kernels
+constexpr unsigned kSmallBytes = 4u * (256 + kSWN + 8 + 36);  // fc1's bias, fire factors, NaN flags, kernels
 
 // LDS plan of R rows' rollout; false when it does not fit
 bool wide_plan(int C, int R, int H, int W, int c_out, int n_out, SplitWide *sp) {
