@@ -770,7 +770,9 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
     }
     if (!packed || !x_in || !given || (!clamp && cell->c_in > 0) || !x_out || !x_rec) return NCA_OK;
     const bool split = split_resident(cell, rows, H, W);
-    if (fire->adaptive || rows < 1 || n_steps < 1 || (!split && !takes_stream32(cell, rows, H, W))) return NCA_OK;
+    const bool s64 = g_path == 0 && cell->precision == NCA_BF16 && cell->channels == 64 && cell->hidden == 256 &&
+                     takes_resident(cell, rows, H, W);
+    if (fire->adaptive || rows < 1 || n_steps < 1 || (!split && !s64 && !takes_stream32(cell, rows, H, W))) return NCA_OK;
     nca::RolloutParams p = base_params(cell, packed, rows, H, W);
     p.x_in = x_in;
     p.x_out = x_out;
@@ -792,6 +794,8 @@ int rollout_recorded(const nca_cell_desc *cell, const void *packed, int64_t rows
         *used = true;
         return hip_check(split_rollout(cell->channels, p, st), "split rollout launch");
     }
+    // the boards that its single steps run on too (else *used stays false)
+    if (s64) return hip_check(nca::launch_stream64(p, st, kLdsBytes, used), "streamed rollout launch");
     int P = xch ? recorded_pieces(cell, rows, H, W) : 1;
     if (P > 1 && xch_bytes < nca::stream32_xch_bytes(rows, P, W)) P = 1;
     const int rc = hip_check(nca::launch_stream32(p, st, kLdsBytes, used, P, static_cast<uint64_t *>(xch)),

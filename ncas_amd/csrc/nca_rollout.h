@@ -56,7 +56,7 @@ struct RolloutParams {
     float *conf_out;
     int32_t *fired_out;
     float *x_rec;        // or null: the state after step s of the call goes to x_rec + s rec_stride
-    int64_t rec_stride;  // (the streamed C = 32 kernel and the fp32 C = 16 kernel only)
+    int64_t rec_stride;  // (the streamed kernels and the fp32 kernels of nca_split.h only)
     float *x_rec0;       // or null: the call's input state copied there (the same kernels, with x_rec)
     int64_t rows;
     int H, W;

@@ -136,6 +136,10 @@ struct StParams {
     unsigned off_w1q, off_w2h;
 };
 
+// REC: also write the state after every step to a.x_rec (the BPTT chunk's forward; 128 boards of 9x9, 32
+// steps: 255 us in one launch, 842 us as a launch per step, each of which loads the weights, the
+// tables and the state anew). The stores are the update lanes' own, beside the hidden waves' MFMAs.
+template <bool REC>
 __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {
     using S = St64;
     constexpr int NT = 512;
@@ -661,6 +665,8 @@ __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {
             const unsigned kHr = sp.l_H + (unsigned)n * S::HS + 16u * ((unsigned)g ^ hx);
             int cbU = RH - 48;    // cinfo index of the update tile's first cell: (16 (i-3)) mod RH
             int rbU = RING - 48;  // its ring slot: (16 (i-3)) mod RING
+            int sU = -1;          // its step (REC)
+            const uint32_t magic = 0xffffffffu / (uint32_t)HWn + 1;  // c / HWn = mulhi(c, magic) for c < 2^16, HWn > 1
             uint2 ciu = make_uint2(0u, 0u), ciu_n = ciu;
             auto uinterval = [&](auto up_c, auto last_c) __attribute__((always_inline)) {
                 constexpr bool DUP = decltype(up_c)::value, LAST = decltype(last_c)::value;
@@ -694,6 +700,16 @@ __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {
                         acc[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w2f[mt][kt], hb[kt], acc[mt], 0, 0, 0);
                 bool ok = true;
                 if (LAST) ok = 16 * (i - 3) + n < total;
+                float *xr = nullptr;
+                if (REC) {  // where the lane's cell is recorded
+                    int c = cbU + n, sc = sU;
+                    if (c >= RH) {
+                        c -= RH;
+                        ++sc;
+                    }
+                    const int r = HWn > 1 ? (int)__umulhi((uint32_t)c, magic) : c;
+                    if (ok && r < Rw) xr = a.x_rec + sc * a.rec_stride + ((rbase + r) * S::C + 4 * iq0) * (int64_t)HWn + (c - r * HWn);
+                }
 #pragma unroll
                 for (int mt = 0; mt < 2; ++mt) {
                     const uint32_t d01 = cvt_pk_bf16(acc[mt][0], acc[mt][1]), d23 = cvt_pk_bf16(acc[mt][2], acc[mt][3]);
@@ -710,12 +726,19 @@ __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {
                         lds_st128f(smem, madr + 64u * mt, make_float4(u[0], u[1], u[2], u[3]));
                         lds_st64(smem, padr + 32u * mt, make_uint2(cvt_pk_bf16(u[0], u[1]), cvt_pk_bf16(u[2], u[3])));
                     }
+                    if (REC && xr) {
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) xr[(int64_t)(16 * mt + v) * HWn] = u[v];
+                    }
                 }
             };
             auto advance = [&]() __attribute__((always_inline)) {
                 ++i;
                 cbU += 16;
-                if (cbU >= RH) cbU -= RH;
+                if (cbU >= RH) {
+                    cbU -= RH;
+                    if (REC) ++sU;
+                }
                 rbU += 16;
                 if (rbU >= RING) rbU -= RING;
                 ciu = ciu_n;
@@ -740,6 +763,8 @@ __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {
     }
 
     // ---- write back
+    if (REC && a.x_rec0)
+        for (int e = tid; e < Rw * S::C * HWn; e += NT) a.x_rec0[rbase * S::C * HWn + e] = a.x_in[rbase * S::C * HWn + e];
     for (int e = tid; e < Rw * S::C * HWn; e += NT) {
         const int r = e / (S::C * HWn), rem = e - r * S::C * HWn, ch = rem / HWn, q = rem - ch * HWn;
         a.x_out[rbase * S::C * HWn + e] = m_at(r, q, ch);

@@ -15,6 +15,7 @@ namespace nca {
 // the LDS and 16-bit halo offsets.
 hipError_t launch_stream64(const RolloutParams &p, hipStream_t st, unsigned lds_limit, bool *used) {
     *used = false;
+    if (p.x_rec && p.adaptive) return hipSuccess;  // recording is for uniform firing
     if (p.W + 1 > 16 || 2 * (p.W + 2) + 2 * p.H > 64 || p.noise || p.fire_f32) return hipSuccess;
     const int hw = p.H * p.W, nq4 = (hw + 3) / 4;
     const bool batched = !p.adaptive && !p.fire_u8;
@@ -46,7 +47,7 @@ hipError_t launch_stream64(const RolloutParams &p, hipStream_t st, unsigned lds_
     sp.l_evp = L.evp;
     sp.off_w1q = p.off_w1q;
     sp.off_w2h = p.off_w2h;
-    auto kfn = rollout_stream64;
+    auto kfn = p.x_rec ? rollout_stream64<true> : rollout_stream64<false>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kfn),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)L.total);
     if (e != hipSuccess) return e;
