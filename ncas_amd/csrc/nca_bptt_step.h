@@ -16,7 +16,7 @@
 // fragments come from the L2 once per tile, 16 bytes a lane, instead of staying in registers, so
 // that two workgroups fit a CU and the fp32 C = 64 cell (576 KB of weights) runs the same code.
 //
-// z, h, g_a and g_dx of up to G steps are kept tile-major ([tile][feature][32 cells]: a tile's
+// z, h, g_a and g_dx of up to G steps (160 MB) are kept tile-major ([tile][feature][32 cells]: a tile's
 // stores are one contiguous run, and so are 16 features of 32 cells, an MFMA operand), and
 // `weight_grads` sums dW1 = g_a z^T, dW2 = g_dx h^T, db1 and db2 over all their cells at once: a
 // split-K product over G * M cells writes its partial sums once per group where one over each
