@@ -261,7 +261,7 @@ __global__ void pack_all(PackArgs a) {
         pack_small(a.head_b, a.nhb, reinterpret_cast<float *>(pk + a.L.headb), 0, 0, 1);
         pack_small(a.pad_vec, a.C, reinterpret_cast<float *>(pk + a.L.padv), 0, 0, 1);
     } else if (part == 0) {
-        pack_frags(a.w1, a.HD, a.F, a.bf, 0, (void *)(pk + a.L.w1), pb, kPB);
+        if (a.bf) pack_frags(a.w1, a.HD, a.F, a.bf, 0, (void *)(pk + a.L.w1), pb, kPB);  // fp32: the backward's
     } else if (part == 1) {
         pack_frags(a.w2, a.C, a.HD, a.bf, 0, (void *)(pk + a.L.w2), pb, kPB);
     } else if (part == 2 && !a.bf) {

@@ -8,7 +8,8 @@
 //                             runs outside autocast, reference src/nca/rollout.py:184-186)
 //   headb  float[n_out]
 //   padv   float[C]           wall border value
-//   w1     MFMA A fragments of fc1: [m-tile (hidden/16)][k-tile][lane 64][slot]
+//   w1     MFMA A fragments of fc1: [m-tile (hidden/16)][k-tile][lane 64][slot]; fp32 cells: bw1, whose
+//          unit element s is k-tile 4 k-block + s
 //   w2     MFMA A fragments of fc2: [m-tile (C/16)][k-tile][lane 64][slot]
 //   w2h    (bf16 only) fc2 fragments for the streamed kernel, whose hidden activations sit in
 //          LDS in the order of fc1's accumulators: physical position p = 64 w + 16 g + 4 mt + v
@@ -65,7 +66,7 @@ __host__ __device__ inline PackedLayout packed_layout(int C, int heads, int hidd
     o = align256(o + sizeof(float) * C);
     const size_t esz = bf16 ? 2 : 4;
     L.w1 = o;
-    o = align256(o + esz * (size_t)hidden * heads * C);
+    o = align256(o + (bf16 ? 2 * (size_t)hidden * heads * C : 0));
     L.w2 = o;
     o = align256(o + esz * (size_t)C * hidden);
     L.w2h = o;  // bf16 cells: fc2 fragments in the streamed kernel's hidden order
@@ -75,6 +76,7 @@ __host__ __device__ inline PackedLayout packed_layout(int C, int heads, int hidd
     L.w2k = o;  // bf16 cells: fc2 fragments per hidden quarter
     o = align256(o + (bf16 ? 2 * (size_t)C * hidden : 0));
     L.bw1 = o;
+    if (!bf16) L.w1 = o;
     o = align256(o + esz * (size_t)hidden * heads * C);
     L.bw1t = o;
     o = align256(o + esz * (size_t)hidden * heads * C);

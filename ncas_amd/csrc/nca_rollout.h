@@ -244,7 +244,8 @@ __global__ void __launch_bounds__(256, 1) rollout_resident(RolloutParams a) {
     for (int mt = 0; mt < S::MT1; ++mt) {
 #pragma unroll
         for (int kt = 0; kt < S::KT1; ++kt) {
-            const size_t idx = ((size_t)(wave * S::MT1 + mt) * S::KT1 + kt) * 64 + lane;
+            const size_t m1 = wave * S::MT1 + mt;
+            const size_t idx = BF16 ? (m1 * S::KT1 + kt) * 64 + lane : ((m1 * (S::KT1 / 4) + kt / 4) * 64 + lane) * 4 + kt % 4;
             w1f[mt][kt] = reinterpret_cast<const fr_t *>(a.packed + a.off_w1)[idx];
         }
 #pragma unroll

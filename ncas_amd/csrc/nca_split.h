@@ -102,7 +102,7 @@ __device__ __forceinline__ f32x4 mlp16_fp32(const float z[4][4], const float *w1
         for (int k = 0; k < 4; ++k)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                h = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[(mt * 16 + 4 * k + g) * 64 + 16 * c + l16], z[k][c], h, 0, 0, 0);
+                h = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[((mt * 4 + k) * 64 + 16 * c + l16) * 4 + g], z[k][c], h, 0, 0, 0);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
             dx = __builtin_amdgcn_mfma_f32_16x16x4f32(w2[(4 * mt + g) * 64 + 16 * v + l16], h[v] > 0.0f ? h[v] : 0.0f, dx, 0, 0, 0);

@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                 f32x16 h = bias();
 #pragma unroll 1
                 for (int kk = 0; kk < 4 * C; kk += 2) {
-                    const float av = w1f[((2 * w + (n >> 4)) * C + (kk >> 2)) * 64 + ((kk & 3) + hf) * 16 + (n & 15)];
+                    const float av = w1f[(((2 * w + (n >> 4)) * (C / 4) + (kk >> 4)) * 64 + ((kk & 3) + hf) * 16 + (n & 15)) * 4 + ((kk >> 2) & 3)];
                     h = __builtin_amdgcn_mfma_f32_32x32x2f32(av, zf[(kk + hf) * RC + 32 * tr + n], h, 0, 0, 0);
                 }
 #pragma unroll

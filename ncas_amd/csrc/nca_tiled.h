@@ -158,7 +158,8 @@ __global__ void __launch_bounds__(256, 1) step_tiled(TiledParams tp) {
     for (int mt = 0; mt < T::MT1; ++mt) {
 #pragma unroll
         for (int kt = 0; kt < T::KT1; ++kt) {
-            const size_t idx = ((size_t)(wave * T::MT1 + mt) * T::KT1 + kt) * 64 + lane;
+            const size_t m1 = wave * T::MT1 + mt;
+            const size_t idx = BF16 ? (m1 * T::KT1 + kt) * 64 + lane : ((m1 * (T::KT1 / 4) + kt / 4) * 64 + lane) * 4 + kt % 4;
             w1f[mt][kt] = reinterpret_cast<const fr_t *>(a.packed + a.off_w1)[idx];
         }
 #pragma unroll
