@@ -14,8 +14,10 @@
 //
 // The exponent range is fp32's. A value that rounds to an infinite h (or is infinite or NaN) makes
 // m or l NaN, hence every output of its cell: a tile with a NaN among fc1's or fc2's sums is
-// computed again on fp32 MFMA (a branch uniform over the wave), so infinities and NaN come out
-// as they do there.
+// computed again on fp32 MFMA (a branch uniform over the wave), and the cells with a NaN of their
+// own take that result, so infinities and NaN come out as they do there. An MFMA's columns
+// are its cells and do not mix: the tile's other cells keep theirs, so that a cell's
+// bits do not depend on which cells share its tile.
 #pragma once
 
 #include "nca_rollout.h"
@@ -89,7 +91,7 @@ __device__ __forceinline__ Split8 lds_frag3(const unsigned char *wl, int first, 
     return Split8{p[0], p[64], p[128]};
 }
 
-// fp32 MFMA on the forward's packed fp32 fragments (global memory): tiles with a NaN
+// fp32 MFMA on the forward's packed fp32 fragments (global memory): tiles that hold a NaN
 __device__ __forceinline__ f32x4 mlp16_fp32(const float z[4][4], const float *w1, const float *w2, const float *b1L, f32x4 b2v,
                                             int lane) {
     const int g = lane >> 4, l16 = lane & 15;
@@ -154,7 +156,14 @@ __device__ __forceinline__ f32x4 mlp16_split(const float z[4][4], const unsigned
     }
     f32x4 dx = (dl[0] + dl[1]) + ds;
     bad |= __builtin_isunordered(dx[0], dx[1]) | __builtin_isunordered(dx[2], dx[3]);
-    if (__ballot(bad)) dx = mlp16_fp32(z, w1, w2, b1L, b2v, lane);
+    const uint64_t nan = __ballot(bad);
+    if (nan) {
+        const uint64_t cells = nan | nan >> 16 | nan >> 32 | nan >> 48;  // bits 0..15: over the cell's four lanes
+        const f32x4 d = mlp16_fp32(z, w1, w2, b1L, b2v, lane);
+        const bool own = (cells >> (lane & 15)) & 1;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) dx[v] = own ? d[v] : dx[v];
+    }
     return dx;
 }
 

@@ -63,8 +63,8 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     float4 *RED = reinterpret_cast<float4 *>(smem + sp.l_red);
     float *b1L = reinterpret_cast<float *>(smem + sp.l_small);
     float *fireG = b1L + HD;                                // GLOBAL: fire factors of the pass's cells
-    // NaN among a 32-cell tile's sums, for even and odd passes: a pass clears the other's after its first
-    // barrier, when every wave is past the last look at them
+    // the cells of each 32-cell tile with a NaN among their sums, a bit each, for even and odd passes: a
+    // pass clears the other's after its first barrier, when every wave is past the last look at them
     int *badL = reinterpret_cast<int *>(fireG + kSWN), *bad = badL;
     f32x4 *kernL = reinterpret_cast<f32x4 *>(badL + 8);      // the 4 kernels' weights of each tap
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hf = lane >> 5;
@@ -375,11 +375,14 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             add(&Split8::h, &Split8::m);
             add(&Split8::h, &Split8::h);
         };
-        // marks tiles with a NaN among h
+        // marks cells with a NaN among h
         auto mark = [&](int rd) __attribute__((always_inline)) {
 #pragma unroll
-            for (int tr = 0; tr < NTR; ++tr)
-                if (rd * NTR + tr < kSWNT && __ballot(nanh[rd & 1][tr]) && lane == 0) bad[rd * NTR + tr] = 1;
+            for (int tr = 0; tr < NTR; ++tr) {
+                if (rd * NTR + tr >= kSWNT) break;
+                const uint64_t m = __ballot(nanh[rd & 1][tr]);
+                if (m && lane == 0) atomicOr(&bad[rd * NTR + tr], (int)(m | m >> 32));
+            }
         };
         // one MFMA, then VALU work beside it
         auto mix = [&](int mfmas) __attribute__((always_inline)) {
@@ -397,7 +400,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                     make_float4(d[4 * v], d[4 * v + 1], d[4 * v + 2], d[4 * v + 3]);
         };
         // the update of the round's items: the sums from RED and the new state, without a branch, then the
-        // rest; a NaN of dx marks the round's tiles
+        // rest; a NaN of dx marks its cell. again: only the marked cells
         auto sums = [&](f32x4 xo, int gv, float f, f32x4 &u) __attribute__((always_inline)) {
             float4 r[8];
 #pragma unroll
@@ -417,11 +420,18 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         };
         auto finish = [&](int t0, f32x4 u, int gv, float f, bool nan, bool again) __attribute__((always_inline)) {
             const int k = 32 * t0 + ic, gq = g0 + k;
-            const bool live = gq < ncell && k < kSWN;
+            bool live = gq < ncell && k < kSWN;
             const int gc = live ? gq : g0;
-            if (!again && __ballot(live && nan) && lane == 0) {
-                bad[t0] = 1;  // a wave's lanes lie in one of the round's tiles, or in both
-                if (NTR > 1 && t0 + 1 < kSWNT) bad[t0 + 1] = 1;
+            if (again) {
+                live = live && ((bad[t0 + (ic >> 5)] >> (ic & 31)) & 1);
+            } else if (const uint64_t m = __ballot(live && nan); m && lane == 0) {
+                // a wave's lanes are the round's 64 cells, or two quads of its 32
+                if (NTR > 1) {
+                    atomicOr(&bad[t0], (int)m);
+                    if (t0 + 1 < kSWNT) atomicOr(&bad[t0 + 1], (int)(m >> 32));
+                } else {
+                    atomicOr(&bad[t0], (int)(m | m >> 32));
+                }
             }
             if (a.noise || (first && c_in > 0) || (!GLOBAL && (a.x_rec || a.fire_f32)) || (GLOBAL && OUT_NCHW)) {
                 const int row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
@@ -470,7 +480,8 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                 f = a.fire_f32 ? a.fire_f32[rbase * HWn + gc] : fireL[(s & 1) * sp.R * HWn + gc] ? 1.0f : 0.0f;
             }
         };
-        // a NaN among a round's sums: its cells on fp32 MFMA (z through RED, feature-major)
+        // a NaN among a round's sums: its tiles on fp32 MFMA (z through RED, feature-major), whose result the
+        // marked cells take
         auto redo = [&](int t0) {
             const int k = 32 * t0 + ic, gq = g0 + k;
             const int gc = gq < ncell && k < kSWN ? gq : g0;

@@ -1,0 +1,44 @@
+"""fp32 cells on the bf16 matrix cores (nca_split.h): a row's result is its own. Boards that share tiles,
+passes or workgroups with a board of infinities or NaN keep their bits, and fused rollouts with such
+a board equal chained steps."""
+
+import pytest
+import torch
+
+from test_gpu_split import _run, _state
+
+pytestmark = pytest.mark.gpu
+
+# several rows per workgroup in LDS, and boards that run step by step; rows whose tiles and passes
+# cross from one board into the next
+CASES = [("maze_c16", (13, 13), 515), ("maze_c16", (5, 7), 600), ("maze_c16", (33, 35), 3),
+         ("maze_hard_c32", (5, 7), 700), ("maze_hard_c32", (13, 13), 3), ("maze_hard_c32", (24, 25), 5),
+         ("sudoku_c64", (9, 9), 515), ("sudoku_c64", (4, 5), 600)]
+
+
+def _same(a, b):
+    return torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())
+
+
+@pytest.mark.parametrize("name,shape,rows", CASES)
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3.4e38])
+@pytest.mark.parametrize("gated", [False, True])
+def test_a_board_does_not_change_its_neighbours(name, shape, rows, bad, gated):
+    m, md, x, g4, cl = _state(name, rows, shape, 4)
+    kw = dict(p_fire=0.8, p_low=0.2, tau=0.6) if gated else dict(p_fire=0.6)
+    xb = x.clone()
+    rb = rows // 2
+    xb[rb, m.cfg.channels - 1, -1, -1] = bad  # the board's last cell: beside the next board's first
+    xb[rb, m.cfg.channels - 1, 0, 0] = bad
+    others = torch.arange(rows) != rb
+    for n in (1, 3):
+        y, conf, fired = _run(md, x, g4, cl, n, **kw)
+        yb, confb, firedb = _run(md, xb, g4, cl, n, **kw)
+        assert not torch.equal(yb[rb], y[rb])  # (3.4e38, finite in fp32 and infinite in bf16, may stay finite)
+        assert torch.equal(yb[others], y[others]) and torch.equal(confb[others], conf[others])
+        assert torch.equal(firedb[others], fired[others])
+    cur, total = xb, 0
+    for t in range(3):
+        cur, c1, f1 = _run(md, cur, g4, cl, 1, step0=t, **kw)
+        total = total + f1
+    assert _same(yb, cur) and _same(confb, c1) and torch.equal(firedb, total)
