@@ -484,13 +484,14 @@ int launch_rollout(nca::RolloutParams p, hipStream_t st) {
 }
 
 // Does the call run on the fp32 kernels on the bf16 matrix cores (nca_split.h)? Every call of a shape
-// does or does not, whatever its steps, so that fused rollouts equal chained steps bit for bit.
-// Boards that fit neither their LDS plan nor the 31-bit offsets of their per-step kernel, and the few
-// that fit only the generic resident kernel's plan (which needs no workspace), stay there.
+// does or does not, whatever its steps and rows, so that fused rollouts equal chained steps, and a row
+// alone the same row among others, bit for bit. Boards that fit neither their LDS plan nor, one by one,
+// the 31-bit offsets of their per-step kernel, and the few that fit only the generic resident kernel's
+// plan (which needs no workspace), stay there.
 bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
     if (g_path != 0 || g_window_steps > 1 || d->precision != NCA_FP32 || d->channels != 16 || d->hidden != 128) return false;
     if (nca::split16_resident_fits(H, W, d->c_out, d->n_out)) return true;
-    return !takes_resident(d, rows, H, W) && nca::split16_step_fits(rows, H, W);
+    return !takes_resident(d, rows, H, W) && nca::split16_step_fits(H, W);
 }
 
 // The same for the C = 32 and C = 64 cells. The per-step kernel takes the C = 32 boards that the generic
@@ -499,7 +500,7 @@ bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
 bool takes_split_wide(const nca_cell_desc *d, int64_t rows, int H, int W) {
     if (g_path != 0 || d->precision != NCA_FP32 || d->hidden != 256 || (d->channels != 32 && d->channels != 64)) return false;
     if (nca::split_wide_resident_fits(d->channels, H, W, d->c_out, d->n_out)) return true;
-    return !takes_resident(d, rows, H, W) && nca::split_wide_step_fits(d->channels, rows, H, W);
+    return !takes_resident(d, rows, H, W) && nca::split_wide_step_fits(d->channels, H, W);
 }
 
 // Does a rollout or recorded chunk run on one of these kernels in LDS, in one launch?
@@ -655,7 +656,7 @@ int launch_cell(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t
         // one step on the per-step kernel, whose tiles spread over the whole device (out of place: in
         // place it would need a workspace); more of them in LDS where the boards fit
         const size_t sb = state_bytes(d, p.rows, p.H, p.W);
-        const bool fits = C == 16 ? nca::split16_step_fits(p.rows, p.H, p.W) : nca::split_wide_step_fits(C, p.rows, p.H, p.W);
+        const bool fits = C == 16 ? nca::split16_step_fits(p.H, p.W) : nca::split_wide_step_fits(C, p.H, p.W);
         const bool one = p.n_steps == 1 && fits && !overlaps(p.x_in, sb, p.x_out, sb);
         if (one || !split_resident(d, p.rows, p.H, p.W)) return run_tiled(d, p, st, ws, ws_bytes);
         return hip_check(split_rollout(C, p, st), "split rollout launch");

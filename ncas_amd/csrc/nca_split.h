@@ -184,9 +184,9 @@ __device__ __forceinline__ void stencil16(const f32x4 tp[9], const float *kern, 
 }
 
 struct Split16Step {
-    RolloutParams a;  // x_in -> x_out of this step (distinct buffers)
+    RolloutParams a;  // x_in -> x_out of this step (distinct buffers); fire_u8: this step's masks
     const unsigned char *wsplit;
-    int step;         // step index within the call (Philox counter step0 + step, mask slice)
+    int step;         // step index within the call (Philox counter step0 + step)
     int64_t n_tiles;  // rows * tiles_per_row
     int tiles_per_row;
     int64_t tiles_per_wg;

@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(kS16T, 1) step_split16(Split16Step sp) {
         in.gv = a.given[cell];
         // loaded without a branch (an absent mask loads something else, unused)
         in.fin = *(a.fire_f32 ? a.fire_f32 + cell : a.x_in + cell);
-        in.fu8 = *(a.fire_u8 ? a.fire_u8 + (int64_t)sp.step * a.rows * HWn + cell : a.given + cell);
+        in.fu8 = *(a.fire_u8 ? a.fire_u8 + cell : a.given + cell);
         if (FIRST) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {

@@ -58,9 +58,9 @@ bool split16_resident_fits(int H, int W, int c_out, int n_out) {
     return resident_plan(1, H, W, c_out, n_out, &sp);
 }
 
-bool split16_step_fits(int64_t rows, int H, int W) {
-    // 31-bit byte offsets into the cell-major state (cells past a row's end store at 2^31)
-    return rows * (int64_t)H * W * 16 * (int64_t)sizeof(float) < ((int64_t)1 << 31);
+bool split16_step_fits(int H, int W) {
+    // a row within 31-bit byte offsets into the cell-major state (cells past a row's end store at 2^31)
+    return (int64_t)H * W * 16 * (int64_t)sizeof(float) < ((int64_t)1 << 31);
 }
 
 hipError_t split16_rollout(const RolloutParams &p, hipStream_t st) {
@@ -82,17 +82,21 @@ hipError_t split16_rollout(const RolloutParams &p, hipStream_t st) {
 hipError_t split16_step(const RolloutParams &p, int step, int first, int in_nchw, int out_nchw, hipStream_t st) {
     Split16Step sp;
     memset(&sp, 0, sizeof(sp));
-    sp.a = p;
     sp.wsplit = p.packed + p.off_split;
     sp.step = step;
     sp.tiles_per_row = (p.H * p.W + 15) / 16;
-    sp.n_tiles = p.rows * (int64_t)sp.tiles_per_row;
     static const int n_cu = cu_count();
-    sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
-    if (sp.n_tiles < 1) return hipSuccess;
-    const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
-    if (in_nchw) return out_nchw ? launch_step<true, true>(sp, grid, first, st) : launch_step<true, false>(sp, grid, first, st);
-    return out_nchw ? launch_step<false, true>(sp, grid, first, st) : launch_step<false, false>(sp, grid, first, st);
+    const int64_t per = step_launch_rows(16, p.rows, p.H, p.W);
+    for (int64_t r0 = 0; r0 < p.rows; r0 += per) {
+        sp.a = step_rows(p, 16, step, r0, p.rows - r0 < per ? p.rows - r0 : per);
+        sp.n_tiles = sp.a.rows * (int64_t)sp.tiles_per_row;
+        sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
+        const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
+        const hipError_t e = in_nchw ? (out_nchw ? launch_step<true, true>(sp, grid, first, st) : launch_step<true, false>(sp, grid, first, st))
+                                     : (out_nchw ? launch_step<false, true>(sp, grid, first, st) : launch_step<false, false>(sp, grid, first, st));
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace nca

@@ -38,6 +38,7 @@ struct SplitWide {
     RolloutParams a;
     const unsigned char *wsplit;
     int step, first;            // per-step launches: step index within the call, first step of the call
+                                // (a.fire_u8: the step's masks)
     int n_cells, n_tiles, tiles_per_wg;
     int R;                      // rollouts in LDS: rows per workgroup
     unsigned l_Z, l_red, l_small, l_P, l_ci, l_fire, l_given, l_fired, l_head, total;
@@ -205,7 +206,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         if (a.fire_f32) {
             f = a.fire_f32[gc];
         } else if (a.fire_u8) {
-            f = a.fire_u8[(int64_t)sp.step * ncell + gc] ? 1.0f : 0.0f;
+            f = a.fire_u8[gc] ? 1.0f : 0.0f;
         } else {
             const uint64_t key = a.step_seeds ? a.step_seeds[sp.step] : a.seed;
             float u4[4];

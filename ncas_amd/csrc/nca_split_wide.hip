@@ -62,9 +62,9 @@ bool split_wide_resident_fits(int C, int H, int W, int c_out, int n_out) {
     return wide_plan(C, 1, H, W, c_out, n_out, &sp);
 }
 
-bool split_wide_step_fits(int C, int64_t rows, int H, int W) {
-    // 31-bit byte offsets into the state
-    return C == 32 && rows * (int64_t)H * W * C * (int64_t)sizeof(float) < ((int64_t)1 << 31);
+bool split_wide_step_fits(int C, int H, int W) {
+    // a row within 31-bit byte offsets into the state
+    return C == 32 && (int64_t)H * W * C * (int64_t)sizeof(float) < ((int64_t)1 << 31);
 }
 
 hipError_t split_wide_rollout(int C, const RolloutParams &p, hipStream_t st) {
@@ -89,22 +89,26 @@ hipError_t split_wide_rollout(int C, const RolloutParams &p, hipStream_t st) {
 hipError_t split_wide_step(const RolloutParams &p, int step, int first, int in_nchw, int out_nchw, hipStream_t st) {
     SplitWide sp;
     memset(&sp, 0, sizeof(sp));
-    sp.a = p;
     sp.wsplit = p.packed + p.off_split;
     sp.step = step;
     sp.first = first;
-    sp.n_cells = (int)(p.rows * p.H * p.W);
-    if (sp.n_cells < 1) return hipSuccess;
-    sp.n_tiles = (sp.n_cells + kSWN - 1) / kSWN;
-    static const int n_cu = cu_count();
-    sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
     sp.l_Z = 0;
     sp.l_red = 2 * kSWZ;
     sp.l_small = sp.l_red + kSWRed;
     sp.total = st_al16(sp.l_small + kSmallBytes);
-    const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
-    if (in_nchw) return out_nchw ? launch<32, true, true, true>(sp, grid, st) : launch<32, true, true, false>(sp, grid, st);
-    return out_nchw ? launch<32, true, false, true>(sp, grid, st) : launch<32, true, false, false>(sp, grid, st);
+    static const int n_cu = cu_count();
+    const int64_t per = step_launch_rows(32, p.rows, p.H, p.W);
+    for (int64_t r0 = 0; r0 < p.rows; r0 += per) {
+        sp.a = step_rows(p, 32, step, r0, p.rows - r0 < per ? p.rows - r0 : per);
+        sp.n_cells = (int)(sp.a.rows * p.H * p.W);
+        sp.n_tiles = (sp.n_cells + kSWN - 1) / kSWN;
+        sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
+        const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
+        const hipError_t e = in_nchw ? (out_nchw ? launch<32, true, true, true>(sp, grid, st) : launch<32, true, true, false>(sp, grid, st))
+                                     : (out_nchw ? launch<32, true, false, true>(sp, grid, st) : launch<32, true, false, false>(sp, grid, st));
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
 }
 
 }  // namespace nca

@@ -5,7 +5,10 @@ a board equal chained steps."""
 import pytest
 import torch
 
-from test_gpu_split import _run, _state
+from cells import make_model
+from ncas_amd.inference import rollout_steps
+from ncas_amd.step import make_step
+from test_gpu_split import DEV, _run, _state
 
 pytestmark = pytest.mark.gpu
 
@@ -42,3 +45,32 @@ def test_a_board_does_not_change_its_neighbours(name, shape, rows, bad, gated):
         cur, c1, f1 = _run(md, cur, g4, cl, 1, step0=t, **kw)
         total = total + f1
     assert _same(yb, cur) and _same(confb, c1) and torch.equal(firedb, total)
+
+
+@pytest.mark.parametrize("name,shape", [("maze_c16", (201, 201)), ("maze_hard_c32", (30, 30))])
+def test_rows_beyond_2_gib(name, shape):
+    """A state of more than 2 GiB runs on the kernels that its rows run on alone: the same bits, with
+    drawn, injected and float fire masks, noise, and fired counts."""
+    m = make_model(name).to(DEV)
+    C, c_in = m.cfg.channels, m.cfg.c_in
+    rows = 2**31 // (4 * C * shape[0] * shape[1]) + 9
+    g = torch.Generator(DEV).manual_seed(8)
+    x = torch.randn((rows, C, *shape), generator=g, device=DEV) * 0.3
+    given4 = torch.rand((rows, 1, *shape), generator=g, device=DEV) < 0.3
+    clamp = torch.randn((rows, c_in, *shape), generator=g, device=DEV)
+    masks = (torch.rand((2, rows, 1, *shape), generator=g, device=DEV) < 0.6).to(torch.uint8)
+    fire = masks[0].float() * 0.5
+    noise = torch.randn((rows, C, *shape), generator=g, device=DEV)
+    step = make_step(m)
+    parts = [slice(0, 2), slice(rows // 2 - 1, rows // 2 + 2), slice(rows - 3, rows)]
+    with torch.no_grad():
+        for n in (1, 2):
+            for kw in (dict(p_fire=0.8, p_low=0.2, tau=0.6), dict(masks=masks[:n])):
+                y, conf, fired = rollout_steps(m, x, given4, clamp, n, seed=5, want_fired=True, **kw)
+                for s in parts:
+                    ks = dict(masks=masks[:n, s]) if "masks" in kw else dict(kw, row0=s.start)
+                    ys, cs, fs = rollout_steps(m, x[s], given4[s], clamp[s], n, seed=5, want_fired=True, **ks)
+                    assert torch.equal(y[s], ys) and torch.equal(conf[s], cs) and torch.equal(fired[s], fs)
+        y = step(x, given4, clamp, fire, noise)
+        for s in parts:
+            assert torch.equal(y[s], step(x[s], given4[s], clamp[s], fire[s], noise[s]))
