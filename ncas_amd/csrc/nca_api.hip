@@ -487,9 +487,14 @@ int launch_rollout(nca::RolloutParams p, hipStream_t st) {
 // does or does not, whatever its steps and rows, so that fused rollouts equal chained steps, and a row
 // alone the same row among others, bit for bit. Boards that fit neither their LDS plan nor, one by one,
 // the 31-bit offsets of their per-step kernel, and the few that fit only the generic resident kernel's
-// plan (which needs no workspace), stay there.
+// plan (which needs no workspace), stay there. So do boards of at most 16 cells, one tile of the generic
+// kernel, which splits it over its waves and holds the weights in registers: up to 256 boards take 2.4 to 2.9 us
+// a step there and 3.4 here (C = 16), 5.4 to 6.0 and 6.0 to 7.0 (C = 32), 9.0 to 9.7 and 10.2 to 11.7 (C = 64);
+// 4,096 boards of 4x4 22, 88 and 120 us there and 9, 33 and 82 here.
+constexpr int kGenericCells = 16;
 bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
     if (g_path != 0 || g_window_steps > 1 || d->precision != NCA_FP32 || d->channels != 16 || d->hidden != 128) return false;
+    if (H * W <= kGenericCells) return false;
     if (nca::split16_resident_fits(H, W, d->c_out, d->n_out)) return true;
     return !takes_resident(d, rows, H, W) && nca::split16_step_fits(H, W);
 }
@@ -499,6 +504,7 @@ bool takes_split16(const nca_cell_desc *d, int64_t rows, int H, int W) {
 // stay there.
 bool takes_split_wide(const nca_cell_desc *d, int64_t rows, int H, int W) {
     if (g_path != 0 || d->precision != NCA_FP32 || d->hidden != 256 || (d->channels != 32 && d->channels != 64)) return false;
+    if (H * W <= kGenericCells) return false;
     if (nca::split_wide_resident_fits(d->channels, H, W, d->c_out, d->n_out)) return true;
     return !takes_resident(d, rows, H, W) && nca::split_wide_step_fits(d->channels, H, W);
 }

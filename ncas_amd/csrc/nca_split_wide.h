@@ -3,8 +3,8 @@
 // C = 32), and the rollout of boards that fit the LDS in one launch.
 //
 // The weights' three parts (240 KB at C = 32, 480 KB at C = 64) fit neither LDS nor, beside the
-// accumulators, the registers: they stream from L2 and are shared by a pass of 96 cells. Each of 8
-// waves owns 32 hidden units of all 96 cells (three 32x32 accumulator tiles), so that a weight
+// accumulators, the registers: they stream from L2 and are shared by a pass of up to 96 cells. Each of 8
+// waves owns 32 hidden units of all its cells (three 32x32 accumulator tiles), so that a weight
 // fragment is loaded once per pass and workgroup and used for three products, and its loads for
 // the k-step after next are issued as a step's are used. Per interval of 64 features (16
 // channels, 4 kernels) and one barrier, the waves multiply one half of Z (LDS, three parts) while
@@ -28,7 +28,7 @@
 namespace nca {
 
 constexpr int kSWT = 512;                       // threads per workgroup: 8 waves
-constexpr int kSWN = 96, kSWNT = 3;             // cells of a pass, 32-cell tiles
+constexpr int kSWN = 96, kSWNT = 3;             // most cells of a pass, 32-cell tiles
 constexpr int kSWStride = 98;                   // 16-byte units between Z's (quad, half) planes: 4 quads x
                                                 // 4 cells fall on distinct LDS slots
 constexpr unsigned kSWZ = 3u * 4u * 2u * kSWStride * 16u;  // bytes of one Z buffer: [part][quad][half][cell]
@@ -54,8 +54,11 @@ __device__ __forceinline__ f32x16 mfma32(uint4 a, uint4 b, f32x16 c) {
 
 // GLOBAL: one step, the state in global memory (cell-major, or the caller's NCHW); otherwise R rows'
 // whole rollout in LDS, the state twice (a step reads one, writes the other), with a one-cell border.
-template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW>
+// A pass takes NT tiles: a workgroup with few cells would spend a pass of three on nothing (their
+// cells' bits are the same in every form).
+template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW, int NT>
 __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
+    constexpr int PN = 32 * NT;  // cells of a pass
     constexpr int HD = 256, KS = C / 16, MT = C / 32, NQ = C / 4, CP = C + 4;
     constexpr int NTR = 64 / C;  // 32-cell tiles of a reduction round: 512 (cell, quad) items
     const RolloutParams &a = sp.a;
@@ -66,7 +69,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     float *fireG = b1L + HD;                                // GLOBAL: fire factors of the pass's cells
     // the cells of each 32-cell tile with a NaN among their sums, a bit each, for even and odd passes: a
     // pass clears the other's after its first barrier, when every wave is past the last look at them
-    int *badL = reinterpret_cast<int *>(fireG + kSWN), *bad = badL;
+    int *badL = reinterpret_cast<int *>(fireG + PN), *bad = badL;
     f32x4 *kernL = reinterpret_cast<f32x4 *>(badL + 8);      // the 4 kernels' weights of each tap
     const int tid = threadIdx.x, lane = tid & 63, n = lane & 31, hf = lane >> 5;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -147,7 +150,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     // the stencil item of a thread: cell sc, quad sq of an interval's 4. Quads fastest for global loads
     // (64 bytes of a cell), cells fastest for LDS taps (an odd stride of 16-byte slots). Waves 6 and 7
     // repeat waves 0 and 1's: a branch here doubles the intervals' code and spills the accumulators.
-    const int sid = tid < 4 * kSWN ? tid : tid - 4 * kSWN;
+    const int sid = tid % (4 * PN);
     const int sc = GLOBAL ? sid >> 2 : 16 * (sid >> 6) + (sid & 15), sq = GLOBAL ? sid & 3 : (sid >> 4) & 3;
     auto put_half = [&](const float z[4][4], int h, int buf) __attribute__((always_inline)) {
         uint4 *zp = reinterpret_cast<uint4 *>(Zb + buf * kSWZ) + (2 * sq + h) * kSWStride + sc;
@@ -188,19 +191,19 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     };
     Split8 af[2] = {frag(wA, 0), frag(wA, 1)};
 
-    // ---- one pass: cells [g0, g0 + 96) of step s (its index in the call)
+    // ---- one pass: cells [g0, g0 + 32 NT) of step s (its index in the call)
     const float4 b2v = reinterpret_cast<const float4 *>(a.packed + a.off_b2)[tid / (32 * NTR)];
     // GLOBAL: waves 6 and 7 draw the fire factors of the pass's cells. What they read is touched an
     // interval earlier.
     auto warm_fire = [&](int g0) __attribute__((always_inline)) {
-        const int k = tid & 127, gc = k < kSWN && g0 + k < ncell ? g0 + k : g0;
+        const int k = tid & 127, gc = k < PN && g0 + k < ncell ? g0 + k : g0;
         float v = (float)a.given[gc];
         if (a.adaptive && !IN_NCHW) v += a.x_in[(int64_t)gc * C + a.out_off];
         return v;
     };
     auto draw_pass = [&](int g0) __attribute__((always_inline)) {
         const int k = tid - 384, gq = g0 + k;
-        const bool live = k < kSWN && gq < ncell;
+        const bool live = k < PN && gq < ncell;
         const int gc = live ? gq : g0, row = (int)((unsigned)gc / (unsigned)HWn), q = gc - row * HWn;
         float f;
         if (a.fire_f32) {
@@ -223,7 +226,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             }
             f = u < p ? 1.0f : 0.0f;
         }
-        if (k < kSWN) fireG[k] = f;
+        if (k < PN) fireG[k] = f;
         if (a.fired_out) {
             // one addition per row of the wave's cells
             uint64_t rest = __ballot(live && f != 0.0f);
@@ -236,7 +239,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         }
     };
     auto pass = [&](int g0, int g0_next, int s, bool first, Pos &pos) __attribute__((always_inline)) {
-        f32x16 big[kSWNT], small[kSWNT];
+        f32x16 big[NT], small[NT];
         auto bias = [&]() __attribute__((always_inline)) {
             f32x16 r;
 #pragma unroll
@@ -248,7 +251,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         };
         const f32x16 b1v = bias();
 #pragma unroll
-        for (int t = 0; t < kSWNT; ++t) {
+        for (int t = 0; t < NT; ++t) {
             big[t] = b1v;
             small[t] = f32x16{};
         }
@@ -261,13 +264,13 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         auto interval = [&](int i, const Pos &ps, int cq, int next, auto with_stencil) __attribute__((always_inline)) {
             constexpr bool ST = decltype(with_stencil)::value;
             const uint4 *zb = reinterpret_cast<const uint4 *>(Zb + (i & 1) * kSWZ) + hf * kSWStride + n;
-            uint4 v[3][kSWNT];
+            uint4 v[3][NT];
             constexpr int NTP = GLOBAL ? 9 : 4;
             f32x4 tp[NTP], pq;
             float z[4][4];
             auto load_v = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
-                for (int t = 0; t < kSWNT; ++t) v[st % 3][t] = zb[((2 - st % 3) * 8 + 2 * (st / 3)) * kSWStride + 32 * t];
+                for (int t = 0; t < NT; ++t) v[st % 3][t] = zb[((2 - st % 3) * 8 + 2 * (st / 3)) * kSWStride + 32 * t];
             };
             load_v(0);
             load_v(1);
@@ -284,7 +287,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                 }
                 const Split8 &wf = af[j & 1];
 #pragma unroll
-                for (int t = 0; t < kSWNT; ++t) {
+                for (int t = 0; t < NT; ++t) {
                     if (st % 3 == 2)
                         big[t] = mfma32(wf.h, v[2][t], big[t]);
                     else
@@ -292,11 +295,11 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                 }
                 if (st % 3 >= 1) {
 #pragma unroll
-                    for (int t = 0; t < kSWNT; ++t) small[t] = mfma32(wf.m, v[st % 3][t], small[t]);
+                    for (int t = 0; t < NT; ++t) small[t] = mfma32(wf.m, v[st % 3][t], small[t]);
                 }
                 if (st % 3 == 2) {
 #pragma unroll
-                    for (int t = 0; t < kSWNT; ++t) small[t] = mfma32(wf.l, v[2][t], small[t]);
+                    for (int t = 0; t < NT; ++t) small[t] = mfma32(wf.l, v[2][t], small[t]);
                     af[j & 1] = frag(wA, j < 2 ? 4 * i + j + 2 : 4 * next + j - 2);
                 }
                 if constexpr (ST) {
@@ -325,7 +328,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
 
         // ---- fc2 and the update, a round of NTR 32-cell tiles after another: the partial sums of a
         // round meet in RED between two barriers; a round's update runs beside the next one's products
-        constexpr int RC = 32 * NTR, NR = (kSWNT + NTR - 1) / NTR;
+        constexpr int RC = 32 * NTR, NR = (NT + NTR - 1) / NTR;
         const int ic = tid % RC, iq = tid / RC;  // this thread's item of a round: cell, channel quad
         Split8 wf[MT][2];
         bool nanh[2][NTR];
@@ -338,7 +341,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
 #pragma unroll
             for (int tr = 0; tr < NTR; ++tr) {
                 const int t = rd * NTR + tr;
-                if (t >= kSWNT) break;
+                if (t >= NT) break;
                 const f32x16 h = big[t] + small[t];
                 bool nan = false;
 #pragma unroll
@@ -366,7 +369,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                     for (int tr = 0; tr < NTR; ++tr)
 #pragma unroll
                         for (int mt = 0; mt < MT; ++mt)
-                            if (rd * NTR + tr < kSWNT)
+                            if (rd * NTR + tr < NT)
                                 part[tr][mt] = mfma32(wf[mt][j].*pw, hs[rd & 1][tr][j].*ph, part[tr][mt]);
             };
             add(&Split8::l, &Split8::h);
@@ -380,7 +383,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         auto mark = [&](int rd) __attribute__((always_inline)) {
 #pragma unroll
             for (int tr = 0; tr < NTR; ++tr) {
-                if (rd * NTR + tr >= kSWNT) break;
+                if (rd * NTR + tr >= NT) break;
                 const uint64_t m = __ballot(nanh[rd & 1][tr]);
                 if (m && lane == 0) atomicOr(&bad[rd * NTR + tr], (int)(m | m >> 32));
             }
@@ -421,7 +424,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         };
         auto finish = [&](int t0, f32x4 u, int gv, float f, bool nan, bool again) __attribute__((always_inline)) {
             const int k = 32 * t0 + ic, gq = g0 + k;
-            bool live = gq < ncell && k < kSWN;
+            bool live = gq < ncell && k < PN;
             const int gc = live ? gq : g0;
             if (again) {
                 live = live && ((bad[t0 + (ic >> 5)] >> (ic & 31)) & 1);
@@ -429,7 +432,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
                 // a wave's lanes are the round's 64 cells, or two quads of its 32
                 if (NTR > 1) {
                     atomicOr(&bad[t0], (int)m);
-                    if (t0 + 1 < kSWNT) atomicOr(&bad[t0 + 1], (int)(m >> 32));
+                    if (t0 + 1 < NT) atomicOr(&bad[t0 + 1], (int)(m >> 32));
                 } else {
                     atomicOr(&bad[t0], (int)(m | m >> 32));
                 }
@@ -463,7 +466,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         // what the update of this thread's item reads besides
         auto load_item = [&](int t0, f32x4 &xo, int &gv, float &f) __attribute__((always_inline)) {
             const int k = 32 * t0 + ic, gq = g0 + k;
-            const bool live = gq < ncell && k < kSWN;
+            const bool live = gq < ncell && k < PN;
             const int gc = live ? gq : g0;
             if constexpr (GLOBAL) {
                 if (IN_NCHW) {
@@ -485,7 +488,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         // marked cells take
         auto redo = [&](int t0) {
             const int k = 32 * t0 + ic, gq = g0 + k;
-            const int gc = gq < ncell && k < kSWN ? gq : g0;
+            const int gc = gq < ncell && k < PN ? gq : g0;
             float *zf = reinterpret_cast<float *>(RED);
             const float *w1f = reinterpret_cast<const float *>(a.packed + a.off_w1);
             const float *w2f = reinterpret_cast<const float *>(a.packed + a.off_w2);
@@ -558,7 +561,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             for (int tr = 0; tr < NTR; ++tr)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    if (t0 + tr < kSWNT) put_part(tr, mt, part[tr][mt]);
+                    if (t0 + tr < NT) put_part(tr, mt, part[tr][mt]);
             if constexpr (!GLOBAL) load_item(t0, xo[rd], gv[rd], f[rd]);
             __syncthreads();
             f32x4 u;
@@ -572,7 +575,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
             finish(t0, u, gv[rd], f[rd], nan, false);
             __syncthreads();
             bool any = bad[t0] != 0;
-            if (NTR > 1 && t0 + 1 < kSWNT) any |= bad[t0 + 1] != 0;
+            if (NTR > 1 && t0 + 1 < NT) any |= bad[t0 + 1] != 0;
             if (__builtin_amdgcn_readfirstlane(any)) redo(t0);
         }
         bad = bad == badL ? badL + 4 : badL;
@@ -581,12 +584,12 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
     if constexpr (GLOBAL) {
         const int t_begin = (int)blockIdx.x * sp.tiles_per_wg;
         const int t_end = t_begin + sp.tiles_per_wg < sp.n_tiles ? t_begin + sp.tiles_per_wg : sp.n_tiles;
-        Pos pos = locate(t_begin * kSWN + sc);
+        Pos pos = locate(t_begin * PN + sc);
         put_z(pos);
         __syncthreads();
         for (int t = t_begin; t < t_end; ++t) {
-            const int g0 = t * kSWN;
-            pass(g0, t + 1 < t_end ? g0 + kSWN : g0, sp.step, sp.first != 0, pos);
+            const int g0 = t * PN;
+            pass(g0, t + 1 < t_end ? g0 + PN : g0, sp.step, sp.first != 0, pos);
         }
     } else {
         // ---- the rows' state, given flags and cell table; the constant border
@@ -677,7 +680,7 @@ __global__ void __launch_bounds__(kSWT, 1) split_wide(SplitWide sp) {
         for (int s = 0; s < a.n_steps; ++s) {
             const bool more = s + 1 < a.n_steps;
 #pragma unroll 1
-            for (int g0 = 0; g0 < ncell; g0 += kSWN) {
+            for (int g0 = 0; g0 < ncell; g0 += PN) {
                 Pos pos = locate(g0 + sc);
                 put_z(pos);
                 if (g0 == 0 && more && !a.adaptive) draw_fire(s + 1, cur);

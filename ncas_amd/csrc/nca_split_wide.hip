@@ -46,13 +46,18 @@ int cu_count() {
     return n;
 }
 
-template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW>
+template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW, int NT>
 hipError_t launch(const SplitWide &sp, unsigned grid, hipStream_t st) {
-    auto k = split_wide<C, GLOBAL, IN_NCHW, OUT_NCHW>;
+    auto k = split_wide<C, GLOBAL, IN_NCHW, OUT_NCHW, NT>;
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)sp.total);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k, dim3(grid), dim3(kSWT), sp.total, st, sp);
     return hipGetLastError();
+}
+
+template <int NT>
+hipError_t launch_rollout(int C, const SplitWide &sp, unsigned grid, hipStream_t st) {
+    return C == 32 ? launch<32, false, true, true, NT>(sp, grid, st) : launch<64, false, true, true, NT>(sp, grid, st);
 }
 
 }  // namespace
@@ -70,20 +75,26 @@ bool split_wide_step_fits(int C, int H, int W) {
 hipError_t split_wide_rollout(int C, const RolloutParams &p, hipStream_t st) {
     SplitWide sp;
     memset(&sp, 0, sizeof(sp));
-    // the rows per workgroup with the fewest passes of 96 cells one after another on a CU
+    // the rows per workgroup and 32-cell tiles per pass with the least time on a CU: passes one after
+    // another, of 6.2, 8.2 and 10.7 us (C = 32) or 10.7, 14.6 and 18.8 us (C = 64) for 1, 2 and 3 tiles. With
+    // passes of 96 cells for every board, up to 256 boards of 5x5 took 10.8 and 18.8 us a step
+    // where the fp32 MFMA kernel takes 10.0 and 16.8; 4,096 of 7x7 (C = 64) 320 where passes of 64 take 247.
     static const int n_cu = cu_count();
-    int best = 0;
+    int best = 0, nt = 0;
     int64_t cost = 0;
     for (int R = 1; R <= 16 && wide_plan(C, R, p.H, p.W, p.c_out, p.n_out, &sp); ++R) {
-        const int64_t wgs = (p.rows + R - 1) / R;
-        const int64_t c = ((wgs + n_cu - 1) / n_cu) * (((int64_t)R * p.H * p.W + kSWN - 1) / kSWN);
-        if (!best || c < cost) best = R, cost = c;
+        const int64_t wgs = (p.rows + R - 1) / R, cells = (int64_t)R * p.H * p.W;
+        for (int t = kSWNT; t >= 1; --t) {
+            const int64_t c = ((wgs + n_cu - 1) / n_cu) * ((cells + 32 * t - 1) / (32 * t)) * (4 + 2 * t);
+            if (!best || c < cost) best = R, nt = t, cost = c;
+        }
     }
     if (!best || !wide_plan(C, best, p.H, p.W, p.c_out, p.n_out, &sp)) return hipErrorInvalidValue;
     sp.a = p;
     sp.wsplit = p.packed + p.off_split;
     const unsigned grid = (unsigned)((p.rows + best - 1) / best);
-    return C == 32 ? launch<32, false, true, true>(sp, grid, st) : launch<64, false, true, true>(sp, grid, st);
+    if (nt == 1) return launch_rollout<1>(C, sp, grid, st);
+    return nt == 2 ? launch_rollout<2>(C, sp, grid, st) : launch_rollout<3>(C, sp, grid, st);
 }
 
 hipError_t split_wide_step(const RolloutParams &p, int step, int first, int in_nchw, int out_nchw, hipStream_t st) {
@@ -104,8 +115,9 @@ hipError_t split_wide_step(const RolloutParams &p, int step, int first, int in_n
         sp.n_tiles = (sp.n_cells + kSWN - 1) / kSWN;
         sp.tiles_per_wg = (sp.n_tiles + n_cu - 1) / n_cu;
         const unsigned grid = (unsigned)((sp.n_tiles + sp.tiles_per_wg - 1) / sp.tiles_per_wg);
-        const hipError_t e = in_nchw ? (out_nchw ? launch<32, true, true, true>(sp, grid, st) : launch<32, true, true, false>(sp, grid, st))
-                                     : (out_nchw ? launch<32, true, false, true>(sp, grid, st) : launch<32, true, false, false>(sp, grid, st));
+        const hipError_t e =
+            in_nchw ? (out_nchw ? launch<32, true, true, true, kSWNT>(sp, grid, st) : launch<32, true, true, false, kSWNT>(sp, grid, st))
+                    : (out_nchw ? launch<32, true, false, true, kSWNT>(sp, grid, st) : launch<32, true, false, false, kSWNT>(sp, grid, st));
         if (e != hipSuccess) return e;
     }
     return hipSuccess;

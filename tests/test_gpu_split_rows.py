@@ -74,3 +74,27 @@ def test_rows_beyond_2_gib(name, shape):
         y = step(x, given4, clamp, fire, noise)
         for s in parts:
             assert torch.equal(y[s], step(x[s], given4[s], clamp[s], fire[s], noise[s]))
+
+
+@pytest.mark.parametrize("name", ["maze_c16", "maze_hard_c32", "sudoku_c64"])
+@pytest.mark.parametrize("shape", [(1, 1), (4, 4), (1, 17), (5, 6), (4, 8), (3, 11), (7, 7), (8, 8), (5, 13), (9, 9)])
+@pytest.mark.parametrize("rows", [3, 515])
+def test_a_row_alone_is_the_row_among_others(name, shape, rows):
+    """Boards about the sizes where the kernel (16 cells) and the cells of a pass (32, 64) change: a row's bits
+    are the same alone, among others, and step by step, with and without the outputs that decide
+    where a single step runs."""
+    m, md, x, g4, cl = _state(name, rows, shape, 4)
+    kw = dict(p_fire=0.8, p_low=0.2, tau=0.6)
+    y, conf, fired = _run(md, x, g4, cl, 3, **kw)
+    for r in (0, rows - 1):
+        with torch.no_grad():
+            yr, cr, fr = rollout_steps(md, x[r:r + 1].to(DEV), g4[r:r + 1].to(DEV), cl[r:r + 1].to(DEV), 3, seed=5,
+                                       row0=3 + r, want_fired=True, **kw)
+        assert torch.equal(y[r:r + 1], yr) and torch.equal(conf[r:r + 1], cr) and torch.equal(fired[r:r + 1], fr)
+    for outputs in (False, True):
+        cur = x.to(DEV)
+        for t in range(3):
+            with torch.no_grad():
+                cur, _, _ = rollout_steps(md, cur, g4.to(DEV), cl.to(DEV), 1, seed=5, row0=3, step0=t, want_conf=outputs,
+                                          want_fired=outputs, **kw)
+        assert torch.equal(y, cur)
