@@ -660,10 +660,14 @@ int launch_cell(const nca_cell_desc *d, const nca::RolloutParams &p, hipStream_t
     }
     if (takes_split16(d, p.rows, p.H, p.W) || takes_split_wide(d, p.rows, p.H, p.W)) {
         // one step on the per-step kernel, whose tiles spread over the whole device (out of place: in
-        // place it would need a workspace); more of them in LDS where the boards fit
+        // place it would need a workspace); more of them in LDS where the boards fit. One step with a board
+        // confidence or fired counts too where a workgroup's rows are one tile per wave (C = 16) or one
+        // pass: these are launches of their own beside the per-step kernel (8 boards of 9x9, C = 16: 30 us a
+        // call against 25)
         const size_t sb = state_bytes(d, p.rows, p.H, p.W);
         const bool fits = C == 16 ? nca::split16_step_fits(p.H, p.W) : nca::split_wide_step_fits(C, p.H, p.W);
-        const bool one = p.n_steps == 1 && fits && !overlaps(p.x_in, sb, p.x_out, sb);
+        const bool small = (p.rows + 255) / 256 * p.H * p.W <= (C == 16 ? 256 : 96);
+        const bool one = p.n_steps == 1 && fits && !overlaps(p.x_in, sb, p.x_out, sb) && !(small && (p.conf_out || p.fired_out));
         if (one || !split_resident(d, p.rows, p.H, p.W)) return run_tiled(d, p, st, ws, ws_bytes);
         return hip_check(split_rollout(C, p, st), "split rollout launch");
     }
