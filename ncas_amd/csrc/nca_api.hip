@@ -308,7 +308,11 @@ __global__ void fire_mask_kernel(int64_t rows, int hw, uint64_t seed, int64_t ro
 
 // ------------------------------------------------------------------------------------------
 // Readout: one workgroup per row, cells in chunks of the workgroup size; the board sum runs in
-// cell order (ordered_sum) so that its rounding matches the sequential definition.
+// cell order so that its rounding matches the sequential definition. A small sum soon leaves
+// its binade, so that ordered_sum's blocks fail and are added one by one after all: up to
+// kOrderedSumFrom the values are added from the LDS (boards of 13x13: 4.1 us, 6.9 to 7.9 with ordered_sum
+// from the start; 20x20 7.4, 11.0 to 12.6).
+constexpr float kOrderedSumFrom = 256.0f;
 __global__ void readout_kernel(const float *x, int C, int hw, int out_off, int c_out, int n_out,
                                int head_kind, const float *headw, const float *headb,
                                float *conf_cell, float *conf_board, int32_t *argmax) {
@@ -326,7 +330,14 @@ __global__ void readout_kernel(const float *x, int C, int hw, int out_off, int c
             chunk[threadIdx.x] = cf;
         }
         __syncthreads();
-        if (threadIdx.x < 64) sum = nca::ordered_sum(sum, chunk, hw - base < 256 ? hw - base : 256);
+        if (threadIdx.x < 64) {
+            const int n = hw - base < 256 ? hw - base : 256;
+            if (sum >= kOrderedSumFrom) {
+                sum = nca::ordered_sum(sum, chunk, n);
+            } else {
+                for (int i = 0; i < n; ++i) sum = __fadd_rn(sum, chunk[i]);
+            }
+        }
         __syncthreads();
     }
     if (threadIdx.x == 0 && conf_board) conf_board[r] = __fdiv_rn(sum, (float)hw);
@@ -334,18 +345,17 @@ __global__ void readout_kernel(const float *x, int C, int hw, int out_off, int c
 
 // The readout of large boards in two launches: every cell on the whole device, then one wave per
 // board that adds the cells' confidences in order. One workgroup per row leaves all but `rows` of
-// the CUs idle (16 boards of 201x201: 662 us with the sum on one lane of it, 9 + 69 us in two launches).
-__global__ void readout_cells_kernel(const float *x, int64_t rows, int C, int hw, int out_off, int c_out, int n_out,
+// the CUs idle (16 boards of 201x201: 580 us, 67 us in two launches).
+__global__ void readout_cells_kernel(const float *x, int C, int hw, int out_off, int c_out, int n_out,
                                      int head_kind, const float *headw, const float *headb, float *conf_cell,
                                      int32_t *argmax) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= hw) return;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-        int am;
-        const float cf = nca::cell_readout(x + (r * C + out_off) * (int64_t)hw + q, hw, c_out, n_out, head_kind, headw, headb, &am);
-        conf_cell[r * hw + q] = cf;
-        if (argmax) argmax[r * hw + q] = am;
-    }
+    const int64_t r = blockIdx.y;
+    int am;
+    const float cf = nca::cell_readout(x + (r * C + out_off) * (int64_t)hw + q, hw, c_out, n_out, head_kind, headw, headb, &am);
+    conf_cell[r * hw + q] = cf;
+    if (argmax) argmax[r * hw + q] = am;
 }
 
 __global__ void board_mean_kernel(const float *conf_cell, int hw, float *conf_board) {
@@ -356,16 +366,18 @@ __global__ void board_mean_kernel(const float *conf_cell, int hw, float *conf_bo
 
 // Boards of at least this many cells take two launches where the cells' confidences have a buffer
 // (the caller's, or the per-step path's workspace); below it a row is a few passes of one
-// workgroup and a second launch costs more than it saves.
-constexpr int kReadoutSplit = 2048;
+// workgroup and a second launch costs more than it saves. So it does from about 1,024 rows, whose
+// workgroups fill the device: 46x46, C = 64, 512 rows 299 us in one launch and 220 in two, 1,024 rows 333
+// and 399, 2,048 rows 781 and 814; C = 16, 2,048 rows 49 and 57.
+constexpr int kReadoutSplit = 2048, kReadoutSplitRows = 512;
 
 int launch_readout(hipStream_t st, int64_t rows, const float *x, int C, int hw, int out_off, int c_out, int n_out,
                    int head_kind, const float *headw, const float *headb, float *conf_cell, float *conf_board,
                    int32_t *argmax, float *conf_buf) {
     if (!conf_buf) conf_buf = conf_cell;
-    if (hw >= kReadoutSplit && conf_buf) {
-        hipLaunchKernelGGL(readout_cells_kernel, dim3((unsigned)((hw + 255) / 256), (unsigned)(rows < 65535 ? rows : 65535)),
-                           dim3(256), 0, st, x, rows, C, hw, out_off, c_out, n_out, head_kind, headw, headb, conf_buf, argmax);
+    if (hw >= kReadoutSplit && rows <= kReadoutSplitRows && conf_buf) {
+        hipLaunchKernelGGL(readout_cells_kernel, dim3((unsigned)((hw + 255) / 256), (unsigned)rows),
+                           dim3(256), 0, st, x, C, hw, out_off, c_out, n_out, head_kind, headw, headb, conf_buf, argmax);
         if (conf_board)
             hipLaunchKernelGGL(board_mean_kernel, dim3((unsigned)rows), dim3(64), 0, st, conf_buf, hw, conf_board);
     } else {

@@ -60,3 +60,18 @@ def test_rollout_confidence_equals_readout():
             for n in (1, 2, 3):
                 y, conf, _ = rollout_steps(m, x, given4, clamp, n, precision=precision)
                 assert torch.equal(conf, readout(m, y)[1])
+
+
+def test_many_rows_equal_few():
+    """Boards of several kilocells are read out in two launches or, from some hundred rows, in one: the
+    same bits."""
+    from ncas_amd.readout import readout
+
+    m = make_model("maze_c16").cuda()
+    g = torch.Generator("cuda").manual_seed(4)
+    x = torch.randn((515, 16, 46, 45), generator=g, device="cuda")
+    conf, board, cls = readout(m, x)
+    for r in (0, 514):
+        c1, b1, k1 = readout(m, x[r:r + 1])
+        assert torch.equal(conf[r:r + 1], c1) and torch.equal(board[r:r + 1], b1) and torch.equal(cls[r:r + 1], k1)
+    assert np.array_equal(board.cpu().numpy(), _sequential_mean(conf))
