@@ -362,7 +362,10 @@ typedef struct nca_bptt_loss {
     const float *step_weights;  /* host (n_chunk): loss weight of each chunk step */
 } nca_bptt_loss;
 
-/* Workspace bytes of nca_bptt_backward for this shape (0 if the cell is unsupported). */
+/* Workspace bytes of nca_bptt_backward for this shape (0 if the cell is unsupported). Cells outside the
+ * one-launch backward (bf16, C = 32) keep operands of several steps there, up to 160 MB or one step's, whichever is
+ * more; a workspace sized for fewer steps (n_chunk >= 1) is enough, with weight-gradient sums
+ * over fewer steps at a time. */
 size_t nca_bptt_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t height,
                                 int32_t width, int32_t n_chunk);
 

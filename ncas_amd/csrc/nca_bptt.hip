@@ -1214,6 +1214,14 @@ StepLayout step_layout(const Dims &d, int n) {
     return L;
 }
 
+// The layout of the longest groups that a workspace of `bytes` holds (groups of one step, which is the
+// least, if none does): any workspace that was sized for this shape serves, whatever its n_chunk.
+StepLayout step_layout_in(const Dims &d, int n, size_t bytes) {
+    StepLayout L = step_layout(d, n);
+    for (int g = L.group - 1; L.total > bytes && g >= 1; --g) L = step_layout(d, g);
+    return L;
+}
+
 size_t backward_ws_bytes(const Dims &d, int n) {
     return fused_mlp(d) ? (size_t)ws_layout(d, n).total * sizeof(float) : step_layout(d, n).total;
 }
@@ -1280,7 +1288,7 @@ int backward_steps(const Dims &d, const void *packed, const float *states, int64
                    const float *grad_final, nca_cell_grads *grads, float *grad_x0, float *loss_out, void *workspace,
                    size_t workspace_bytes, hipStream_t st) {
     int rc = NCA_OK;
-    const StepLayout L = step_layout(d, n_chunk);
+    const StepLayout L = step_layout_in(d, n_chunk, workspace_bytes);
     if (!workspace || workspace_bytes < L.total) return ws_error(L.total);
     float wsum = 0.0f;
     for (int t = 0; t < n_chunk; ++t) wsum += loss->step_weights[t];
