@@ -34,13 +34,6 @@ bool resident_plan(int R, int H, int W, int c_out, int n_out, Split16Resident *s
     return o <= kSplitLds;
 }
 
-int cu_count() {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 256;
-    return n;
-}
-
 template <bool IN_NCHW, bool OUT_NCHW>
 hipError_t launch_step(const Split16Step &sp, unsigned grid, int first, hipStream_t st) {
     auto k = first ? step_split16<IN_NCHW, OUT_NCHW, true> : step_split16<IN_NCHW, OUT_NCHW, false>;
@@ -85,7 +78,7 @@ hipError_t split16_step(const RolloutParams &p, int step, int first, int in_nchw
     sp.wsplit = p.packed + p.off_split;
     sp.step = step;
     sp.tiles_per_row = (p.H * p.W + 15) / 16;
-    static const int n_cu = cu_count();
+    const int n_cu = plan_cus();
     const int64_t per = step_launch_rows(16, p.rows, p.H, p.W);
     for (int64_t r0 = 0; r0 < p.rows; r0 += per) {
         sp.a = step_rows(p, 16, step, r0, p.rows - r0 < per ? p.rows - r0 : per);

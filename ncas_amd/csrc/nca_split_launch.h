@@ -7,6 +7,9 @@
 
 namespace nca {
 
+int device_cus();  // of the current device (nca_api.hip), 0 where it cannot be asked
+inline int plan_cus() { return device_cus() > 0 ? device_cus() : 256; }
+
 // C = 16, 128 hidden units. A row's rollout in LDS (also recorded: x_rec, x_rec0); one step of rows
 // of any size, x_in -> x_out (distinct buffers), in the caller's NCHW layout or cell-major. The step
 // kernels hold 31-bit byte offsets into the state: a launch takes as many rows as these reach, and

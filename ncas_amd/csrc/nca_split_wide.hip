@@ -39,13 +39,6 @@ bool wide_plan(int C, int R, int H, int W, int c_out, int n_out, SplitWide *sp) 
 }
 static_assert(2 * kSWZ >= kSWRed, "RED in Z's place");
 
-int cu_count() {
-    int dev = 0, n = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) return 256;
-    return n;
-}
-
 template <int C, bool GLOBAL, bool IN_NCHW, bool OUT_NCHW, int NT>
 hipError_t launch(const SplitWide &sp, unsigned grid, hipStream_t st) {
     auto k = split_wide<C, GLOBAL, IN_NCHW, OUT_NCHW, NT>;
@@ -79,7 +72,7 @@ hipError_t split_wide_rollout(int C, const RolloutParams &p, hipStream_t st) {
     // another, of 6.2, 8.2 and 10.7 us (C = 32) or 10.7, 14.6 and 18.8 us (C = 64) for 1, 2 and 3 tiles. With
     // passes of 96 cells for every board, up to 256 boards of 5x5 took 10.8 and 18.8 us a step
     // where the fp32 MFMA kernel takes 10.0 and 16.8; 4,096 of 7x7 (C = 64) 320 where passes of 64 take 247.
-    static const int n_cu = cu_count();
+    const int n_cu = plan_cus();
     int best = 0, nt = 0;
     int64_t cost = 0;
     for (int R = 1; R <= 16 && wide_plan(C, R, p.H, p.W, p.c_out, p.n_out, &sp); ++R) {
@@ -107,7 +100,7 @@ hipError_t split_wide_step(const RolloutParams &p, int step, int first, int in_n
     sp.l_red = 2 * kSWZ;
     sp.l_small = sp.l_red + kSWRed;
     sp.total = st_al16(sp.l_small + kSmallBytes);
-    static const int n_cu = cu_count();
+    const int n_cu = plan_cus();
     const int64_t per = step_launch_rows(32, p.rows, p.H, p.W);
     for (int64_t r0 = 0; r0 < p.rows; r0 += per) {
         sp.a = step_rows(p, 32, step, r0, p.rows - r0 < per ? p.rows - r0 : per);
