@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from ncas_amd import _lib
+from ncas_amd.step import step_vjp
 from oracle import nca_oracle as O
 from test_gpu_bptt import DEV, NAMES, _case, _gpu_chunk, _rel, oracle_cell
 
@@ -69,3 +70,28 @@ def test_many_cells_and_groups_match_oracle(name, precision, tol, monkeypatch):
         assert _rel(res.grads[k], ref[k]) <= tol, (k, _rel(res.grads[k], ref[k]))
     if precision == "fp32":
         assert _rel(res.grad_x0, ref["x0"]) <= tol
+
+
+def test_bf16_c32_beyond_32_bit_offsets():
+    """From 2^23 cells a bf16 C = 32 batch runs on back_step<32, 256, true>, as the fused MLP kernel holds 32-bit
+    offsets: the gradients of a step are those of the batch's two halves."""
+    m, md, x, g4, cl, masks, targets = _case("maze_hard_c32")
+    H = W = 30
+    rows = 2**23 // (H * W) + 3
+    g = torch.Generator(DEV).manual_seed(11)
+    x = torch.randn((rows, 32, H, W), generator=g, device=DEV) * 0.3
+    cot = torch.randn((rows, 32, H, W), generator=g, device=DEV)
+    given4 = torch.rand((rows, 1, H, W), generator=g, device=DEV) < 0.3
+    fire = (torch.rand((rows, 1, H, W), generator=g, device=DEV) < 0.6).float()
+    gx, gp = step_vjp(md, x, given4, fire, cot, "bf16")
+    half = rows // 2
+    a = step_vjp(md, x[:half], given4[:half], fire[:half], cot[:half], "bf16")
+    b = step_vjp(md, x[half:], given4[half:], fire[half:], cot[half:], "bf16")
+
+    def rel(p, q):  # (on the GPU: 3e8 values)
+        return float((p - q).norm() / q.norm())
+
+    # the same bf16 operands; a sum in another order rounds g_z to the neighbouring bf16 value now and then
+    assert rel(gx[:half], a[0]) <= 1e-3 and rel(gx[half:], b[0]) <= 1e-3
+    for k in range(5):
+        assert rel(gp[k], a[1][k] + b[1][k]) <= 1e-3, k

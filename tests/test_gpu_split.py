@@ -1,6 +1,7 @@
-"""fp32 cells on the bf16 matrix cores (nca_split.h): steps and rollouts against float64, where the
-error must not exceed that of the fp32 MFMA kernels on the same inputs, and against those kernels
-where a state holds infinities or NaN."""
+"""fp32 C = 16 cells on the bf16 matrix cores (nca_split.h): steps against float64, where the error of
+boards of any size must not exceed 1.4 times that of the fp32 MFMA kernels on the same inputs
+(test_gpu_split_lds.py: over many cells, that error itself), fused rollouts against chained
+steps, and infinities and NaN against those kernels."""
 
 import copy
 

@@ -1,6 +1,7 @@
 """fp32 cells with C = 32 and C = 64 on the bf16 matrix cores (nca_split_wide.h): steps against float64,
-where the error must not exceed that of the fp32 MFMA kernels on the same inputs, fused rollouts
-against chained steps, and infinities and NaN against those kernels."""
+where the error must not exceed 1.4 times that of the fp32 MFMA kernels on the same inputs, and over
+many cells that error itself, fused rollouts against chained steps, and infinities and NaN against
+those kernels."""
 
 import pytest
 import torch
