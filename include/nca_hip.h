@@ -146,17 +146,18 @@ int nca_rollout(const nca_cell_desc *cell, const void *packed, int64_t rows, int
 /* Bytes of workspace that nca_rollout_ws needs for this call shape: 0 when the rows fit the
  * LDS-resident kernels (the whole rollout runs in one launch; bf16 cells with C=32, hidden 256
  * on boards up to 31 wide, such as 30x30, run one board per workgroup), else two state buffers
- * (2 * rows * C * H * W * 4 bytes) for the halo-tiled per-step path. An in-place single step
- * with noise always takes the tiled path and then needs one state buffer. */
+ * (2 * rows * C * H * W * 4 bytes) for the per-step path. */
 size_t nca_rollout_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t height,
                                    int32_t width);
 
 /* nca_rollout with a caller-owned device workspace. Grids whose rows do not fit the resident
- * kernels run one halo-tiled launch per step: the first step reads x_in, the steps in between
+ * kernels run a launch per step: the first step reads x_in, the steps in between
  * keep the state in the workspace (cell-major, two buffers), the last writes x_out. They need
  * workspace_bytes >= nca_rollout_workspace_bytes (one state buffer suffices for n_steps == 2
  * or an in-place single step, none for an out-of-place single step). The workspace must not
- * overlap x_in or x_out. The arithmetic per cell is the generic resident kernel's (nca_set_kernel_path(1)). */
+ * overlap x_in or x_out. fp32 cells on boards of more than 16 cells run on the bf16 matrix cores with
+ * every operand in three bf16 parts (an error of fp32 chains' size or less; C = 64 only where a board
+ * fits the LDS), whatever the rows and the steps of the call; elsewhere the arithmetic per cell is the generic resident kernel's (nca_set_kernel_path(1)). */
 int nca_rollout_ws(const nca_cell_desc *cell, const void *packed, int64_t rows, int32_t height,
                    int32_t width, const float *x_in, const uint8_t *given, const float *clamp,
                    float *x_out, const nca_fire_desc *fire, int32_t n_steps, const float *noise,
@@ -370,8 +371,9 @@ size_t nca_bptt_workspace_bytes(const nca_cell_desc *cell, int64_t rows, int32_t
                                 int32_t width, int32_t n_chunk);
 
 /* Forward of a BPTT chunk: states (n_chunk + 1, rows, C, H, W) receives x0 and the state after
- * every step, equal to nca_rollout's states bit for bit (bf16 C=32 boards up to 31 wide: one
- * fused launch of the streamed kernel that records every step; other cells and grids: one call
+ * every step, equal to nca_rollout's states bit for bit (one launch that records every step for
+ * bf16 C=32 boards up to 31 wide and bf16 C=64 boards up to 15 wide on the streamed kernels and
+ * fp32 boards of more than 16 cells that fit the LDS; other cells and grids: one call
  * per step). fire->adaptive must be 0. States are all that the backward needs: it recomputes
  * everything else. */
 int nca_bptt_forward(const nca_cell_desc *cell, const void *packed, int64_t rows, int32_t height,
@@ -396,8 +398,8 @@ int nca_bptt_forward_ws(const nca_cell_desc *cell, const void *packed, int64_t r
                         size_t workspace_bytes, void *stream);
 
 /* Backward of the chunk whose forward wrote `states` (same cell, packed weights, fire desc).
- * w->w1 and w->w2 are the fp32 master weights (rounded to bf16 on load for bf16 cells, as the
- * forward used them). grad_final (rows, C, H, W), the gradient of a later loss w.r.t. the last
+ * w->w1 and w->w2 are the fp32 master weights of `packed` (bf16 cells with C=32 read them, rounded to bf16
+ * as the forward used them; other cells read `packed`). grad_final (rows, C, H, W), the gradient of a later loss w.r.t. the last
  * state, may be NULL (zero). Writes the parameter gradients of the chunk loss into `grads`
  * (overwritten, not accumulated), grad_x0 (rows, C, H, W; may be NULL), and the loss value into
  * loss_out (device scalar; may be NULL). Deterministic: every sum has a fixed order. */
@@ -417,8 +419,7 @@ size_t nca_step_backward_workspace_bytes(const nca_cell_desc *cell, int64_t rows
  * parameter gradients, overwritten) and grad_x (rows, C, H, W; may be NULL). fire (rows, H, W) fp32
  * is the step's fire value per cell (any real value: g_dx = g_u * fire); the noise and the clamp
  * values do not enter the gradient. grads->head_w / head_b are not written (the step does not use
- * the readout head). w->w1 and w->w2 are the fp32 weights (bf16 cells round them on load like the
- * forward). Any head kind. Deterministic. */
+ * the readout head). w->w1 and w->w2 as for nca_bptt_backward. Any head kind. Deterministic. */
 int nca_step_backward(const nca_cell_desc *cell, const void *packed, const nca_cell_weights *w,
                       int64_t rows, int32_t height, int32_t width, const float *x,
                       const uint8_t *given, const float *fire, const float *grad_out,
@@ -431,12 +432,14 @@ const char *nca_last_error(void);
 /* ABI version (major * 100 + minor). */
 int nca_version(void);
 
-/* Kernel selection: 0 = automatic (the streamed bf16 kernel where the grid allows it, the
+/* Kernel selection: 0 = automatic (the streamed bf16 kernels where the grid allows it, for fp32 boards of
+ * more than 16 cells the kernels on the bf16 matrix cores, the
  * resident kernel where the rows fit LDS, else the per-step path: the wave-per-tile kernel for
  * bf16 cells with 16 channels, the halo-window kernel for other cells; with
  * nca_set_window_steps(T >= 2), bf16 cells with 16 channels on the temporally blocked kernel, T
  * steps per launch on LDS-resident windows, for calls of two or more steps with uniform firing
- * and no noise), 1 = never the streamed kernel, 2 = always the per-step path with one step per
+ * and no noise), 1 = never the streamed kernels nor fp32 on the bf16 matrix cores (as with every path
+ * but 0), 2 = always the per-step path with one step per
  * launch, 3 = always the per-step path on the halo-window kernel, 4 = the temporally blocked
  * kernel wherever it applies (2 steps per launch unless set), also on grids the resident kernels
  * take. Per calling thread (other threads keep their own setting); used by the tests to check
@@ -466,9 +469,9 @@ int nca_set_piece_debug(int32_t spin_limit, int32_t force_timeout, int32_t plan_
 
 /* Test setting of nca_bptt_backward's path: 0 automatic (bf16 cells of 32 channels, 128 features
  * and 256 hidden units run the chunk's whole backward as one launch, on pieces of boards where
- * the device holds them, else on whole boards; other cells, three launches per step), 1 three
- * launches per step, 2 the one-launch backward on whole boards. The gradients of the paths agree
- * to fp32 rounding. No counterpart in the reference. */
+ * the device holds them, else on whole boards), 1 three launches per step for these cells, 2 the
+ * one-launch backward on whole boards. Other cells run one launch per step and one per group of steps
+ * with every setting. The gradients of the paths agree to fp32 rounding. No counterpart in the reference. */
 int nca_set_bptt_backward_path(int32_t path);
 
 #ifdef __cplusplus

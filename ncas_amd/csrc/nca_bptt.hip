@@ -23,8 +23,10 @@
 //
 // Every partial sum belongs to one of 256 fixed cell ranges (slots); each step adds its sums
 // into the slots, and one kernel adds the slots up in slot order after the last step, so the
-// gradients are deterministic (the same bits on every run). fp32 cells: the exact fp32
-// gradients of the forward as computed. bf16 cells: the rounding points are straight-through
+// gradients are deterministic (the same bits on every run). fp32 cells: fp32 gradients; h is
+// recomputed in fp32 chains of its own, so a hidden unit whose input lies within an fp32 rounding of
+// zero may pass the gradient where the forward's sums (nca_split.h) have it at zero, or not pass
+// it where they have it above. bf16 cells: the rounding points are straight-through
 // (derivative 1), the backward uses the forward's bf16-rounded weights and inputs, and the
 // gradients of dx, of fc1's output and of z are rounded to bf16 where the reference's bf16
 // backward rounds them (they are gradients of bf16 tensors; src/nca/engine/triton_mlp.py:46-78),

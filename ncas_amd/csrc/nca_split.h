@@ -12,7 +12,8 @@
 // not, but its 32-cell tiles leave 8 waves per CU, and their waits cost what it saves: 201x201
 // steps 98 us in both forms, 13x13 rollouts 2.40 ms against 1.87.)
 //
-// The exponent range is fp32's. A value that rounds to an infinite h (or is infinite or NaN) makes
+// The exponent range is fp32's, but parts below bf16's least value, 2^-133, are lost: values below 2^-109
+// keep fewer than 24 bits. A value that rounds to an infinite h (or is infinite or NaN) makes
 // m or l NaN, hence every output of its cell: a tile with a NaN among fc1's or fc2's sums is
 // computed again on fp32 MFMA (a branch uniform over the wave), and the cells with a NaN of their
 // own take that result, so infinities and NaN come out as they do there. An MFMA's columns

@@ -141,7 +141,7 @@ def bptt_chunk(model, x, given4, clamp, targets, weights, *, seed: int = 0, step
                                      xs.data_ptr(), g8.data_ptr(), cl.data_ptr(), ctypes.byref(fd),
                                      n, states.data_ptr(), ws.data_ptr(), ws_bytes, stream),
                "nca_bptt_forward_ws")
-    # fp32 master weights for the backward GEMMs (rounded to bf16 on load for bf16 cells)
+    # fp32 master weights (the bf16 C = 32 backward reads them; other cells' reads the packed ones)
     params = _params(model)
     master = [p.detach().to(dev, torch.float32).contiguous() for p in params]
     wts = _lib.CellWeights(*[m.data_ptr() for m in master], None)

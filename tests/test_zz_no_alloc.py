@@ -1,7 +1,7 @@
 """The allocation-free entry point nca_rollout_noalloc, through the C ABI, on the GPU: its results
 equal nca_rollout_ws's (the same call with a caller workspace) bit for bit - states, board
 confidences and fired counts - on two calls in a row, the second with a smaller input, on the
-per-step path (201x201 mazes, bf16 wave-per-tile kernel and fp32 halo-window kernel, an
+per-step path (201x201 mazes, bf16 and fp32, an
 in-place single step) and on a resident-kernel grid; a call whose workspace would exceed the
 scratch is refused with NCA_ERR_UNSUPPORTED before anything runs."""
 
