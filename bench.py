@@ -32,7 +32,8 @@ skips it.
 
 value = rows * H * W * D * steps / wall seconds (cell-updates/s). The roofline block prices the
 rollout kernel's algorithmic FLOPs (2 * (36 C + F * hidden + hidden * C) per cell-update, the
-reference's count_step_flops convention) against the MI355X dense MFMA peak of the compute type,
+reference's count_step_flops convention) against the MI355X dense MFMA peak of the compute type
+(fp32: a sixth of the bf16 peak, as its kernels take six bf16 products for one of fp32),
 or, for the per-step path (maze201) when it is lower, its algorithmic HBM bytes (the fp32 state read and
 written once per step plus the given mask: 8 C + 1 bytes per cell-update) against 8 TB/s. The
 kernel time comes from HIP events recorded on the launch stream around every rollout call. The
@@ -54,7 +55,10 @@ import torch
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 157.3}
+# fp32 rollouts run on the bf16 matrix cores, six bf16 products for one of fp32 (nca_split.h)
+PEAK_TFLOPS = {"bf16": 2500.0, "fp32": 2500.0 / 6}
+PEAK_OF = {"bf16": "bf16 MFMA", "fp32": "bf16 MFMA, six products for one of fp32"}
+FP32_MFMA_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
 
 WORKLOADS = {
@@ -370,7 +374,8 @@ def roofline(name, wl, precision, res):
     flops = flop_per_cell_update(wl["preset"])
     mfma_ceiling = PEAK_TFLOPS[precision] * 1e12 / flops
     block = {"bound": "mfma", "achieved": res["achieved_tflops"], "peak": PEAK_TFLOPS[precision],
-             "unit": "TFLOP/s", "frac": res["frac"], "traffic": traffic_from_profiles(name, precision)}
+             "peak_of": PEAK_OF[precision], "unit": "TFLOP/s", "frac": res["frac"],
+             "traffic": traffic_from_profiles(name, precision)}
     ceilings = {"unit": "cell-updates/s", "mfma": mfma_ceiling, "lds": None, "hbm": None}
     if name == "sudoku9" and precision == "bf16":
         ceilings["lds"] = N_CU * CLOCK_HZ / LDS_CYCLES_PER_CELL_STREAM64
@@ -380,7 +385,7 @@ def roofline(name, wl, precision, res):
         ceilings["hbm"] = hbm_ceiling
         if hbm_ceiling < mfma_ceiling:
             gbs = res["kernel_rate"] * nbytes / 1e9
-            block.update(bound="hbm", achieved=gbs, peak=PEAK_HBM_GBS, unit="GB/s",
+            block.update(bound="hbm", achieved=gbs, peak=PEAK_HBM_GBS, peak_of="HBM", unit="GB/s",
                          frac=gbs / PEAK_HBM_GBS)
     elif block["traffic"]:
         # the resident kernels touch HBM once per launch: the measured bytes per cell-update
@@ -404,6 +409,8 @@ def bptt_entry(wl, precision, steps, warmup, cpu_budget=None):
     of 4x the forward FLOPs per cell-step against the dense MFMA peak of the chunk's compute type
     (fp32 peak beside it), the peak activation memory and the CPU oracle's chunk."""
     res = run_bptt(wl, precision, steps, warmup)
+    # an fp32 chunk's backward runs on fp32 MFMA
+    peak = FP32_MFMA_TFLOPS if precision == "fp32" else PEAK_TFLOPS[precision]
     return {
         "metric": "BPTT cell-steps/sec on 1 MI355X (30x30 C=32, batch 64, 32-step chunk)",
         "value": res["value"], "unit": "cell-steps/s", "n_gpus": 1, "steps": steps,
@@ -412,9 +419,9 @@ def bptt_entry(wl, precision, steps, warmup, cpu_budget=None):
         "config": {"workload": wl["desc"], "rows": res["rows"], "grid": [wl["grid"]] * 2,
                    "depth": wl["depth"]},
         "roofline": {"bound": "mfma", "achieved": res["achieved_tflops"],
-                     "peak": PEAK_TFLOPS[precision], "unit": "TFLOP/s",
-                     "frac": res["achieved_tflops"] / PEAK_TFLOPS[precision], "traffic": None,
-                     "frac_of_fp32_peak": res["achieved_tflops"] / PEAK_TFLOPS["fp32"]},
+                     "peak": peak, "unit": "TFLOP/s",
+                     "frac": res["achieved_tflops"] / peak, "traffic": None,
+                     "frac_of_fp32_peak": res["achieved_tflops"] / FP32_MFMA_TFLOPS},
         "peak_activation_bytes": res["peak_activation_bytes"],
         "states_bytes": res["states_bytes"], "workspace_bytes": res["workspace_bytes"],
         "skipped_updates": res["skipped"], "loss": res["loss"],
