@@ -23,8 +23,8 @@
 // step's M cells read and wrote all of them every step (84 MB a step for C = 64).
 //
 // Against the five GEMM launches, row sums, front, stencil and strip kernels that did a step
-// before (128 boards of 9x9, C = 64, bf16, 32 steps: 665 -> 46 us a step and 97 us per group of 13
-// steps; 64 boards of 13x13, C = 16, fp32: 117 -> 22 us a step and 100 us per group of 18). Every
+// before (128 boards of 9x9, C = 64, bf16, 32 steps: 665 -> 46 us a step and 62 us per group of 9
+// steps; 64 boards of 13x13, C = 16, fp32: 117 -> 22 us a step and 70 us per group of 11). Every
 // stage issues its loads before it uses the first (one at a time they took twice as long: the
 // compiler packs each pair of taps as it arrives), the weight fragments' loads are in flight
 // beside the head, the stores come last (a load waits for the stores issued before it), and the

@@ -137,7 +137,7 @@ struct StParams {
 };
 
 // REC: also write the state after every step to a.x_rec (the BPTT chunk's forward; 128 boards of 9x9, 32
-// steps: 255 us in one launch, 842 us as a launch per step, each of which loads the weights, the
+// steps: 265 us in one launch, 842 us as a launch per step, each of which loads the weights, the
 // tables and the state anew). The stores are the update lanes' own, beside the hidden waves' MFMAs.
 template <bool REC>
 __global__ void __launch_bounds__(512, 1) rollout_stream64(StParams sp) {

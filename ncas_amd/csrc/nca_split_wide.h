@@ -13,14 +13,14 @@
 // (RED) and are added in one order. The largest products and the five smaller ones have sums of
 // their own (a rounding of a smaller sum costs less).
 //
-// Per 16 cells and CU the MFMAs take 1,920 (C = 32) or 3,840 cycles; they are busy for 46 % of the
-// time at C = 64 and 36 % at C = 32. What is left, from versions without each part (64 steps of
+// Per 16 cells and CU the MFMAs take 1,920 (C = 32) or 3,840 cycles; they are busy for 49 % of the
+// time at C = 64 and 35 % at C = 32. What is left, from versions without each part (64 steps of
 // 2,048 boards 9x9 / 32 steps of 512 boards 30x30, fp32): fc1's products alone 6.3 / 4.4 ms, with the
 // stencil 7.9 / 5.4, with fc2 and the update but no stencil 9.6 / 6.9. The registers are full (96 of
 // 256 are fc1's accumulators): what splits a wave's code by a branch (waves without a stencil, half
 // of the waves updating while the others multiply) spilled 200 of them and took twice as long.
-// Measured against the fp32 MFMA kernels: 2,048 boards 9x9, 64 steps 21.2 -> 10.1 ms; 512 boards
-// 30x30, gated, 32 steps 14.9 -> 8.4 ms; error against 64 bits of a step 0.3 to 0.4 of theirs.
+// Measured against the fp32 MFMA kernels: 2,048 boards 9x9, 64 steps 21.2 -> 10.1 to 10.7 ms; 512
+// boards 30x30, gated, 32 steps 14.9 -> 8.4 to 9.5 ms by box; error against 64 bits of a step 0.3 to 0.4 of theirs.
 #pragma once
 
 #include "nca_split.h"
