@@ -6,7 +6,8 @@ the GPU through the C ABI.
 * On the configurations that need it - 201x201 mazes with the C=16 cell, 30x30 hard mazes with
   the C=32 cell and confidence-gated firing - and on ragged grids whose windows end mid-row,
   states stay within max-abs 1e-4 (fp32) / 2e-2 (bf16) of the CPU oracle with the same Philox
-  masks, and fired counts are exact.
+  masks, and fired counts are exact. (These run the automatic choice: fp32 steps on the bf16 matrix
+  cores; test_gpu_long.py holds the fp32 halo-window kernel to the same bound.)
 * bf16 cells with 16 channels run the per-step path on the wave-per-tile kernel; it gives the
   halo-window kernel's results (nca_set_kernel_path(3)) bit for bit on every padding and on grids
   whose last tile ends mid-row, with Philox, per-step-key and injected masks.
